@@ -10,6 +10,7 @@
 #include <string.h>
 
 #include <algorithm>
+#include <atomic>
 #include <chrono>
 
 #include "../../include/egs.h"
@@ -64,6 +65,8 @@ constexpr int kPinStats = 640;    // 6 x u64
 constexpr int kPinViol = 704;     // 1 x u64
 constexpr int kPinCert = 1024;    // certification readbacks (2 x 64 + 4 + 64 ints)
 constexpr int kPinOne = 1281;     // the constant 1 (raises ring[12])
+constexpr int kPinWhole = 1344;   // a WholeResult
+static_assert(kPinWhole * 4 + sizeof(egs::WholeResult) <= 4 * 2048, "the read-back area holds a WholeResult");
 constexpr int kProbeWant = 100;   // offset in a probe slot of ring[13] when it needs a copy of its own
 // The transpose costs about ten dense rounds to build, and a sparse round saves at most one
 // dense round: build it once this many rounds have wanted it (a proof usually leaves only a
@@ -73,6 +76,8 @@ constexpr int kCertFirstCap = 64;     // longest-path passes per candidate at th
 constexpr int kCertCandidates = 8;    // gap thresholds tried per attempt (plus the last-round rise set)
 constexpr int kCertEvery = 7;         // default rounds before the first proof attempt
 constexpr int kGraphSizes = 6;        // captured batches of 1, 2, 4, ..., 32 rounds
+constexpr int kWholeDenseN = 1 << 16; // single launches sweep every round densely; above this size a run of
+                                     // sparse rounds goes to the round kernels
 constexpr int kStopBatch = 4;         // rounds queued ahead of the host when a stop flag is polled
 
 double egs_now_ms() {
@@ -92,7 +97,7 @@ int pow2ceil(int x) {
 struct Layout {
     size_t ptr, edges, cptr, cpred, val, stamp, l0, l1, dbig, dhuge, sbig, shuge, lcnt, mode, ring, rounds, misc,
         tile, fill, stats, statsum, sigma, h, hist, bfcnt, bits, hacc, hcnt, hbest, hflag, tcounts, toffs, tscan,
-        titems, slen, sbase, sedges, bigmask, total;
+        titems, slen, sbase, sedges, bigmask, whole, total;
     int64_t tcounts_cap;
     int sub_cap;
     bool phased;
@@ -159,6 +164,7 @@ constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
     L.sbase = L.phased ? take(4 * ptiles * egs::kMaxPhases * egs::kSliceWaves) : 0;
     L.sedges = L.phased ? take(8 * m) : 0;
     L.bigmask = L.phased ? take(8 * ((size_t)n_cap / 64 + 2)) : 0;
+    L.whole = take(sizeof(egs::WholeCtl));
     L.total = off;
     return L;
 }
@@ -192,6 +198,13 @@ struct egs_solver {
     int2 *d_sedges = nullptr;
     unsigned long long *d_bigmask = nullptr;
     long long *d_h = nullptr;
+    egs::WholeCtl *d_whole = nullptr;
+    egs::WholePlan whole{};           // nb > 0: iterate() runs the game in single launches (egs_whole.hip)
+    unsigned whole_seq = 0;           // launches so far
+    int whole_max_nb = 0;             // workgroups of such a launch at most
+    int64_t whole_wait = egs::kWholeWait;
+    int64_t whole_rounds = 0;         // rounds of the run they have done
+    egs_stats whole_st{};             // what those rounds counted
     int wmax = 0;
     int cert_every = 32, cert_gap = 32, cert_max_passes = 1024;
     int cert_cap = 64;        // longest-path passes per candidate; doubles while attempts run out of passes
@@ -261,6 +274,7 @@ static void bind_layout(egs_solver *s, char *b, const Layout &L) {
     s->d_tscan = (int *)(b + L.tscan);
     s->d_titems = (int2 *)(b + L.titems);
     s->tcounts_cap = L.tcounts_cap;
+    s->d_whole = (egs::WholeCtl *)(b + L.whole);
     if (L.phased) {
         s->d_slen = (uint8_t *)(b + L.slen);
         s->d_sbase = (int *)(b + L.sbase);
@@ -350,9 +364,16 @@ static hipError_t replay_batch(egs_solver *s, int k) {
     return hipGraphLaunch(s->graph[k], s->stream);
 }
 
+// The large-route workers of a server share the compute units a slice leaves free.
+void egs::solver_limit_whole(egs_solver *s, int max_nb) { s->whole_max_nb = std::min(s->cus, max_nb); }
+
 extern "C" {
 
 const char *egs_last_error(void) { return g_err; }
+
+// Wait limit of the single launches' barriers in microseconds (tests force it to 0: a launch
+// then gives up as soon as a workgroup has to wait, and the round kernels take over).
+void egs_solver_whole_wait(egs_solver *s, int64_t us) { s->whole_wait = us * 100; }
 
 int egs_device_query(int device, egs_device_info *out) {
     if (!out) return fail(EGS_E_ARG, "egs_device_query: null output");
@@ -437,6 +458,7 @@ int egs_solver_create(int device, int32_t n_cap, int64_t m_cap, egs_solver **out
     egs_solver *s = new egs_solver();
     s->device = device;
     if (hipDeviceGetAttribute(&s->cus, hipDeviceAttributeMultiprocessorCount, device) != hipSuccess) s->cus = 256;
+    s->whole_max_nb = s->cus;
     s->n_cap = n_cap;
     s->m_cap = m_cap;
     const Layout L = make_layout(n_cap, m_cap);
@@ -654,6 +676,7 @@ static void bind_game(egs_solver *s, int32_t n, int32_t n0, int64_t m, int32_t m
     g.rounds_done = s->d_rounds;
     s->loaded = true;
     s->prepared = false;
+    s->whole = egs::WholePlan{};
 }
 
 static int pick_shape(egs_solver *s, const egs_options *o) {
@@ -750,11 +773,8 @@ static hipError_t build_csc(egs_solver *s) {
     return e;
 }
 
-int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
-    if (!s || !s->loaded) return fail(EGS_E_STATE, "egs_solver_prepare: no game loaded");
-    HIP_TRY(hipSetDevice(s->device));
-    int rc = pick_shape(s, opt);
-    if (rc) return rc;
+// Set-up of the round kernels: counters, static hub lists, slice layout, initial frontier.
+static int prepare_rounds(egs_solver *s) {
     // graphs hold the launch arguments they were captured with: kept while those stay the same
     if (memcmp(&s->graph_g, &s->g, sizeof(s->g)) != 0 || memcmp(&s->graph_sh, &s->sh, sizeof(s->sh)) != 0) {
         drop_graphs(s);
@@ -764,7 +784,6 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     // The set-up is timed by its own events and not waited for: the first round queues
     // behind it at once, and its time and the initial frontier are read after a later wait.
     // (The no-allocation solver has no events: it times on the host and waits here.)
-    HIP_TRY(close_prepare(s));
     const bool lazy = s->ev_pa && s->ev_pb;
     double t0 = 0;
     if (lazy) HIP_TRY(hipEventRecord(s->ev_pa, s->stream));
@@ -774,7 +793,6 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     // (config-2-like games sweep densely until a proof ends them).  Rounds stay dense while
     // it is missing; a round that would have gone sparse raises ring[13], and the host
     // builds the transpose at its next probe and opens sparse rounds (ring[12]).
-    s->csc_built = false;
     if (s->g.dense_min > s->g.n) HIP_TRY(build_csc(s));     // dense sweeps switched off
     if (s->sh.use_block)             // shared lifts of the vertices above huge_deg start empty
         HIP_TRY(egs::launch_hbest_reset(s->g, s->stream));
@@ -797,11 +815,170 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
         s->st.ms_prepare = ms;
         s->st.initial_active = (int32_t)list_total(s, s->h_probe + kPinInit);
     }
+    return EGS_OK;
+}
+
+// Single launches suit a solve whose options leave the round kernels' shape open and that
+// nothing has to stop part-way (the stop flag is polled between rounds on the host).
+static bool takes_whole(const egs_options *o) {
+    return !o || (o->group == 0 && o->big_deg == 0 && o->huge_deg == 0 && o->grid == 0 && o->batch_rounds == 0 &&
+                  o->dense_pct == 0 && o->slices == 0 && o->phase_wgs_per_cu == 0 && o->graphs == 0 && !o->stop_flag);
+}
+
+// Hand a run over from single launches to the round kernels: their whole set-up when it has
+// not begun, else the counters and lists, with the values reached and the next round a full
+// sweep (none when the run has converged).
+static int leave_whole(egs_solver *s) {
+    if (s->whole.nb == 0) return EGS_OK;
+    s->whole.nb = 0;
+    if (s->whole_rounds == 0 && !s->st.converged) return prepare_rounds(s);
+    HIP_TRY(egs::launch_prepare_reset(s->g, s->stream));
+    if (s->sh.use_block) HIP_TRY(egs::launch_hbest_reset(s->g, s->stream));
+    HIP_TRY(egs::launch_classify(s->g, s->d_ring + 9, s->stream));
+    HIP_TRY(egs::launch_resume(s->g, (int)s->next_round, s->st.converged != 0, s->stream));
+    return EGS_OK;
+}
+
+// Workgroups of the single launches under way per device.  A launch whose workgroups would not
+// all fit beside those of other solvers is not made (they would wait for each other until
+// their limit); the round kernels take the game.
+struct WholeRoom {
+    std::atomic<int> &used;
+    int want;
+    bool ok;
+    WholeRoom(const egs_solver *s) : used(slots()[(unsigned)s->device % 64]), want(0), ok(true) {
+        if (s->whole.nb == 1) return;                          // waits for nobody
+        // two workgroups of 1,024 threads share a compute unit when their LDS allows
+        want = s->whole.nb * (egs::whole_lds(s->whole) > 79 * 1024 ? 2 : 1);
+        ok = used.fetch_add(want) + want <= 2 * s->cus;
+    }
+    ~WholeRoom() { used.fetch_sub(want); }
+    static std::atomic<int> *slots() {
+        static std::atomic<int> u[64];
+        return u;
+    }
+};
+
+// Rounds in single launches until the fixpoint, `limit` more rounds, or a state that the
+// round kernels serve better; *status tells which (kWholeNone: the launch gave up waiting for
+// its workgroups, and the values are some state between its start and the fixpoint).
+static int run_whole(egs_solver *s, int64_t limit, int *status) {
+    // a launch of this many rounds ends within tens of milliseconds
+    constexpr int64_t kRoundsPerLaunch = 8192;
+    egs::WholeArgs a{};
+    const egs::DevGame &g = s->g;
+    a.n = g.n;
+    a.n0 = g.n0;
+    a.mg = g.mg;
+    a.wmax = s->wmax;
+    a.m = g.m;
+    a.ptr = g.ptr;
+    a.edges = g.edges;
+    a.val = g.val;
+    a.rise = g.rise;
+    a.h = s->d_h;
+    a.ctl = s->d_whole;
+    a.nbmax = s->whole.nbmax;
+    a.wait = s->whole_wait;
+    a.every = s->cert_every;
+    a.max_passes = s->cert_max_passes;
+    a.max_cands = kCertCandidates;
+    a.sparse_exit = g.n > kWholeDenseN ? kSparseWantRounds : 0;
+    a.dense_min = g.dense_min;
+    // the result comes back through the pinned block, which the kernel stores into; the
+    // no-allocation solver has none and copies it from device memory
+    egs::WholeResult *res = (egs::WholeResult *)(s->h_probe + kPinWhole);
+    a.out = s->no_alloc ? (egs::WholeResult *)s->d_misc : res;
+    *status = egs::kWholeNone;
+    WholeRoom room(s);
+    if (!room.ok) return EGS_OK;
+    *status = egs::kWholeLimit;
+    while (*status == egs::kWholeLimit && limit > 0) {
+        a.limit = std::min(limit, kRoundsPerLaunch);
+        a.round0 = s->whole_rounds;
+        a.next_cert = s->next_cert;
+        a.gap = (int)s->cert_gap;
+        a.cap = s->cert_cap;
+        a.seq = ++s->whole_seq;
+        __atomic_store_n(&res->done, 0u, __ATOMIC_RELEASE);     // no launch of this solver is running
+        if (s->whole_rounds > 0) HIP_TRY(egs::launch_whole_prep(s->whole, g, s->d_whole, false, s->stream));
+        HIP_TRY(egs::launch_whole(s->whole, a, s->stream));
+        bool got;
+        if (s->no_alloc) {
+            HIP_TRY(hipMemcpyAsync(res, a.out, sizeof(*res), hipMemcpyDeviceToHost, s->stream));
+            HIP_TRY(hipStreamSynchronize(s->stream));
+            got = res->done == a.seq;
+        } else {
+            // spin on the pinned word (stored last), asking the stream now and then so that a
+            // launch that ended without it is noticed
+            const volatile unsigned *done = &res->done;
+            hipError_t q = hipErrorNotReady;
+            while (q == hipErrorNotReady) {
+                for (int k = 0; k < 4096 && __atomic_load_n(done, __ATOMIC_ACQUIRE) != a.seq; k++) __builtin_ia32_pause();
+                if (__atomic_load_n(done, __ATOMIC_ACQUIRE) == a.seq) break;
+                q = hipStreamQuery(s->stream);
+            }
+            got = __atomic_load_n(done, __ATOMIC_ACQUIRE) == a.seq;
+            if (!got) HIP_TRY(q);
+        }
+        if (!got) {
+            *status = egs::kWholeNone;
+            break;
+        }
+        const int64_t ran = res->rounds - s->whole_rounds;
+        if (s->whole_rounds == 0) {
+            s->st.initial_active = (int32_t)res->initial;
+            s->st.ms_prepare += 1e-5 * (double)res->ticks_setup;
+        } else {
+            s->st.ms_iterate += 1e-5 * (double)res->ticks_setup;
+        }
+        s->st.ms_iterate += 1e-5 * (double)(res->ticks - res->ticks_setup);
+        s->whole_st.processed += ran * g.n;
+        s->whole_st.edges_relaxed += res->edges;
+        s->whole_st.lifted += res->lifted;
+        s->st.cert_attempts += res->attempts;
+        s->st.certificates += res->certs;
+        s->st.cert_passes += res->passes;
+        s->st.top_marked += res->marked;
+        s->st.cert_pruned += res->pruned;
+        s->whole_rounds = res->rounds;
+        s->next_round = res->rounds + 1;
+        s->next_cert = res->next_cert;
+        s->cert_gap = res->gap;
+        s->cert_cap = res->cap;
+        limit -= ran;
+        *status = res->status;
+    }
+    s->st.phases = s->whole_rounds;
+    s->st.processed = s->whole_st.processed;
+    s->st.edges_relaxed = s->whole_st.edges_relaxed;
+    s->st.lifted = s->whole_st.lifted;
+    s->st.converged = *status == egs::kWholeDone;
+    return EGS_OK;
+}
+
+int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
+    if (!s || !s->loaded) return fail(EGS_E_STATE, "egs_solver_prepare: no game loaded");
+    HIP_TRY(hipSetDevice(s->device));
+    int rc = pick_shape(s, opt);
+    if (rc) return rc;
+    HIP_TRY(close_prepare(s));
+    s->csc_built = false;
     s->next_round = 1;
     s->cert_gap = s->cert_every;
     s->next_cert = s->cert_every;
     s->cert_cap = std::min(kCertFirstCap, s->cert_max_passes);
     s->cert_pass_hint = 0;
+    s->whole_rounds = 0;
+    s->whole_st = egs_stats{};
+    s->whole = takes_whole(opt) ? egs::whole_plan(s->g.n, s->g.m, s->g.mg, s->wmax, s->max_outdeg, s->whole_max_nb) : egs::WholePlan{};
+    if (s->whole.nb > 0) {
+        HIP_TRY(egs::launch_whole_prep(s->whole, s->g, s->d_whole, true, s->stream));
+        memset(&s->st, 0, sizeof(s->st));
+    } else {
+        rc = prepare_rounds(s);
+        if (rc) return rc;
+    }
     s->prepared = true;
     return EGS_OK;
 }
@@ -817,9 +994,10 @@ static int queue_stats(egs_solver *s) {
 
 static int collect_stats(egs_solver *s) {
     const unsigned long long *h = (const unsigned long long *)(s->h_probe + kPinStats);
-    s->st.processed = (int64_t)h[0];
-    s->st.edges_relaxed = (int64_t)h[1];
-    s->st.lifted = (int64_t)h[2];
+    // on top of the rounds done in single launches
+    s->st.processed = (int64_t)h[0] + s->whole_st.processed;
+    s->st.edges_relaxed = (int64_t)h[1] + s->whole_st.edges_relaxed;
+    s->st.lifted = (int64_t)h[2] + s->whole_st.lifted;
     s->st.pred_visits = (int64_t)h[3];
     s->st.phases = (int32_t)h[4];
     s->st.csc_built = s->csc_built ? 1 : 0;
@@ -833,6 +1011,22 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
     int64_t limit = s->phase_cap - (s->next_round - 1);
     if (max_phases >= 0 && max_phases < limit) limit = max_phases;
     if (s->next_round + limit > 0x7ffffff0LL) limit = 0x7ffffff0LL - s->next_round;
+    if (s->whole.nb > 0) {
+        int status = egs::kWholeNone, rc = EGS_OK;
+        if (max_phases < 0 && !s->st.converged) {
+            const int64_t before = s->whole_rounds;
+            rc = run_whole(s, limit, &status);
+            if (rc) return rc;
+            limit -= s->whole_rounds - before;
+        }
+        if (status == egs::kWholeDone || status == egs::kWholeLimit || s->st.converged) {
+            if (st) *st = s->st;
+            return s->st.converged ? 1 : 0;
+        }
+        rc = leave_whole(s);
+        if (rc) return rc;
+        if (status == egs::kWholeSparse) HIP_TRY(build_csc(s));
+    }
     double t0 = 0;
     HIP_TRY(mark_start(s, &t0));
     int64_t launched = 0;
@@ -989,6 +1183,7 @@ void *egs_solver_stream(egs_solver *s) { return s ? (void *)s->stream : nullptr;
 int egs_solver_read_csc(egs_solver *s, int32_t *cptr, int32_t *cpred) {
     if (!s || !s->prepared) return fail(EGS_E_STATE, "egs_solver_read_csc: not prepared");
     HIP_TRY(hipSetDevice(s->device));
+    if (int rc = leave_whole(s)) return rc;
     if (!s->csc_built) HIP_TRY(build_csc(s));
     HIP_TRY(hipMemcpyAsync(cptr, s->d_cptr, sizeof(int) * ((size_t)s->g.n + 1), hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(hipMemcpyAsync(cpred, s->d_cpred, sizeof(int) * (size_t)s->g.m, hipMemcpyDeviceToHost, s->stream));
@@ -1010,6 +1205,7 @@ int egs_solver_count_violations(egs_solver *s, int64_t *violations) {
 int egs_solver_set_values(egs_solver *s, const int32_t *host_values) {
     if (!s || !s->prepared || !host_values) return fail(EGS_E_STATE, "egs_solver_set_values: call egs_solver_prepare first");
     HIP_TRY(hipSetDevice(s->device));
+    if (int rc = leave_whole(s)) return rc;
     HIP_TRY(hipMemcpyAsync(s->d_val, host_values, sizeof(int) * (size_t)s->g.n, hipMemcpyHostToDevice, s->stream));
     // the values may hold TOP: the phased rounds then read their TOP masks (ring[15])
     HIP_TRY(hipMemcpyAsync(s->d_ring + 15, s->h_probe + kPinOne, sizeof(int), hipMemcpyHostToDevice, s->stream));
@@ -1020,6 +1216,7 @@ int egs_solver_set_values(egs_solver *s, const int32_t *host_values) {
 int egs_solver_top_certificate(egs_solver *s, int32_t max_passes, int64_t *host_h, int32_t *passes) {
     if (!s || !s->prepared || !host_h) return fail(EGS_E_STATE, "egs_solver_top_certificate: call egs_solver_prepare first");
     HIP_TRY(hipSetDevice(s->device));
+    if (int rc = leave_whole(s)) return rc;
     egs::CertBuffers cb{s->d_hist, s->d_h, s->d_bfcnt, s->d_bits, s->h_probe + kPinCert};
     egs::CertResult cr;
     const int got = egs::certify_all_top(s->g, cb, s->wmax, max_passes > 0 ? max_passes : (1 << 16),
@@ -1089,6 +1286,7 @@ static int noalloc_setup(int dev) {
     s.device = dev;
     s.no_alloc = true;
     if (hipDeviceGetAttribute(&s.cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) s.cus = 256;
+    s.whole_max_nb = s.cus;
     s.n_cap = kNoAllocN;
     s.m_cap = kNoAllocM;
     s.block = nullptr;                 // not owned: never freed

@@ -4,7 +4,12 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+struct egs_solver;
+
 namespace egs {
+
+// Workgroups of a solver's single launches (egs_whole.hip) at most.
+void solver_limit_whole(egs_solver *s, int max_nb);
 
 // Frontier lists are split into kSub sub-queues of sub_cap slots plus one overflow region
 // of n slots; a workgroup appends to sub-queue (blockIdx.x % kSub), so no counter sees
@@ -106,6 +111,61 @@ struct LaunchShape {
     int wave_grid, block_grid;
 };
 
+// A whole solve in one launch (egs_whole.hip).
+constexpr int kWholeMaxNb = 256;           // workgroups at most
+constexpr int kWholeGroups = 8;            // groups of workgroups in a vote
+constexpr int64_t kWholeWait = 400000;     // barrier wait limit (4 ms) before a launch gives up
+constexpr int kWholeOneN = 5999, kWholeOneM = 16384;   // one workgroup up to this size
+// Vertices + edges per workgroup while workgroups are left.  Device time of a solve (degree
+// 2..16, us) at shares of 1,536 / 2,304 / 3,072 / 4,608 / 6,144: n = 9,973: 71 / 71 / 74 / 85 / 93;
+// n = 30,011: 113 / 100 / 96 / 102 / 101; n = 87,148: 166 / 166 / 166 / 170 / 161.
+constexpr int kWholeShare = 3072;
+constexpr int kWholeShareMax = 7168;       // past this (all workgroups in use) the round kernels win:
+                                           // n = 262,147, degree 8: 444 us against 353
+enum : int { kWholeNone = 0, kWholeDone = 1, kWholeLimit = 2, kWholeSparse = 3 };
+
+struct WholeCtl {
+    unsigned long long root[4][16];        // vote words, a cache line each: all groups,
+    unsigned long long group[4][kWholeGroups][16];    // the workgroups of a group,
+    unsigned long long release[4][kWholeGroups][16];  // the total, handed to a group
+    unsigned long long abort_flag, pad0[15];
+    unsigned long long sum[16];            // edges relaxed, lifts
+    int hist[2][128];                      // value histograms of the proof attempts, in turn
+    int bound[kWholeMaxNb + 1];            // first vertex of each workgroup
+};
+struct WholeResult {
+    int status, attempts, certs, pruned, gap, cap;
+    long long rounds, initial, passes, marked, edges, lifted, next_cert, ticks_setup, ticks;
+    unsigned done;                         // the launch's seq, stored last
+};
+struct WholeArgs {
+    int n, n0, mg, wmax;
+    int64_t m;
+    const int *ptr;
+    const int2 *edges;
+    int *val, *rise;                       // rise: null without proofs
+    long long *h;
+    WholeCtl *ctl;
+    WholeResult *out;
+    int nbmax;                             // vertices of a workgroup at most (LDS)
+    int64_t limit;                         // rounds of this launch at most
+    int64_t round0, next_cert;             // rounds already run; the round of the next attempt
+    int every, gap, cap, max_passes, max_cands;
+    int sparse_exit;                       // leave after this many rounds below dense_min (0: never)
+    int64_t dense_min;
+    int64_t wait;                          // barrier wait limit in 100 MHz ticks
+    unsigned seq;
+};
+struct WholePlan {
+    int nb, nbmax, threads, per;           // workgroups (0: not for this game), LDS vertices, threads, edges a thread
+    int64_t share;                         // vertices + edges per workgroup
+    int small_d, small_v;                  // a thread per vertex: edge slots, vertices a thread (0: not)
+};
+WholePlan whole_plan(int n, int64_t m, int mg, int wmax, int max_outdeg, int max_nb);
+size_t whole_lds(const WholePlan &p);
+hipError_t launch_whole_prep(const WholePlan &p, const DevGame &g, WholeCtl *ctl, bool fresh, hipStream_t st);
+hipError_t launch_whole(const WholePlan &p, const WholeArgs &a, hipStream_t st);
+
 hipError_t launch_pack(const int *succ, const int *w, int2 *edges, int64_t m, hipStream_t st);
 hipError_t launch_unpack(const uint32_t *packed, int shift, int2 *edges, int64_t m, hipStream_t st);
 hipError_t launch_transpose(const DevGame &g, int *tile_sum, int *fill, hipStream_t st);
@@ -139,6 +199,9 @@ int pack_shift(int n, int wmax);
 // Round j of a batch (absolute round ring[14] + j); launch_advance ends the batch.
 hipError_t launch_round(const DevGame &g, const LaunchShape &sh, int j, hipStream_t st);
 hipError_t launch_advance(const DevGame &g, int rounds, hipStream_t st);
+// Round `next` is the first of the round kernels on values reached otherwise (after
+// launch_prepare_reset): a full sweep, or none when they have converged.
+hipError_t launch_resume(const DevGame &g, int next, bool converged, hipStream_t st);
 hipError_t launch_prepare_reset(const DevGame &g, hipStream_t st);
 hipError_t launch_sum_stats(const DevGame &g, int nslots, unsigned long long *out, hipStream_t st);
 hipError_t launch_degree_stats(const int *ptr, int n, int *out, hipStream_t st);

@@ -953,6 +953,28 @@ hipError_t launch_advance(const DevGame &g, int rounds, hipStream_t st) {
     return hipGetLastError();
 }
 
+// The state of round `next` - 1 done elsewhere: nothing queued or claimed (stamps), the next
+// round named a full sweep, its input a count without items.
+__global__ __launch_bounds__(256) void k_resume(DevGame g, int next, int converged) {
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += (int64_t)gridDim.x * blockDim.x)
+        g.stamp[v] = 0;
+    if (blockIdx.x == 0 && threadIdx.x == 0) {
+        g.ring[14] = next;
+        g.ring[15] = 1;
+        *g.rounds_done = next - 1;
+        if (!converged) {
+            g.ring[11] = next;
+            g.mode[3] = next;
+            g.lcnt[(next % 3) * kListCounters] = 1;
+        }
+    }
+}
+
+hipError_t launch_resume(const DevGame &g, int next, bool converged, hipStream_t st) {
+    hipLaunchKernelGGL(k_resume, dim3(grid_for(g.n, 256, 1024)), dim3(256), 0, st, g, next, converged ? 1 : 0);
+    return hipGetLastError();
+}
+
 hipError_t launch_round(const DevGame &g, const LaunchShape &sh, int j, hipStream_t st) {
     const dim3 grid(g.round_grid + (g.hub_fused ? g.wave_grid + g.block_grid : 0));
 #define EGS_ROUND(GG)                                                                            \

@@ -1,0 +1,203 @@
+"""Whole solves in one launch (egs_whole.hip): exact against the oracle or the round kernels
+at the sizes where its forms begin and end, and the hand-over to the round kernels."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from conftest import lfp, to_oracle_game
+
+pytestmark = pytest.mark.gpu
+
+TOP = 2147483647
+
+
+def _say(msg):
+    print(f"[gpu-case] {msg}", flush=True)
+
+
+def _rounds(s, **opt):
+    """The loaded game by the round kernels (an explicit lane count keeps them)."""
+    import egsolver_amd as E
+    s.prepare(E.options(group=4, **opt))
+    conv, st = s.iterate()
+    assert conv
+    return s.values()
+
+
+# (n, degree kind, lo, hi, alpha, W): a thread per vertex with 4, 8 and 16 slots and one or two
+# vertices a thread, then past its edges; one workgroup and past its vertices and edges;
+# complete digraphs; hubs in one workgroup's share and beyond a share; the largest shares
+GAMES = [(2, 0, 1, 1, 0, 5), (61, 1, 2, 6, 0, 10), (1024, 1, 1, 16, 0, 50), (1025, 1, 1, 16, 0, 50), (1024, 1, 1, 17, 0, 50),
+         (2048, 0, 4, 4, 0, 10), (2049, 0, 4, 4, 0, 10), (2048, 1, 1, 8, 0, 30), (1500, 2, 1, 300, 1.8, 30),
+         (4096, 0, 4, 4, 0, 10), (4097, 0, 4, 4, 0, 10), (5999, 0, 1, 1, 0, 20), (6000, 0, 1, 1, 0, 20),
+         (130, 3, 0, 0, 0, 40), (400, 3, 0, 0, 0, 40), (12345, 1, 1, 9, 0, 100), (20011, 2, 1, 9000, 1.9, 60),
+         (60000, 2, 1, 13000, 2.1, 60), (87149, 1, 2, 16, 0, 1000), (203000, 0, 8, 8, 0, 100), (204000, 0, 8, 8, 0, 100)]
+
+
+@pytest.mark.parametrize("i", range(len(GAMES)))
+def test_whole_solve_exact(oracle, i):
+    import egsolver_amd as E
+    n, kind, lo, hi, alpha, wmax = GAMES[i]
+    g = E.generate(E.GenParams(n=n, seed=40 + i, deg_kind=kind, deg_lo=lo, deg_hi=hi, alpha=alpha, wmax=wmax))
+    _say(f"whole solve n {g.n} m {g.m} maxdeg {g.max_outdeg}")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        want = lfp(oracle, to_oracle_game(g)) if g.m < 40000 else _rounds(s)
+        opts = [{}, {"certify_every": 2}, {"certify_every": 3, "cert_max_passes": 2}]
+        if n <= 2500:
+            opts.append({"certify_every": -1})
+        for opt in opts:
+            s.prepare(E.options(**opt))
+            assert not s.values().any()                     # values are reset before the run
+            conv, st = s.iterate()
+            assert conv and st.converged
+            vals = s.values()
+            assert np.array_equal(vals, want), (opt, np.count_nonzero(vals != want))
+            assert s.violations() == 0
+        conv, again = s.iterate()                           # a converged run stays as it is
+        assert conv and again.phases == st.phases
+
+
+def _climber(n, mg):
+    """Vertex 0 (owner 1) climbs one unit a round on its self-loop until it passes MG; the others
+    reach the last one, whose edges make up MG, from either owner."""
+    import egsolver_amd as E
+    succ = np.full(n, n - 1, np.int32)
+    w = np.zeros(n, np.int32)
+    succ[0], w[0] = 0, -1
+    succ[1], w[1] = 0, -(mg - 1)
+    ptr = np.arange(n + 1, dtype=np.int32)
+    g = E.Game(n=n, n0=0, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(n, ptr, w), ext_of_int=np.arange(n, dtype=np.int32))
+    assert g.mg == mg
+    want = np.zeros(n, np.int32)
+    want[:2] = TOP
+    return g, want
+
+
+@pytest.mark.parametrize("n", [100, 3000, 9000])
+def test_rounds_past_one_launch(n):
+    """20,000 plain rounds span several launches of 8,192; the round cap stops between them."""
+    import egsolver_amd as E
+    g, want = _climber(n, 20000)
+    _say(f"climber n {n}")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        s.prepare(E.options(certify_every=-1))
+        conv, st = s.iterate()
+        assert conv and st.phases == 20002 and st.initial_active == 2
+        assert np.array_equal(s.values(), want)
+        for cap in (1, 9000):
+            s.prepare(E.options(certify_every=-1, max_phases=cap))
+            conv, st = s.iterate()
+            assert not conv and st.phases == cap
+            assert s.values()[0] == cap
+        s.prepare()
+        conv, st = s.iterate()
+        assert conv and st.certificates >= 1
+        assert np.array_equal(s.values(), want)
+
+
+@pytest.mark.parametrize("n,hi", [(1000, 6), (3000, 40), (30011, 16)])
+def test_hand_over_to_round_kernels(n, hi):
+    """A solved or half-run game used through the other entry points: a capped first run and its
+    resumption, the transpose, the certificate of the TOP set, and replaced values."""
+    import egsolver_amd as E
+    from egsolver_amd import verify
+    g = E.generate(E.GenParams(n=n, seed=3, deg_kind=1, deg_lo=2, deg_hi=hi, wmax=100))
+    _say(f"hand over n {g.n} m {g.m}")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        want = _rounds(s)
+        s.prepare()
+        conv, st = s.iterate(max_phases=3)
+        assert not conv and st.phases == 3
+        assert np.all(s.values() <= want)
+        conv, st = s.iterate()
+        assert conv and np.array_equal(s.values(), want)
+        s.prepare(E.options(max_phases=4))
+        conv, st = s.iterate()
+        assert not conv and st.phases == 4
+        assert np.all(s.values() <= want)
+        s.prepare()
+        s.iterate()
+        rep = verify.certify(s, g, s.values())
+        assert rep["ok"], rep
+        assert np.array_equal(s.values(), want)
+        s.prepare()
+        cptr, _ = s.csc()
+        assert cptr[-1] == g.m
+        conv, _ = s.iterate()
+        assert conv and np.array_equal(s.values(), want)
+        s.prepare()
+        s.set_values(want)
+        assert s.violations() == 0
+
+
+@pytest.mark.parametrize("n", [9973, 87148])
+def test_launch_that_gives_up(n):
+    """With no patience for its barrier a launch leaves at the first wait; the round kernels
+    finish from the values reached, to the same fixpoint."""
+    import egsolver_amd as E
+    from egsolver_amd import _native as N
+    g = E.generate(E.GenParams(n=n, seed=8, deg_kind=1, deg_lo=2, deg_hi=16, wmax=100))
+    _say(f"no patience n {g.n} m {g.m}")
+    fn = N.egs().egs_solver_whole_wait
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_int64]
+    fn.restype = None
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        want = _rounds(s)
+        fn(s.h, 0)
+        for _ in range(3):
+            s.prepare()
+            conv, _ = s.iterate()
+            assert conv and np.array_equal(s.values(), want)
+            assert s.violations() == 0
+
+
+def test_weights_near_the_value_range(oracle):
+    """MG plus a weight past 2^31 (a TOP value less a weight would fall below MG): such games
+    stay with the round kernels and their overflow rules."""
+    import egsolver_amd as E
+    ptr = np.array([0, 2, 4, 5], np.int32)
+    succ = np.array([1, 2, 0, 2, 2], np.int32)
+    w = np.array([2147000000, -2000000000, 5, -100000000, 3], np.int32)
+    g = E.Game(n=3, n0=1, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(3, ptr, w), ext_of_int=np.arange(3, dtype=np.int32))
+    _say(f"heavy weights mg {g.mg}")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        s.prepare()
+        conv, _ = s.iterate()
+        assert conv and s.violations() == 0
+        assert np.array_equal(s.values(), lfp(oracle, to_oracle_game(g)))
+
+
+def test_several_solvers_at_once():
+    """Solvers on several threads: their launches share the device or leave it to the round
+    kernels, with the same values."""
+    import threading
+    import egsolver_amd as E
+    games = [E.generate(E.GenParams(n=n, seed=60 + i, deg_kind=1, deg_lo=2, deg_hi=16, wmax=100))
+             for i, n in enumerate((87148, 60000, 87148, 30011, 120000, 1999))]
+    want = []
+    for g in games:
+        with E.Solver(g.n, g.m) as s:
+            s.load(g)
+            want.append(_rounds(s))
+    bad = []
+
+    def work(i):
+        with E.Solver(games[i].n, games[i].m) as s:
+            s.load(games[i])
+            for _ in range(5):
+                s.prepare()
+                conv, _ = s.iterate()
+                if not conv or not np.array_equal(s.values(), want[i]):
+                    bad.append(i)
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(len(games))]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad
