@@ -894,26 +894,9 @@ static void launch_bf_pass(int G, int grid, hipStream_t st, const DevGame &g, lo
     }
 }
 
-__global__ void k_abs_wmax(const int2 *__restrict__ edges, int64_t m, int *__restrict__ out) {
-    int mx = 0;
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m; e += (int64_t)gridDim.x * blockDim.x) {
-        const int w = edges[e].y;
-        mx = max(mx, w < 0 ? -w : w);
-    }
-    for (int d = 32; d >= 1; d >>= 1) mx = max(mx, __shfl_xor(mx, d, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, mx);
-}
-
 // ---------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------
-
-hipError_t launch_abs_wmax(const DevGame &g, int *out, hipStream_t st) {
-    hipError_t err = hipMemsetAsync(out, 0, sizeof(int), st);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_abs_wmax, dim3(grid_for(g.m, 256, 2048)), dim3(256), 0, st, g.edges, g.m, out);
-    return hipGetLastError();
-}
 
 // Admissible thresholds (host side): B_j = W * 2^j with some non-TOP value above it and
 // B_j <= MG - W; first those with an empty window, smallest first, then the smallest whose

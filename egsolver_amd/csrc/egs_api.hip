@@ -58,13 +58,13 @@ int64_t egs_max_loop_c(int64_t m, int64_t n, int64_t mg, int64_t maxloop) {
 // Offsets (in ints) inside the solver's pinned readback block.
 constexpr int kPinProbe = 2048;   // 2 x kProbeStride: per-batch counter probes
 constexpr int kProbeStride = 512;
-constexpr int kPinDeg = 256;
 constexpr int kPinInit = 320;     // kListCounters ints
 constexpr int kPinConv = 448;     // kListCounters ints
 constexpr int kPinStats = 640;    // 6 x u64
 constexpr int kPinViol = 704;     // 1 x u64
 constexpr int kPinCert = 1024;    // certification readbacks (2 x 64 + 4 + 64 ints)
 constexpr int kPinOne = 1281;     // the constant 1 (raises ring[12])
+constexpr int kPinLoad = 768;     // a LoadResult
 constexpr int kPinWhole = 1344;   // a WholeResult
 static_assert(kPinWhole * 4 + sizeof(egs::WholeResult) <= 4 * 2048, "the read-back area holds a WholeResult");
 constexpr int kProbeWant = 100;   // offset in a probe slot of ring[13] when it needs a copy of its own
@@ -200,6 +200,7 @@ struct egs_solver {
     long long *d_h = nullptr;
     egs::WholeCtl *d_whole = nullptr;
     egs::WholePlan whole{};           // nb > 0: iterate() runs the game in single launches (egs_whole.hip)
+    unsigned load_seq = 0;            // loads whose record was asked for
     unsigned whole_seq = 0;           // launches so far
     int whole_max_nb = 0;             // workgroups of such a launch at most
     int64_t whole_wait = egs::kWholeWait;
@@ -306,6 +307,40 @@ static hipError_t probe_mark(egs_solver *s, int slot) {
 }
 static hipError_t probe_wait(egs_solver *s, int slot) {
     return s->ev_probe[slot] ? hipEventSynchronize(s->ev_probe[slot]) : hipStreamSynchronize(s->stream);
+}
+
+// Wait for the word `done`, stored last by queued work that ends, to become seq: a spin on the
+// pinned word that asks the stream now and then, so that work that ended without storing it is
+// noticed (false).  On return the work's stores to pinned memory are visible.
+static hipError_t wait_word(egs_solver *s, const unsigned *done, unsigned seq, bool *got) {
+    hipError_t q = hipErrorNotReady;
+    for (;;) {
+        for (int k = 0; k < 4096 && __atomic_load_n(done, __ATOMIC_ACQUIRE) != seq; k++) __builtin_ia32_pause();
+        *got = __atomic_load_n(done, __ATOMIC_ACQUIRE) == seq;
+        if (*got) return hipSuccess;
+        if (q != hipErrorNotReady) return q;         // the stream was done before this last look
+        q = hipStreamQuery(s->stream);
+    }
+}
+
+// The record of a load (launch_load_finish last on the stream), on the host.  The no-allocation
+// solver has no pinned block and copies it from device memory.
+static hipError_t read_load(egs_solver *s, const egs::LoadPartial *part, int nparts, const int *n0, const int *bad,
+                            egs::LoadResult **out) {
+    egs::LoadResult *res = (egs::LoadResult *)(s->h_probe + kPinLoad);
+    *out = res;
+    const unsigned seq = ++s->load_seq;
+    __atomic_store_n(&res->done, 0u, __ATOMIC_RELEASE);
+    egs::LoadResult *to = s->no_alloc ? (egs::LoadResult *)s->d_misc : res;
+    hipError_t e = egs::launch_load_finish(part, nparts, n0, bad, seq, to, s->stream);
+    if (e != hipSuccess) return e;
+    if (s->no_alloc) {
+        e = hipMemcpyAsync(res, to, sizeof(*res), hipMemcpyDeviceToHost, s->stream);
+        return e == hipSuccess ? hipStreamSynchronize(s->stream) : e;
+    }
+    bool got = false;
+    e = wait_word(s, &res->done, seq, &got);
+    return got ? hipSuccess : e != hipSuccess ? e : hipErrorUnknown;
 }
 
 // Items in a list from its counters (sub-queues clamp at sub_cap; the rest overflowed).
@@ -522,19 +557,13 @@ int egs_solver_load(egs_solver *s, int mem, int32_t n, int32_t n0, int64_t m, in
         HIP_TRY(e2);
     } else if (mem == EGS_MEM_DEVICE) {
         // device inputs are trusted to be a valid CSR of this shape (the caller owns them)
-        HIP_TRY(hipMemcpyAsync(s->d_ptr, ptr, sizeof(int) * ((size_t)n + 1), hipMemcpyDeviceToDevice, s->stream));
-        HIP_TRY(egs::launch_pack(succ, w, s->d_edges, m, s->stream));
-        HIP_TRY(egs::launch_degree_stats(s->d_ptr, n, s->d_misc, s->stream));
-        HIP_TRY(hipMemcpyAsync(s->h_probe + kPinDeg, s->d_misc, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
-        s->max_outdeg = s->h_probe[kPinDeg];
-        egs::DevGame tmp{};
-        tmp.edges = s->d_edges;
-        tmp.m = m;
-        HIP_TRY(egs::launch_abs_wmax(tmp, s->d_misc, s->stream));
-        HIP_TRY(hipMemcpyAsync(s->h_probe + kPinDeg, s->d_misc, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
-        s->wmax = s->h_probe[kPinDeg];
+        egs::LoadPartial *part = (egs::LoadPartial *)s->d_stats;     // prepare clears it later
+        egs::LoadResult *res;
+        int nparts = 0;
+        HIP_TRY(egs::launch_load_device(ptr, succ, w, n, m, s->d_ptr, s->d_edges, part, &nparts, s->stream));
+        HIP_TRY(read_load(s, part, nparts, nullptr, nullptr, &res));
+        s->max_outdeg = res->dmax;
+        s->wmax = res->wmax;
     } else {
         return fail(EGS_E_ARG, "mem must be EGS_MEM_HOST or EGS_MEM_DEVICE");
     }
@@ -591,37 +620,32 @@ int egs_solver_load_read_order(egs_solver *s, int mem, int32_t n, int64_t m, con
         b.rsucc = rsucc;
         b.rw = rw;
     }
-    HIP_TRY(egs::launch_read_order_check(b.rptr, b.rsucc, n, m, s->d_misc + 8, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->h_probe + kPinDeg, s->d_misc + 8, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    const int bad = s->h_probe[kPinDeg];
-    if (bad & 1) return fail(EGS_E_ARG, "read-order offsets must run from 0 to m");
-    if (bad & 2) return fail(EGS_E_ARG, "a vertex has no out-edge");
-    if (bad & 4) return fail(EGS_E_ARG, "a successor is out of range");
+    // the check's verdict stays on the device: the kernels after it return at once on a bad
+    // game, and the host reads it with the result
+    int *d_bad = s->d_misc + 24;
+    HIP_TRY(egs::launch_read_order_check(b.rptr, b.rsucc, n, m, d_bad, s->stream));
     b.flag0 = s->d_sigma;
     b.pre0 = s->d_fill;
     b.rev = s->d_dbig;
     b.ext_of_int = s->d_sbig;
     b.deg = s->d_dhuge;
     b.scan_tiles = s->d_tile;
-    unsigned long long *d_mg = (unsigned long long *)s->d_misc;
-    HIP_TRY(egs::launch_internalise(b, n, s->d_ptr, s->d_edges, d_mg, s->stream));
-    unsigned long long *h_mg = (unsigned long long *)(s->h_probe + kPinViol);
-    HIP_TRY(hipMemcpyAsync(h_mg, d_mg, sizeof(unsigned long long), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->h_probe + kPinDeg + 1, s->d_fill + n, sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    if (ext_of_int)
+    egs::LoadPartial *part = nullptr;
+    egs::LoadResult *res;
+    int nparts = 0;
+    HIP_TRY(egs::launch_internalise(b, n, d_bad, s->d_ptr, s->d_edges, &part, &nparts, s->stream));
+    HIP_TRY(read_load(s, part, nparts, s->d_fill + n, d_bad, &res));
+    if (res->bad & 1) return fail(EGS_E_ARG, "read-order offsets must run from 0 to m");
+    if (res->bad & 2) return fail(EGS_E_ARG, "a vertex has no out-edge");
+    if (res->bad & 4) return fail(EGS_E_ARG, "a successor is out of range");
+    if (res->mg > 0x7fffffffULL) return fail(EGS_E_ARG, "Error too high weights --> overflow (MG past INT32_MAX)");
+    if (ext_of_int) {
         HIP_TRY(hipMemcpyAsync(ext_of_int, s->d_sbig, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(egs::launch_degree_stats(s->d_ptr, n, s->d_misc + 2, s->stream));
-    egs::DevGame tmp{};
-    tmp.edges = s->d_edges;
-    tmp.m = m;
-    HIP_TRY(egs::launch_abs_wmax(tmp, s->d_misc + 3, s->stream));
-    HIP_TRY(hipMemcpyAsync(s->h_probe + kPinDeg + 2, s->d_misc + 2, 2 * sizeof(int), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    if (*h_mg > 0x7fffffffULL) return fail(EGS_E_ARG, "Error too high weights --> overflow (MG past INT32_MAX)");
-    const int32_t n0 = s->h_probe[kPinDeg + 1], mg = (int32_t)*h_mg;
-    s->max_outdeg = s->h_probe[kPinDeg + 2];
-    s->wmax = s->h_probe[kPinDeg + 3];
+        HIP_TRY(hipStreamSynchronize(s->stream));
+    }
+    const int32_t n0 = res->n0, mg = (int32_t)res->mg;
+    s->max_outdeg = res->dmax;
+    s->wmax = res->wmax;
     bind_game(s, n, n0, m, mg);
     if (n0_out) *n0_out = n0;
     if (mg_out) *mg_out = mg;
@@ -903,23 +927,13 @@ static int run_whole(egs_solver *s, int64_t limit, int *status) {
         __atomic_store_n(&res->done, 0u, __ATOMIC_RELEASE);     // no launch of this solver is running
         if (s->whole_rounds > 0) HIP_TRY(egs::launch_whole_prep(s->whole, g, s->d_whole, false, s->stream));
         HIP_TRY(egs::launch_whole(s->whole, a, s->stream));
-        bool got;
+        bool got = false;
         if (s->no_alloc) {
             HIP_TRY(hipMemcpyAsync(res, a.out, sizeof(*res), hipMemcpyDeviceToHost, s->stream));
             HIP_TRY(hipStreamSynchronize(s->stream));
             got = res->done == a.seq;
         } else {
-            // spin on the pinned word (stored last), asking the stream now and then so that a
-            // launch that ended without it is noticed
-            const volatile unsigned *done = &res->done;
-            hipError_t q = hipErrorNotReady;
-            while (q == hipErrorNotReady) {
-                for (int k = 0; k < 4096 && __atomic_load_n(done, __ATOMIC_ACQUIRE) != a.seq; k++) __builtin_ia32_pause();
-                if (__atomic_load_n(done, __ATOMIC_ACQUIRE) == a.seq) break;
-                q = hipStreamQuery(s->stream);
-            }
-            got = __atomic_load_n(done, __ATOMIC_ACQUIRE) == a.seq;
-            if (!got) HIP_TRY(q);
+            HIP_TRY(wait_word(s, &res->done, a.seq, &got));
         }
         if (!got) {
             *status = egs::kWholeNone;

@@ -2,6 +2,7 @@
 #pragma once
 
 #include <hip/hip_runtime.h>
+#include <limits.h>
 #include <stdint.h>
 
 struct egs_solver;
@@ -166,7 +167,47 @@ size_t whole_lds(const WholePlan &p);
 hipError_t launch_whole_prep(const WholePlan &p, const DevGame &g, WholeCtl *ctl, bool fresh, hipStream_t st);
 hipError_t launch_whole(const WholePlan &p, const WholeArgs &a, hipStream_t st);
 
-hipError_t launch_pack(const int *succ, const int *w, int2 *edges, int64_t m, hipStream_t st);
+// What a load has to know of its game, reduced on the device: one partial per workgroup, then
+// launch_load_finish adds them up and stores the record (`done`, its number, last).
+struct LoadPartial {
+    unsigned long long mg;                 // sum over the workgroup's rows of max(0, max -w)
+    int dmax, wmax;                        // largest out-degree and |w|
+};
+struct LoadResult {
+    unsigned long long mg;
+    int dmax, wmax, n0, bad;
+    unsigned done;
+};
+constexpr int kLoadGrid = 1024;            // workgroups (and partials) at most
+// Workgroup maxima and the sum of x, d and w to *out, by thread 0 (256 threads).
+__device__ __forceinline__ void load_partial(unsigned long long x, int d, int w, LoadPartial *out) {
+    __shared__ unsigned long long sx[4];
+    __shared__ int sd[4], sw[4];
+    for (int k = 32; k >= 1; k >>= 1) {
+        x += __shfl_xor(x, k, 64);
+        d = max(d, __shfl_xor(d, k, 64));
+        w = max(w, __shfl_xor(w, k, 64));
+    }
+    const int wid = threadIdx.x >> 6;
+    if ((threadIdx.x & 63) == 0) {
+        sx[wid] = x;
+        sd[wid] = d;
+        sw[wid] = w;
+    }
+    __syncthreads();
+    if (threadIdx.x == 0)
+        *out = LoadPartial{sx[0] + sx[1] + sx[2] + sx[3], max(max(sd[0], sd[1]), max(sd[2], sd[3])),
+                           max(max(sw[0], sw[1]), max(sw[2], sw[3]))};
+}
+
+// |w| as the host checks take it (INT_MIN counts as INT_MAX).
+__device__ __forceinline__ int load_abs(int w) { return w < 0 ? (w == INT_MIN ? INT_MAX : -w) : w; }
+// Device arrays into the solver's ptr and edges, with the statistics (mg is not summed).
+hipError_t launch_load_device(const int *ptr, const int *succ, const int *w, int n, int64_t m, int *ptr_out,
+                              int2 *edges, LoadPartial *part, int *nparts, hipStream_t st);
+hipError_t launch_load_finish(const LoadPartial *part, int nparts, const int *n0, const int *bad, unsigned seq,
+                              LoadResult *out, hipStream_t st);
+
 hipError_t launch_unpack(const uint32_t *packed, int shift, int2 *edges, int64_t m, hipStream_t st);
 hipError_t launch_transpose(const DevGame &g, int *tile_sum, int *fill, hipStream_t st);
 // The transpose as a two-level stable counting sort (egs_transpose.hip): cpred in ascending
@@ -178,7 +219,9 @@ int64_t transpose_counts_len(int n, int64_t m);
 bool transpose_sorted_fits(int n, int64_t m, int64_t counts_cap, int64_t items_cap);
 hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int *scan_tiles, int2 *items,
                                    hipStream_t st);
-hipError_t launch_exclusive_scan(const int *in, int n, int *tile_sum, int *out, hipStream_t st);
+// bad (may be null): a non-zero word makes the kernels return at once.
+hipError_t launch_exclusive_scan(const int *in, int n, int *tile_sum, int *out, hipStream_t st,
+                                 const int *bad = nullptr);
 constexpr int kTrTileEdges = 1 << 14;        // edges per tile of the sorted transpose
 
 // A game in read order on the device and the work arrays of its renaming (egs_ingest.hip).
@@ -188,8 +231,10 @@ struct ReadOrderBuffers {
     int *flag0, *pre0, *rev, *ext_of_int, *deg, *scan_tiles;   // n (+1) each; scan_tiles n/4096 + 1
 };
 hipError_t launch_read_order_check(const int *rptr, const int *rsucc, int n, int64_t m, int *bad, hipStream_t st);
-hipError_t launch_internalise(const ReadOrderBuffers &b, int n, int *ptr, int2 *edges, unsigned long long *mg,
-                              hipStream_t st);
+// bad (may be null): a non-zero word makes every kernel return at once.  The partials take the
+// place of flag0; their number goes to *nparts.
+hipError_t launch_internalise(const ReadOrderBuffers &b, int n, const int *bad, int *ptr, int2 *edges,
+                              LoadPartial **part, int *nparts, hipStream_t st);
 hipError_t launch_classify(const DevGame &g, int *counts, hipStream_t st);
 // in_slices: the slice set-up (init) already stored the initial state of the vertices up to
 // big_deg and counted, without listing, the active ones (no transpose: round 1 sweeps densely)
@@ -204,7 +249,6 @@ hipError_t launch_advance(const DevGame &g, int rounds, hipStream_t st);
 hipError_t launch_resume(const DevGame &g, int next, bool converged, hipStream_t st);
 hipError_t launch_prepare_reset(const DevGame &g, hipStream_t st);
 hipError_t launch_sum_stats(const DevGame &g, int nslots, unsigned long long *out, hipStream_t st);
-hipError_t launch_degree_stats(const int *ptr, int n, int *out, hipStream_t st);
 hipError_t launch_violations(const DevGame &g, unsigned long long *out, hipStream_t st);
 hipError_t launch_winning(const int *val, int n, unsigned *out, hipStream_t st);
 hipError_t launch_hbest_reset(const DevGame &g, hipStream_t st);
@@ -235,7 +279,6 @@ struct CertResult {
     int cap_hit;         // some candidate ran out of passes (neither converged nor diverged)
     int last_passes;     // passes of the last candidate that converged (0: none did)
 };
-hipError_t launch_abs_wmax(const DevGame &g, int *out, hipStream_t st);
 int gap_candidates(const int *win, const int *flo, int wmax, int mg, int64_t *out, int max_out);
 // The value histogram of the next attempt, queued with its read-back into the pinned area.
 hipError_t certify_prefetch(const DevGame &g, const CertBuffers &cb, int wmax, hipStream_t st);

@@ -55,9 +55,14 @@ __global__ __launch_bounds__(256) void k_ro_place_edges(const int2 *__restrict__
 }
 
 // meta = {1, n0 = owner-0 count (pre0[n]), MG}; MG fits 31 bits (checked on the host).
-__global__ void k_ro_meta(const int *__restrict__ pre0, int n, const unsigned long long *__restrict__ mg,
-                          ReadOrderMeta *__restrict__ meta) {
-    if (blockIdx.x == 0 && threadIdx.x == 0) *meta = ReadOrderMeta{1, pre0[n], (int)*mg, 0};
+__global__ __launch_bounds__(256) void k_ro_meta(const int *__restrict__ pre0, int n,
+                                                 const LoadPartial *__restrict__ part, int nparts,
+                                                 ReadOrderMeta *__restrict__ meta) {
+    __shared__ LoadPartial total;
+    unsigned long long mg = 0;
+    for (int i = threadIdx.x; i < nparts; i += blockDim.x) mg += part[i].mg;
+    load_partial(mg, 0, 0, &total);
+    if (threadIdx.x == 0) *meta = ReadOrderMeta{1, pre0[n], (int)total.mg, 0};
 }
 
 // The slice's descriptors of games internalised on the device get their owner count and MG.
@@ -689,12 +694,12 @@ int egs_server_submit_read_order(egs_server *s, int32_t n, int64_t m, const uint
     const size_t ptr_b = 4 * ((size_t)n + 1), n1 = al256(ptr_b);
     const size_t body = large ? footprint_large(n, m, shift > 0) : footprint(n, m, wm);
     const size_t bytes = body + al256(4 * (size_t)n);            // + ext_of_int
-    // work space: the read-order arrays, the partition's scans, the internal int2 edges, MG
+    // work space: the read-order arrays, the partition's scans, the internal int2 edges
     const size_t o_rptr = al256((size_t)n), o_rsucc = o_rptr + n1, o_rw = o_rsucc + al256(4 * (size_t)m);
     const size_t in_end = o_rw + al256(4 * (size_t)m);
     const size_t o_flag0 = in_end, o_pre0 = o_flag0 + n1, o_rev = o_pre0 + n1, o_deg = o_rev + n1;
     const size_t o_tiles = o_deg + n1, o_edges = o_tiles + al256(4 * ((size_t)n / 4096 + 4));
-    const size_t o_mg = o_edges + al256(8 * (size_t)m), tbytes = o_mg + 256;
+    const size_t tbytes = o_edges + al256(8 * (size_t)m);
     if (!s->alloc.fits(bytes)) return sfail(EGS_E_CAPACITY, "arena full (%zu bytes wanted)", bytes);
     int sb = 0;
     int rc = staging_reserve(s, in_end, &sb);
@@ -725,14 +730,15 @@ int egs_server_submit_read_order(egs_server *s, int32_t n, int64_t m, const uint
     b.ext_of_int = ext;
     b.deg = (int *)(T + o_deg);
     b.scan_tiles = (int *)(T + o_tiles);
-    unsigned long long *d_mg = (unsigned long long *)(T + o_mg);
-    SHIP(egs::launch_internalise(b, n, (int *)base, (int2 *)(T + o_edges), d_mg, s->copy));
+    egs::LoadPartial *part = nullptr;
+    int nparts = 0;
+    SHIP(egs::launch_internalise(b, n, nullptr, (int *)base, (int2 *)(T + o_edges), &part, &nparts, s->copy));
     const size_t o_e = n1, o_w = o_e + al256(4 * (size_t)m);
     hipLaunchKernelGGL(egs::k_ro_place_edges, dim3(egs::grid_for(m, 256, 4096)), dim3(256), 0, s->copy,
                        (const int2 *)(T + o_edges), m, shift, large && !shift ? 1 : 0, (void *)(base + o_e),
                        (int *)(base + o_w));
-    hipLaunchKernelGGL(egs::k_ro_meta, dim3(1), dim3(64), 0, s->copy, (const int *)b.pre0, n,
-                       (const unsigned long long *)d_mg, s->d_meta + ticket);
+    hipLaunchKernelGGL(egs::k_ro_meta, dim3(1), dim3(256), 0, s->copy, (const int *)b.pre0, n,
+                       (const egs::LoadPartial *)part, nparts, s->d_meta + ticket);
     SHIP(hipGetLastError());
     Transient tr{tat, tbytes, nullptr};
     if (!s->spare_events.empty()) {

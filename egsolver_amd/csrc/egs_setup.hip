@@ -5,6 +5,9 @@
 // Replaces EG_gpu_traspose_graph + cuSPARSE csr2csc (src/dev_EG_alg.cu:277-290,
 // src/csr2csc.cu:54-66).  The predecessor weights the reference also transposes are never
 // read by its kernels (src/dev_EG_alg.cu:283) and are not built here.
+#include <algorithm>
+#include <climits>
+
 #include "egs_device.h"
 #include "egs_internal.h"
 
@@ -14,11 +17,59 @@ namespace egs {
 // setup kernels
 // ---------------------------------------------------------------------------------------
 
-__global__ void k_pack_edges(const int *__restrict__ succ, const int *__restrict__ w,
-                             int2 *__restrict__ edges, int64_t m) {
-    for (int64_t e = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; e < m;
-         e += (int64_t)gridDim.x * blockDim.x) {
-        edges[e] = make_int2(succ[e], w[e]);
+// A game's device arrays into the solver's: offsets copied, edges interleaved, and the largest
+// degree and |w| taken on the way.  HBM-bound (16 bytes an edge).  A partial per workgroup, not
+// an atomic per wave: 8,192 same-address atomics made the |w| pass 95 us and the degree pass
+// 17 us at n = 87,148 (784K edges); the three passes take 6.2 us together now.
+__global__ __launch_bounds__(256) void k_load_device(const int *__restrict__ ptr, const int *__restrict__ succ,
+                                                     const int *__restrict__ w, int n, int64_t m,
+                                                     int *__restrict__ ptr_out, int2 *__restrict__ edges,
+                                                     LoadPartial *__restrict__ part) {
+    const int64_t step = (int64_t)gridDim.x * blockDim.x, t0 = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int dmax = 0, wmax = 0;
+    for (int64_t v = t0; v <= n; v += step) {
+        const int s = ptr[v];
+        ptr_out[v] = s;
+        if (v < n) dmax = max(dmax, ptr[v + 1] - s);
+    }
+    for (int64_t e0 = t0; e0 < m; e0 += 4 * step) {
+        int su[4], we[4];
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int64_t e = e0 + k * step;
+            su[k] = e < m ? succ[e] : 0;
+            we[k] = e < m ? w[e] : 0;
+        }
+#pragma unroll
+        for (int k = 0; k < 4; k++) {
+            const int64_t e = e0 + k * step;
+            if (e < m) edges[e] = make_int2(su[k], we[k]);
+            wmax = max(wmax, load_abs(we[k]));
+        }
+    }
+    load_partial(0, dmax, wmax, part + blockIdx.x);
+}
+
+__global__ __launch_bounds__(256) void k_load_finish(const LoadPartial *__restrict__ part, int nparts, const int *n0,
+                                                     const int *bad, unsigned seq, LoadResult *out) {
+    __shared__ LoadPartial total;
+    unsigned long long mg = 0;
+    int d = 0, w = 0;
+    for (int i = threadIdx.x; i < nparts; i += blockDim.x) {
+        const LoadPartial p = part[i];
+        mg += p.mg;
+        d = max(d, p.dmax);
+        w = max(w, p.wmax);
+    }
+    load_partial(mg, d, w, &total);
+    if (threadIdx.x == 0) {
+        out->mg = total.mg;
+        out->dmax = total.dmax;
+        out->wmax = total.wmax;
+        out->n0 = n0 ? *n0 : 0;
+        out->bad = bad ? *bad : 0;
+        __threadfence_system();
+        __hip_atomic_store(&out->done, seq, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
     }
 }
 
@@ -37,8 +88,9 @@ constexpr int SCAN_ITEMS = 16;
 constexpr int SCAN_TILE = SCAN_THREADS * SCAN_ITEMS;
 
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_tiles(const int *__restrict__ cnt, int n,
-                                                             int *__restrict__ tile_sum) {
+                                                             int *__restrict__ tile_sum, const int *bad) {
     __shared__ int lds[SCAN_THREADS / 64];
+    if (bad && *bad) return;
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
     int s = 0;
 #pragma unroll
@@ -51,8 +103,9 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_tiles(const int *__restri
     if (threadIdx.x == 0) tile_sum[blockIdx.x] = total;
 }
 
-__global__ __launch_bounds__(SCAN_THREADS) void k_scan_sums(int *__restrict__ tile_sum, int tiles) {
+__global__ __launch_bounds__(SCAN_THREADS) void k_scan_sums(int *__restrict__ tile_sum, int tiles, const int *bad) {
     __shared__ int lds[SCAN_THREADS / 64];
+    if (bad && *bad) return;
     int carry = 0;
     for (int b = 0; b < tiles; b += SCAN_THREADS) {
         int i = b + threadIdx.x;
@@ -66,9 +119,10 @@ __global__ __launch_bounds__(SCAN_THREADS) void k_scan_sums(int *__restrict__ ti
 
 __global__ __launch_bounds__(SCAN_THREADS) void k_scan_apply(const int *__restrict__ cnt, int n,
                                                              const int *__restrict__ tile_off,
-                                                             int *__restrict__ out) {
+                                                             int *__restrict__ out, const int *bad) {
     __shared__ int items[SCAN_TILE];
     __shared__ int lds[SCAN_THREADS / 64];
+    if (bad && *bad) return;
     const int64_t base = (int64_t)blockIdx.x * SCAN_TILE;
     // coalesced load of the tile into LDS
 #pragma unroll
@@ -242,16 +296,6 @@ hipError_t launch_winning(const int *val, int n, unsigned *out, hipStream_t st) 
     return hipGetLastError();
 }
 
-__global__ void k_degree_max(const int *__restrict__ ptr, int n, int *__restrict__ out) {
-    int mx = 0;
-    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < n;
-         v += (int64_t)gridDim.x * blockDim.x) {
-        mx = max(mx, ptr[v + 1] - ptr[v]);
-    }
-    for (int d = 32; d >= 1; d >>= 1) mx = max(mx, __shfl_xor(mx, d, 64));
-    if ((threadIdx.x & 63) == 0) atomicMax(out, mx);
-}
-
 // out[0..3]: the summed statistics; out[4]: the last round that ran; out[5]: the size of the
 // next round's input list (round ring[14]; 0 = the least fixpoint), so that one read-back
 // closes a run.
@@ -310,20 +354,27 @@ hipError_t launch_unpack(const uint32_t *packed, int shift, int2 *edges, int64_t
     return hipGetLastError();
 }
 
-hipError_t launch_pack(const int *succ, const int *w, int2 *edges, int64_t m, hipStream_t st) {
-    if (m > 0)
-        hipLaunchKernelGGL(k_pack_edges, dim3(grid_for(m, 256, 8192)), dim3(256), 0, st, succ, w, edges, m);
+hipError_t launch_load_device(const int *ptr, const int *succ, const int *w, int n, int64_t m, int *ptr_out,
+                              int2 *edges, LoadPartial *part, int *nparts, hipStream_t st) {
+    *nparts = grid_for(std::max<int64_t>(m / 4, n), 256, kLoadGrid);
+    hipLaunchKernelGGL(k_load_device, dim3(*nparts), dim3(256), 0, st, ptr, succ, w, n, m, ptr_out, edges, part);
+    return hipGetLastError();
+}
+
+hipError_t launch_load_finish(const LoadPartial *part, int nparts, const int *n0, const int *bad, unsigned seq,
+                              LoadResult *out, hipStream_t st) {
+    hipLaunchKernelGGL(k_load_finish, dim3(1), dim3(256), 0, st, part, nparts, n0, bad, seq, out);
     return hipGetLastError();
 }
 
 // Exclusive scan of in[0..n) into out[0..n] (out[n] = total); in == out is allowed (each
 // tile is read whole into LDS before it is written).  tile_sum holds ceil(n / SCAN_TILE).
-hipError_t launch_exclusive_scan(const int *in, int n, int *tile_sum, int *out, hipStream_t st) {
+hipError_t launch_exclusive_scan(const int *in, int n, int *tile_sum, int *out, hipStream_t st, const int *bad) {
     const int tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
     if (tiles == 0) return hipMemsetAsync(out, 0, sizeof(int), st);
-    hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(SCAN_THREADS), 0, st, in, n, tile_sum);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, st, tile_sum, tiles);
-    hipLaunchKernelGGL(k_scan_apply, dim3(tiles), dim3(SCAN_THREADS), 0, st, in, n, tile_sum, out);
+    hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(SCAN_THREADS), 0, st, in, n, tile_sum, bad);
+    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, st, tile_sum, tiles, bad);
+    hipLaunchKernelGGL(k_scan_apply, dim3(tiles), dim3(SCAN_THREADS), 0, st, in, n, tile_sum, out, bad);
     return hipGetLastError();
 }
 
@@ -333,11 +384,7 @@ hipError_t launch_transpose(const DevGame &g, int *tile_sum, int *fill, hipStrea
     hipError_t err;
     if ((err = hipMemsetAsync(fill, 0, sizeof(int) * (size_t)(n + 1), st)) != hipSuccess) return err;
     hipLaunchKernelGGL(k_indegree, dim3(grid_for(m, 256, 4096)), dim3(256), 0, st, g.edges, m, fill);
-    const int tiles = (n + SCAN_TILE - 1) / SCAN_TILE;
-    hipLaunchKernelGGL(k_scan_tiles, dim3(tiles), dim3(SCAN_THREADS), 0, st, fill, n, tile_sum);
-    hipLaunchKernelGGL(k_scan_sums, dim3(1), dim3(SCAN_THREADS), 0, st, tile_sum, tiles);
-    hipLaunchKernelGGL(k_scan_apply, dim3(tiles), dim3(SCAN_THREADS), 0, st, fill, n, tile_sum,
-                       const_cast<int *>(g.cptr));
+    if ((err = launch_exclusive_scan(fill, n, tile_sum, const_cast<int *>(g.cptr), st)) != hipSuccess) return err;
     if ((err = hipMemcpyAsync(fill, g.cptr, sizeof(int) * (size_t)(n + 1), hipMemcpyDeviceToDevice, st)) != hipSuccess)
         return err;
     hipLaunchKernelGGL(k_scatter_preds, dim3(grid_for(n, 256, 4096)), dim3(256), 0, st, g.ptr, g.edges,
@@ -376,13 +423,6 @@ hipError_t launch_violations(const DevGame &g, unsigned long long *out, hipStrea
     hipError_t err = hipMemsetAsync(out, 0, sizeof(unsigned long long), st);
     if (err != hipSuccess) return err;
     hipLaunchKernelGGL(k_violations, dim3(grid_for(g.n, 256, 2048)), dim3(256), 0, st, g, out);
-    return hipGetLastError();
-}
-
-hipError_t launch_degree_stats(const int *ptr, int n, int *out, hipStream_t st) {
-    hipError_t err = hipMemsetAsync(out, 0, sizeof(int), st);
-    if (err != hipSuccess) return err;
-    hipLaunchKernelGGL(k_degree_max, dim3(grid_for(n, 256, 1024)), dim3(256), 0, st, ptr, n, out);
     return hipGetLastError();
 }
 
