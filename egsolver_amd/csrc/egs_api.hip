@@ -214,6 +214,11 @@ struct egs_solver {
     int2 *d_edges = nullptr;
     unsigned long long *d_stats = nullptr, *d_statsum = nullptr;
     int *h_probe = nullptr;   // pinned: per-batch counter probes + misc readbacks
+    char *h_small = nullptr;  // behind them, out_small bytes for small read-backs
+    size_t out_small = 0;
+    char *h_out = nullptr;    // pinned, 2 x out_half bytes, made at the first larger read-back
+    size_t out_half = 0;
+    bool mirrored = false;    // h_small holds the values of the run that has just converged
     int probe_want[2] = {kProbeWant, kProbeWant};   // where each probe slot holds ring[13]
     hipEvent_t ev_probe[2] = {nullptr, nullptr};
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
@@ -321,6 +326,50 @@ static hipError_t wait_word(egs_solver *s, const unsigned *done, unsigned seq, b
         if (q != hipErrorNotReady) return q;         // the stream was done before this last look
         q = hipStreamQuery(s->stream);
     }
+}
+
+// `bytes` of device memory to a pageable host buffer, after the work queued so far.  A copy
+// into pageable memory runs at 2-4 GB/s up to about 1 MB and 16 GB/s beyond (350 KB took
+// 154 us, 16 MB 1.02 ms); into pinned memory it takes 14 us and 0.30 ms.  So it goes through
+// pinned memory: the small area made with the solver, or two halves of a buffer made at the
+// first larger read, one filling while the other is copied out by the packing threads.
+constexpr size_t kOutSmall = 128 << 10;    // the small area at most
+constexpr size_t kOutHalf = 1 << 20;       // a half of the large buffer at most
+static hipError_t read_back(egs_solver *s, void *dst, const void *src, size_t bytes) {
+    hipError_t e;
+    if (bytes <= s->out_small) {
+        e = hipMemcpyAsync(s->h_small, src, bytes, hipMemcpyDeviceToHost, s->stream);
+        if (e == hipSuccess) e = hipStreamSynchronize(s->stream);
+        if (e == hipSuccess) memcpy(dst, s->h_small, bytes);
+        return e;
+    }
+    const size_t half = std::min(bytes, kOutHalf);
+    if (!s->no_alloc && s->out_half < half) {
+        if (s->h_out) (void)hipHostFree(s->h_out);
+        s->h_out = nullptr;
+        s->out_half = 0;
+        if (hipHostMalloc((void **)&s->h_out, 2 * half, hipHostMallocDefault) == hipSuccess) s->out_half = half;
+        else (void)hipGetLastError();      // the plain copy below needs no buffer
+    }
+    if (s->out_half < half) {
+        e = hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, s->stream);
+        return e == hipSuccess ? hipStreamSynchronize(s->stream) : e;
+    }
+    const int64_t chunks = (int64_t)((bytes + half - 1) / half);
+    auto len = [&](int64_t c) { return std::min(half, bytes - (size_t)c * half); };
+    for (int64_t c = 0; c <= chunks; c++) {
+        if (c > 0) {                       // chunk c - 1 has arrived before chunk c is queued behind it
+            e = hipStreamSynchronize(s->stream);
+            if (e != hipSuccess) return e;
+        }
+        if (c < chunks) {
+            e = hipMemcpyAsync(s->h_out + (size_t)(c & 1) * half, (const char *)src + (size_t)c * half, len(c),
+                               hipMemcpyDeviceToHost, s->stream);
+            if (e != hipSuccess) return e;
+        }
+        if (c > 0) egs_pk_copy((char *)dst + (size_t)(c - 1) * half, s->h_out + (size_t)((c - 1) & 1) * half, len(c - 1));
+    }
+    return hipSuccess;
 }
 
 // The record of a load (launch_load_finish last on the stream), on the host.  The no-allocation
@@ -471,6 +520,7 @@ int egs_solver_destroy(egs_solver *s) {
     drop_graphs(s);
     if (s->block) (void)hipFree(s->block);
     if (s->h_probe) (void)hipHostFree(s->h_probe);
+    if (s->h_out) (void)hipHostFree(s->h_out);
     for (auto &e : s->ev_probe) if (e) (void)hipEventDestroy(e);
     if (s->ev_a) (void)hipEventDestroy(s->ev_a);
     if (s->ev_b) (void)hipEventDestroy(s->ev_b);
@@ -503,10 +553,13 @@ int egs_solver_create(int device, int32_t n_cap, int64_t m_cap, egs_solver **out
         return fail(EGS_E_NOMEM, "hipMalloc of %zu bytes failed", L.total);
     }
     bind_layout(s, (char *)s->block, L);
-    if (hipHostMalloc((void **)&s->h_probe, 4 * (kPinProbe + 2 * kProbeStride), hipHostMallocDefault) != hipSuccess) {
+    constexpr size_t kProbeBytes = 4 * (kPinProbe + 2 * kProbeStride);
+    s->out_small = std::min(kOutSmall, 4 * ((size_t)n_cap + 32));
+    if (hipHostMalloc((void **)&s->h_probe, kProbeBytes + s->out_small, hipHostMallocDefault) != hipSuccess) {
         egs_solver_destroy(s);
         return fail(EGS_E_NOMEM, "hipHostMalloc failed");
     }
+    s->h_small = (char *)s->h_probe + kProbeBytes;
     s->h_probe[kPinOne] = 1;
     if (hipStreamCreateWithFlags(&s->stream, hipStreamNonBlocking) != hipSuccess ||
         hipEventCreate(&s->ev_probe[0]) != hipSuccess || hipEventCreate(&s->ev_probe[1]) != hipSuccess ||
@@ -640,8 +693,8 @@ int egs_solver_load_read_order(egs_solver *s, int mem, int32_t n, int64_t m, con
     if (res->bad & 4) return fail(EGS_E_ARG, "a successor is out of range");
     if (res->mg > 0x7fffffffULL) return fail(EGS_E_ARG, "Error too high weights --> overflow (MG past INT32_MAX)");
     if (ext_of_int) {
-        HIP_TRY(hipMemcpyAsync(ext_of_int, s->d_sbig, sizeof(int) * (size_t)n, hipMemcpyDeviceToHost, s->stream));
-        HIP_TRY(hipStreamSynchronize(s->stream));
+        s->mirrored = false;
+        HIP_TRY(read_back(s, ext_of_int, s->d_sbig, sizeof(int) * (size_t)n));
     }
     const int32_t n0 = res->n0, mg = (int32_t)res->mg;
     s->max_outdeg = res->dmax;
@@ -701,6 +754,7 @@ static void bind_game(egs_solver *s, int32_t n, int32_t n0, int64_t m, int32_t m
     s->loaded = true;
     s->prepared = false;
     s->whole = egs::WholePlan{};
+    s->mirrored = false;
 }
 
 static int pick_shape(egs_solver *s, const egs_options *o) {
@@ -853,6 +907,7 @@ static bool takes_whole(const egs_options *o) {
 // not begun, else the counters and lists, with the values reached and the next round a full
 // sweep (none when the run has converged).
 static int leave_whole(egs_solver *s) {
+    s->mirrored = false;
     if (s->whole.nb == 0) return EGS_OK;
     s->whole.nb = 0;
     if (s->whole_rounds == 0 && !s->st.converged) return prepare_rounds(s);
@@ -912,6 +967,8 @@ static int run_whole(egs_solver *s, int64_t limit, int *status) {
     // the result comes back through the pinned block, which the kernel stores into; the
     // no-allocation solver has none and copies it from device memory
     egs::WholeResult *res = (egs::WholeResult *)(s->h_probe + kPinWhole);
+    // one workgroup stores its values into the small read-back area on its way out
+    a.mirror = s->whole.nb == 1 && 4 * (size_t)g.n <= s->out_small ? (int *)s->h_small : nullptr;
     a.out = s->no_alloc ? (egs::WholeResult *)s->d_misc : res;
     *status = egs::kWholeNone;
     WholeRoom room(s);
@@ -962,6 +1019,7 @@ static int run_whole(egs_solver *s, int64_t limit, int *status) {
         s->cert_cap = res->cap;
         limit -= ran;
         *status = res->status;
+        s->mirrored = a.mirror != nullptr;
     }
     s->st.phases = s->whole_rounds;
     s->st.processed = s->whole_st.processed;
@@ -985,6 +1043,7 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     s->cert_pass_hint = 0;
     s->whole_rounds = 0;
     s->whole_st = egs_stats{};
+    s->mirrored = false;
     s->whole = takes_whole(opt) ? egs::whole_plan(s->g.n, s->g.m, s->g.mg, s->wmax, s->max_outdeg, s->whole_max_nb) : egs::WholePlan{};
     if (s->whole.nb > 0) {
         HIP_TRY(egs::launch_whole_prep(s->whole, s->g, s->d_whole, true, s->stream));
@@ -1173,9 +1232,13 @@ int egs_solver_stats(egs_solver *s, egs_stats *st) {
 
 int egs_solver_read_values(egs_solver *s, int32_t *host_values) {
     if (!s || !s->loaded || !host_values) return fail(EGS_E_STATE, "egs_solver_read_values: nothing to read");
+    const size_t bytes = sizeof(int) * (size_t)s->g.n;
+    if (s->mirrored) {
+        memcpy(host_values, s->h_small, bytes);
+        return EGS_OK;
+    }
     HIP_TRY(hipSetDevice(s->device));
-    HIP_TRY(hipMemcpyAsync(host_values, s->d_val, sizeof(int) * (size_t)s->g.n, hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
+    HIP_TRY(read_back(s, host_values, s->d_val, bytes));
     return EGS_OK;
 }
 
@@ -1184,9 +1247,8 @@ int egs_solver_read_winning(egs_solver *s, uint32_t *host_bits) {
     HIP_TRY(hipSetDevice(s->device));
     // the proof bitmaps are idle outside an attempt: the first holds ceil(n/32) words
     HIP_TRY(egs::launch_winning(s->d_val, s->g.n, s->d_bits, s->stream));
-    HIP_TRY(hipMemcpyAsync(host_bits, s->d_bits, sizeof(uint32_t) * (((size_t)s->g.n + 31) / 32), hipMemcpyDeviceToHost,
-                           s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
+    s->mirrored = false;                     // the small read-back area is used
+    HIP_TRY(read_back(s, host_bits, s->d_bits, sizeof(uint32_t) * (((size_t)s->g.n + 31) / 32)));
     return EGS_OK;
 }
 
@@ -1237,8 +1299,7 @@ int egs_solver_top_certificate(egs_solver *s, int32_t max_passes, int64_t *host_
                                          s->sh.use_wave != 0, s->stream, cr);
     if (got == -1) return fail(EGS_E_HIP, "certificate: %s", hipGetErrorString(hipGetLastError()));
     if (got == -2) return fail(EGS_E_ARG, "certificate: potentials of this game could overflow 64 bits");
-    HIP_TRY(hipMemcpyAsync(host_h, s->d_h, sizeof(int64_t) * (size_t)s->g.n, hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
+    HIP_TRY(read_back(s, host_h, s->d_h, sizeof(int64_t) * (size_t)s->g.n));
     if (passes) *passes = cr.passes;
     return got;
 }

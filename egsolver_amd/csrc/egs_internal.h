@@ -116,7 +116,8 @@ struct LaunchShape {
 constexpr int kWholeMaxNb = 256;           // workgroups at most
 constexpr int kWholeGroups = 8;            // groups of workgroups in a vote
 constexpr int64_t kWholeWait = 400000;     // barrier wait limit (4 ms) before a launch gives up
-constexpr int kWholeOneN = 5999, kWholeOneM = 16384;   // one workgroup up to this size
+constexpr int kWholeOneN = 5999, kWholeOneM = 8192;    // one workgroup up to this size (8 edges a thread; with
+                                           // 16 it spills: n = 4,000, degree 4: 160 us against 120 on 8 workgroups)
 // Vertices + edges per workgroup while workgroups are left.  Device time of a solve (degree
 // 2..16, us) at shares of 1,536 / 2,304 / 3,072 / 4,608 / 6,144: n = 9,973: 71 / 71 / 74 / 85 / 93;
 // n = 30,011: 113 / 100 / 96 / 102 / 101; n = 87,148: 166 / 166 / 166 / 170 / 161.
@@ -148,6 +149,7 @@ struct WholeArgs {
     long long *h;
     WholeCtl *ctl;
     WholeResult *out;
+    int *mirror;                           // a copy of the values for the host (one workgroup; may be null)
     int nbmax;                             // vertices of a workgroup at most (LDS)
     int64_t limit;                         // rounds of this launch at most
     int64_t round0, next_cert;             // rounds already run; the round of the next attempt

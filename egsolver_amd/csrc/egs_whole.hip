@@ -472,7 +472,10 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
         }
     }
     if (ONE)
-        for (int i = tid; i < nb; i += T) a.val[i] = own[i];
+        for (int i = tid; i < nb; i += T) {
+            a.val[i] = own[i];
+            if (a.mirror) a.mirror[i] = own[i];
+        }
     // statistics: edges and lifts of the launch (processed = vertices times its rounds)
     {
         const unsigned long long lf = lifted;
@@ -748,6 +751,7 @@ __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
         const int v = q * T + tid;
         if (v < a.n) {
             a.val[v] = val[q];
+            if (a.mirror) a.mirror[v] = val[q];
             if (a.rise) a.rise[v] = rise[q];
         }
     }

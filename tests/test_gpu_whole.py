@@ -30,7 +30,7 @@ def _rounds(s, **opt):
 # complete digraphs; hubs in one workgroup's share and beyond a share; the largest shares
 GAMES = [(2, 0, 1, 1, 0, 5), (61, 1, 2, 6, 0, 10), (1024, 1, 1, 16, 0, 50), (1025, 1, 1, 16, 0, 50), (1024, 1, 1, 17, 0, 50),
          (2048, 0, 4, 4, 0, 10), (2049, 0, 4, 4, 0, 10), (2048, 1, 1, 8, 0, 30), (1500, 2, 1, 300, 1.8, 30),
-         (4096, 0, 4, 4, 0, 10), (4097, 0, 4, 4, 0, 10), (5999, 0, 1, 1, 0, 20), (6000, 0, 1, 1, 0, 20),
+         (2731, 0, 3, 3, 0, 10), (2730, 0, 3, 3, 0, 10), (5999, 0, 1, 1, 0, 20), (6000, 0, 1, 1, 0, 20),
          (130, 3, 0, 0, 0, 40), (400, 3, 0, 0, 0, 40), (12345, 1, 1, 9, 0, 100), (20011, 2, 1, 9000, 1.9, 60),
          (60000, 2, 1, 13000, 2.1, 60), (87149, 1, 2, 16, 0, 1000), (203000, 0, 8, 8, 0, 100), (204000, 0, 8, 8, 0, 100)]
 
