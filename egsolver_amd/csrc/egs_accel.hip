@@ -27,6 +27,7 @@
 #include <algorithm>
 #include <climits>
 
+#include "egs_bins.h"
 #include "egs_device.h"
 #include "egs_internal.h"
 
@@ -156,6 +157,11 @@ constexpr int kCntSlots = 64;
 
 constexpr int kBigU = 4;   // edges in flight per lane in the workgroup-per-vertex kernels
 constexpr int kClosureU = 4;   // edges in flight per thread in k_closure (one thread per vertex)
+// A pass is binned after one that changed this part of the vertices.  With hubs, which nearly
+// every change makes k_bf_all read whole, much sooner: on the skewed 2^20 game its passes
+// over the first candidate took 186 us and more at 1/64 changed, 60 us at a few hundred, a
+// binned pass 50 us.
+constexpr int kBinPassPart = 64, kBinPassPartHubs = 2048;
 constexpr int kBfU = 2;        // edges in flight per lane in k_bf_pass
 
 // Closure check, member count and the first pass of the longest-path game, in one sweep
@@ -514,12 +520,18 @@ __global__ __launch_bounds__(256) void k_closure_big(DevGame g, int B, int last,
 // nothing leaves a closed D and a fixpoint on it.  Changed vertices set their bit in `cur`;
 // `clear` (the bitmap of pass p+1, last read in pass p-1) is zeroed.  The pass returns at
 // once when pass p-1 changed nothing or the potentials have passed the divergence bound.
+// A pass does nothing when the one before changed nothing, or when it changed so many vertices
+// (at least bin_min, if that is not 0) that the binned kernels take it.
+__device__ __forceinline__ bool bf_idle(int changed, int bin_min) {
+    return changed == 0 || (bin_min && changed >= bin_min);
+}
+
 template <int G>
 __device__ __forceinline__ void bf_pass_part(const DevGame &g, long long *__restrict__ h, long long bound,
                                              const unsigned *__restrict__ prev, unsigned *__restrict__ cur,
                                              unsigned *__restrict__ clear, int p, int *__restrict__ cnt,
-                                             int *__restrict__ flags, int bid, int nblk) {
-    if (cnt[(p - 1) % kCntSlots] == 0 || flags[1]) return;
+                                             int *__restrict__ flags, int bin_min, int bid, int nblk) {
+    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || flags[1]) return;
     const int64_t words = bm_total(g.n);
     for (int64_t i = (int64_t)bid * blockDim.x + threadIdx.x; i < words; i += (int64_t)nblk * blockDim.x)
         clear[i] = 0u;
@@ -639,17 +651,18 @@ template <int G>
 __global__ __launch_bounds__(256) void k_bf_pass(DevGame g, long long *__restrict__ h, long long bound,
                                                  const unsigned *__restrict__ prev, unsigned *__restrict__ cur,
                                                  unsigned *__restrict__ clear, int p, int *__restrict__ cnt,
-                                                 int *__restrict__ flags) {
-    bf_pass_part<G>(g, h, bound, prev, cur, clear, p, cnt, flags, blockIdx.x, gridDim.x);
+                                                 int *__restrict__ flags, int bin_min) {
+    bf_pass_part<G>(g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, blockIdx.x, gridDim.x);
 }
 
 // Pass p for the vertices of the big list (big_deg < deg <= huge_deg; launched after
 // k_bf_pass for the same p), one workgroup each, with the same rule and updates.
 __device__ __forceinline__ void bf_big_part(const DevGame &g, long long *__restrict__ h, long long bound,
                                             const unsigned *__restrict__ prev, unsigned *__restrict__ cur, int p,
-                                            int *__restrict__ cnt, int *__restrict__ flags, int bid, int nblk) {
+                                            int *__restrict__ cnt, int *__restrict__ flags, int bin_min, int bid,
+                                            int nblk) {
     __shared__ long long sm[4];
-    if (cnt[(p - 1) % kCntSlots] == 0 || flags[1]) return;
+    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || flags[1]) return;
     const long long scale = (long long)g.n + 1;
     const int nb = g.ring[9], items = nb;               // the huge list: k_bf_huge
     int local = 0;
@@ -711,7 +724,7 @@ __device__ __forceinline__ void bf_big_part(const DevGame &g, long long *__restr
 __global__ __launch_bounds__(256) void k_bf_big(DevGame g, long long *__restrict__ h, long long bound,
                                                 const unsigned *__restrict__ prev, unsigned *__restrict__ cur,
                                                 int p, int *__restrict__ cnt, int *__restrict__ flags) {
-    bf_big_part(g, h, bound, prev, cur, p, cnt, flags, blockIdx.x, gridDim.x);
+    bf_big_part(g, h, bound, prev, cur, p, cnt, flags, 0, blockIdx.x, gridDim.x);
 }
 
 // Pass p for the vertices above huge_deg, each shared by up to `per` workgroups: a
@@ -724,11 +737,12 @@ constexpr int kHugeChunkBf = 2048;
 
 __device__ __forceinline__ void bf_huge_part(const DevGame &g, long long *__restrict__ h, long long bound,
                                              const unsigned *__restrict__ prev, unsigned *__restrict__ cur, int p,
-                                             int *__restrict__ cnt, int *__restrict__ flags, int bid, int nblk) {
+                                             int *__restrict__ cnt, int *__restrict__ flags, int bin_min, int bid,
+                                             int nblk) {
     __shared__ long long sm[4];
     __shared__ long long s_best;
     __shared__ int s_last, s_flag;
-    if (cnt[(p - 1) % kCntSlots] == 0 || flags[1]) return;
+    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || flags[1]) return;
     const int nh = g.ring[10];
     if (nh == 0) return;
     const long long scale = (long long)g.n + 1;
@@ -814,7 +828,7 @@ __device__ __forceinline__ void bf_huge_part(const DevGame &g, long long *__rest
 __global__ __launch_bounds__(256) void k_bf_huge(DevGame g, long long *__restrict__ h, long long bound,
                                                  const unsigned *__restrict__ prev, unsigned *__restrict__ cur,
                                                  int p, int *__restrict__ cnt, int *__restrict__ flags) {
-    bf_huge_part(g, h, bound, prev, cur, p, cnt, flags, blockIdx.x, gridDim.x);
+    bf_huge_part(g, h, bound, prev, cur, p, cnt, flags, 0, blockIdx.x, gridDim.x);
 }
 
 // One pass over every member in one launch: workgroups [0, grid) run the pass over the
@@ -826,11 +840,158 @@ template <int G>
 __global__ __launch_bounds__(256) void k_bf_all(DevGame g, long long *__restrict__ h, long long bound,
                                                 const unsigned *__restrict__ prev, unsigned *__restrict__ cur,
                                                 unsigned *__restrict__ clear, int p, int *__restrict__ cnt,
-                                                int *__restrict__ flags, int grid, int big_grid, int huge_grid) {
+                                                int *__restrict__ flags, int bin_min, int grid, int big_grid,
+                                                int huge_grid) {
     const int b = blockIdx.x;
-    if (b < grid) bf_pass_part<G>(g, h, bound, prev, cur, clear, p, cnt, flags, b, grid);
-    else if (b < grid + big_grid) bf_big_part(g, h, bound, prev, cur, p, cnt, flags, b - grid, big_grid);
-    else bf_huge_part(g, h, bound, prev, cur, p, cnt, flags, b - grid - big_grid, huge_grid);
+    if (b < grid) bf_pass_part<G>(g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, b, grid);
+    else if (b < grid + big_grid) bf_big_part(g, h, bound, prev, cur, p, cnt, flags, bin_min, b - grid, big_grid);
+    else bf_huge_part(g, h, bound, prev, cur, p, cnt, flags, bin_min, b - grid - big_grid, huge_grid);
+}
+
+// ---------------------------------------------------------------------------------------
+// the closure check and the passes of binned games (egs_bins.h)
+// ---------------------------------------------------------------------------------------
+//
+// The closure check's fold is the rounds' fold: with d = f(u) - w over the edges into D, the
+// first pass's candidate (n+1) w + 1 + (n+1) (MG - f(u)) is (n+1) (MG - d) + 1, so owner 0's
+// maximum and owner 1's minimum of it are the round's minimum and maximum of d.  A successor
+// outside D (and not at TOP) gives INT_MIN: it poisons owner 0's minimum (closure breaks) and is
+// no candidate of owner 1's maximum; one at TOP gives a d past mg + wmax, which ends the path.
+// A pass is the same with 8-byte candidates w' + h, a successor outside D counting as +inf and
+// one at TOP as -inf, for every member: it reads and writes 22 bytes an edge whatever changed,
+// so it runs while many vertices change (bin_min), and k_bf_pass, which evaluates only
+// vertices with a changed successor, after that.
+
+constexpr long long kBinInf = 1ll << 62;       // far past every potential of a binned game
+
+__global__ __launch_bounds__(1024) void k_bin_gather_d(DevGame g, int B, int last) {
+    extern __shared__ __align__(16) int vals[];
+    int slice, part;
+    bin_place(g, blockIdx.x, slice, part);
+    BinWalk walk;
+    walk.start(g, slice, part, g.bin_parts);
+    bin_load(g, slice, (const int *)g.val, vals,
+             [&](int x, int v) { return x == EGS_TOP || in_d_x(g, v, x, B, last) ? x : -1; });
+    __syncthreads();
+    auto diff = [&](uint32_t e) {
+        const int x = vals[e & (kBinSlice - 1)];
+        return x < 0 ? INT_MIN : __builtin_elementwise_sub_sat(x, (int)e >> 15);
+    };
+    walk.run([&](int k, uint32_t e0, uint32_t e1) { *(int2 *)(g.cand + k) = make_int2(diff(e0), diff(e1)); });
+}
+
+// What k_closure does after its edge loop, for a chunk; bits and clear are zero on entry.
+__global__ __launch_bounds__(256) void k_bin_closure(DevGame g, int wmax, int B, int last, long long bound,
+                                                     long long *__restrict__ h, unsigned *__restrict__ bits,
+                                                     int *__restrict__ cnt, int *__restrict__ flags) {
+    extern __shared__ __align__(16) int dkey[];
+    const int4 desc = g.bdesc[blockIdx.x];
+    const int v0 = desc.x, nv = desc.y & kBinNv, n0l = g.n0 - v0;
+    for (int i = threadIdx.x; i <= nv; i += 256) dkey[i] = INT_MAX;
+    __syncthreads();
+    bin_fold<int, int4>(g, g.cand, desc.z, desc.w, n0l, nv, dkey);
+    __syncthreads();
+    const long long scale = (long long)g.n + 1;
+    int members = 0, changed = 0, removed = 0;
+    for (int i = threadIdx.x; i < nv; i += 256) {
+        const int v = v0 + i, x = g.val[v];
+        int f = dkey[i];
+        const bool split = (i == 0 && (desc.y & kBinSplitFirst)) || (i == nv - 1 && (desc.y & kBinSplitLast));
+        if (split && !bin_share_fold(g, v, f)) continue;
+        long long hv;
+        if (x == EGS_TOP) {
+            hv = kHTop;
+        } else if (!in_d_x(g, v, x, B, last)) {
+            hv = kHOut;
+        } else {
+            members++;
+            hv = scale * ((long long)g.mg - x);
+            const int d = f ^ (i >= n0l ? -1 : 0);
+            bool up = false;
+            if (d == INT_MIN) {
+                hv = kHOut;
+                up = true;
+                removed++;
+            } else if (d <= g.mg + wmax) {
+                const long long best = scale * ((long long)g.mg - d) + 1;
+                if (best > hv) {
+                    hv = best;
+                    up = true;
+                    if (best > bound) atomicOr(&flags[1], 1);
+                }
+            }
+            if (up) {
+                bm_set(bits, g.n, v);
+                changed++;
+            }
+        }
+        h[v] = hv;
+    }
+    block_add(members, &flags[3]);
+    block_add(removed, &flags[0]);
+    block_add(changed, &cnt[0]);
+}
+
+__global__ __launch_bounds__(1024) void k_bin_gather_h(DevGame g, const long long *__restrict__ h, int parts, int p,
+                                                       const int *__restrict__ cnt, const int *__restrict__ flags,
+                                                       int bin_min) {
+    extern __shared__ __align__(16) long long hs[];
+    if (cnt[(p - 1) % kCntSlots] < bin_min || flags[1]) return;
+    int slice, part;
+    bin_place(g, blockIdx.x, slice, part);
+    BinWalk walk;
+    walk.start(g, slice, part, parts);
+    bin_load(g, slice, h, hs, [](long long x, int) { return x == kHOut ? kBinInf : x == kHTop ? -kBinInf : x; });
+    __syncthreads();
+    const int iscale = g.n + 1;
+    long long *cand = (long long *)g.cand;
+    walk.run([&](int k, uint32_t e0, uint32_t e1) {
+        longlong2 c;
+        c.x = (long long)iscale * ((int)e0 >> 15) + hs[e0 & (kBinSlice - 1)];
+        c.y = (long long)iscale * ((int)e1 >> 15) + hs[e1 & (kBinSlice - 1)];
+        *(longlong2 *)(cand + k) = c;            // w' is one more: added after the fold
+    });
+}
+
+__global__ __launch_bounds__(256) void k_bin_pass(DevGame g, long long bound, long long *__restrict__ h,
+                                                  unsigned *__restrict__ cur, unsigned *__restrict__ clear, int p,
+                                                  int *__restrict__ cnt, int *__restrict__ flags, int bin_min) {
+    extern __shared__ __align__(16) long long hkey[];
+    const int4 desc = g.bdesc[blockIdx.x];
+    if (cnt[(p - 1) % kCntSlots] < bin_min || flags[1]) return;
+    const int64_t words = bm_total(g.n);
+    for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (int64_t)gridDim.x * blockDim.x)
+        clear[i] = 0u;
+    if (blockIdx.x == 0 && threadIdx.x == 0) cnt[(p + 1) % kCntSlots] = 0;
+    const int v0 = desc.x, nv = desc.y & kBinNv, n0l = g.n0 - v0;
+    for (int i = threadIdx.x; i <= nv; i += 256) hkey[i] = LLONG_MAX;
+    __syncthreads();
+    bin_fold<long long, longlong2, false>(g, (const long long *)g.cand, desc.z, desc.w, n0l, nv, hkey);
+    __syncthreads();
+    int changed = 0, removed = 0;
+    for (int i = threadIdx.x; i < nv; i += 256) {
+        const int v = v0 + i;
+        const long long hv = h[v];
+        if (hv < 0) continue;                    // every chunk of v sees the same until its last applies
+        const bool owner1 = i >= n0l;
+        long long best = hkey[i] ^ (owner1 ? 0ll : -1ll);
+        const bool split = (i == 0 && (desc.y & kBinSplitFirst)) || (i == nv - 1 && (desc.y & kBinSplitLast));
+        if (split && !bin_share_best(g, v, owner1, best)) continue;
+        best += 1;
+        if (best > kBinInf / 2) {                // breaks closure (see k_closure)
+            h[v] = kHOut;
+            removed++;
+        } else if (best > hv) {
+            h[v] = best;
+            if (best > bound) atomicOr(&flags[1], 1);
+        } else {
+            continue;
+        }
+        bm_set(cur, g.n, v);
+        changed++;
+    }
+    block_add(removed, &flags[0]);
+    block_add(changed, &cnt[p % kCntSlots]);
 }
 
 // Starting state of the vertices above huge_deg, in one pass: the shared lifts' partial keys
@@ -872,25 +1033,26 @@ __global__ __launch_bounds__(256) void k_mark_top(DevGame g, const long long *__
 
 static void launch_bf_all(int G, int grid, int big_grid, int huge_grid, hipStream_t st, const DevGame &g,
                           long long *h, long long bound, const unsigned *prev, unsigned *cur, unsigned *clear, int p,
-                          int *cnt, int *flags) {
+                          int *cnt, int *flags, int bin_min) {
     const dim3 all(grid + big_grid + huge_grid), t(256);
     switch (G) {
-    case 1: hipLaunchKernelGGL(k_bf_all<1>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, grid, big_grid, huge_grid); break;
-    case 2: hipLaunchKernelGGL(k_bf_all<2>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, grid, big_grid, huge_grid); break;
-    case 4: hipLaunchKernelGGL(k_bf_all<4>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, grid, big_grid, huge_grid); break;
-    case 8: hipLaunchKernelGGL(k_bf_all<8>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, grid, big_grid, huge_grid); break;
-    default: hipLaunchKernelGGL(k_bf_all<16>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, grid, big_grid, huge_grid); break;
+    case 1: hipLaunchKernelGGL(k_bf_all<1>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, grid, big_grid, huge_grid); break;
+    case 2: hipLaunchKernelGGL(k_bf_all<2>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, grid, big_grid, huge_grid); break;
+    case 4: hipLaunchKernelGGL(k_bf_all<4>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, grid, big_grid, huge_grid); break;
+    case 8: hipLaunchKernelGGL(k_bf_all<8>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, grid, big_grid, huge_grid); break;
+    default: hipLaunchKernelGGL(k_bf_all<16>, all, t, 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min, grid, big_grid, huge_grid); break;
     }
 }
 
 static void launch_bf_pass(int G, int grid, hipStream_t st, const DevGame &g, long long *h, long long bound,
-                           const unsigned *prev, unsigned *cur, unsigned *clear, int p, int *cnt, int *flags) {
+                           const unsigned *prev, unsigned *cur, unsigned *clear, int p, int *cnt, int *flags,
+                           int bin_min) {
     switch (G) {
-    case 1: hipLaunchKernelGGL(k_bf_pass<1>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags); break;
-    case 2: hipLaunchKernelGGL(k_bf_pass<2>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags); break;
-    case 4: hipLaunchKernelGGL(k_bf_pass<4>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags); break;
-    case 8: hipLaunchKernelGGL(k_bf_pass<8>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags); break;
-    default: hipLaunchKernelGGL(k_bf_pass<16>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags); break;
+    case 1: hipLaunchKernelGGL(k_bf_pass<1>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min); break;
+    case 2: hipLaunchKernelGGL(k_bf_pass<2>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min); break;
+    case 4: hipLaunchKernelGGL(k_bf_pass<4>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min); break;
+    case 8: hipLaunchKernelGGL(k_bf_pass<8>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min); break;
+    default: hipLaunchKernelGGL(k_bf_pass<16>, dim3(grid), dim3(256), 0, st, g, h, bound, prev, cur, clear, p, cnt, flags, bin_min); break;
     }
 }
 
@@ -978,20 +1140,35 @@ int certify_top(const DevGame &g, const CertBuffers &cb, int wmax, int last, int
     // chunk (closure and first pass, then more) is sized for a few passes, or for what an
     // earlier attempt of the run needed plus two, so that an attempt usually ends after one
     // read-back; later chunks are longer.
-    const int first_chunk = std::max(6, std::min(pass_hint + 2, 32)), chunk = 8;
+    // A binned pass is three launches, and 14 us when there is nothing left for it: those
+    // games queue fewer ahead.
+    const int first_chunk = std::max(6, std::min(pass_hint + 2, g.bins ? 10 : 32)), chunk = g.bins ? 6 : 8;
     // lanes per vertex: about two edges each (on the 2^22-vertex game, with two edges in
     // flight per lane, the solve took 4.41 ms with 4 lanes, 4.43 with 2 and 4.68 with 8)
     int G = 1;
     while (G < 16 && 2 * G < (double)g.m / g.n) G <<= 1;
     const int bf_grid = grid_for((int64_t)g.n * G, 256, 4096);
+    // binned passes where a slice of potentials fits a compute unit, for passes after one that
+    // changed at least bin_min vertices
+    const bool bin_h = g.bins && g.bin_w <= kBinSlice / 2 && (double)bound < (double)(kBinInf / 8);
+    const int bin_min = bin_h ? std::max(1, g.n / (g.hubs ? kBinPassPartHubs : kBinPassPart)) : 0, h_parts = std::max(1, g.bin_parts / 2);
     for (int c = 0; c < ncand; c++) {
         if (stop && *stop) return 0;        // the run is being stopped: no new candidate
         const int B = (int)cands[c];
         res.threshold = B;
         res.tried++;
-        hipLaunchKernelGGL(k_cert_clear, dim3(grid_for(std::max<int64_t>(bm_len - words, kCntSlots), 256, 64)),
-                           dim3(256), 0, st, flags, cb.bfcnt, bm[0] + words, bm_len - words);
-        if (g.phases > 1) {
+        if (g.bins)                         // the binned check sets single bits: both its bitmaps start at zero
+            hipLaunchKernelGGL(k_cert_clear, dim3(grid_for(2 * bm_len, 256, 256)), dim3(256), 0, st, flags, cb.bfcnt,
+                               bm[0], 2 * bm_len);
+        else
+            hipLaunchKernelGGL(k_cert_clear, dim3(grid_for(std::max<int64_t>(bm_len - words, kCntSlots), 256, 64)),
+                               dim3(256), 0, st, flags, cb.bfcnt, bm[0] + words, bm_len - words);
+        if (g.bins) {
+            hipLaunchKernelGGL(k_bin_gather_d, dim3(g.bins * g.bin_parts), dim3(1024), (size_t)g.bin_w * sizeof(int),
+                               st, g, B, last);
+            hipLaunchKernelGGL(k_bin_closure, dim3(g.nchunks), dim3(256), bin_key_slots(g) * sizeof(int), st, g, wmax, B,
+                               last, bound, cb.h, bm[0], cb.bfcnt, flags);
+        } else if (g.phases > 1) {
             const size_t lds = (size_t)g.phase_tiles * kSliceTile * (sizeof(long long) + sizeof(int));
             if (g.sshift)
                 hipLaunchKernelGGL(k_closure_fused<true>, dim3(g.phase_grid), dim3(256), lds, st, g, B, last, bound,
@@ -1003,7 +1180,7 @@ int certify_top(const DevGame &g, const CertBuffers &cb, int wmax, int last, int
             hipLaunchKernelGGL(k_closure, dim3(grid), dim3(256), 0, st, g, B, last, bound, cb.h, bm[0], bm[1], cb.bfcnt,
                                flags);
         }
-        if (has_big)
+        if (has_big && !g.bins)
             hipLaunchKernelGGL(k_closure_big, dim3(3 * kBigGrid), dim3(256), 0, st, g, B, last, bound, cb.h, bm[0],
                                cb.bfcnt, flags, kBigGrid, 2 * kBigGrid);
         int queued = 1;                     // passes queued so far: pass 0 is the closure's
@@ -1013,13 +1190,20 @@ int certify_top(const DevGame &g, const CertBuffers &cb, int wmax, int last, int
             if (stop && *stop) return 0;    // abandon the candidate: nothing was marked
             const int upto = std::min(cap, queued == 1 ? first_chunk : queued + chunk);
             for (int p = queued; p < upto; p++) {
+                if (bin_min) {
+                    hipLaunchKernelGGL(k_bin_gather_h, dim3(g.bins * h_parts), dim3(1024),
+                                       (size_t)g.bin_w * sizeof(long long), st, g, (const long long *)cb.h, h_parts, p,
+                                       (const int *)cb.bfcnt, (const int *)flags, bin_min);
+                    hipLaunchKernelGGL(k_bin_pass, dim3(g.nchunks), dim3(256), bin_key_slots(g) * sizeof(long long), st,
+                                       g, bound, cb.h, bm[p % 3], bm[(p + 1) % 3], p, cb.bfcnt, flags, bin_min);
+                }
                 // with vertices above big_deg, their parts of the pass run in the same launch
                 if (has_big)
                     launch_bf_all(G, bf_grid, kBigGrid, 2 * kBigGrid, st, g, cb.h, bound, bm[(p - 1) % 3], bm[p % 3],
-                                  bm[(p + 1) % 3], p, cb.bfcnt, flags);
+                                  bm[(p + 1) % 3], p, cb.bfcnt, flags, bin_min);
                 else
                     launch_bf_pass(G, bf_grid, st, g, cb.h, bound, bm[(p - 1) % 3], bm[p % 3], bm[(p + 1) % 3], p,
-                                   cb.bfcnt, flags);
+                                   cb.bfcnt, flags, bin_min);
             }
             if (hipMemcpyAsync(fl, flags, sizeof(int) * 4, hipMemcpyDeviceToHost, st) != hipSuccess) return -1;
             if (hipMemcpyAsync(cnt, cb.bfcnt, sizeof(int) * kCntSlots, hipMemcpyDeviceToHost, st) != hipSuccess)
@@ -1117,7 +1301,7 @@ int certify_all_top(const DevGame &g, const CertBuffers &cb, int wmax, int max_p
         const int upto = std::min(max_passes + 1, queued + chunk);
         for (int p = queued; p < upto; p++) {
             launch_bf_pass(G, bf_grid, st, g, cb.h, bound, bm[(p - 1) % 3], bm[p % 3], bm[(p + 1) % 3], p, cb.bfcnt,
-                           flags);
+                           flags, 0);
             if (has_big) {
                 hipLaunchKernelGGL(k_bf_big, dim3(kBigGrid), dim3(256), 0, st, g, cb.h, bound, bm[(p - 1) % 3],
                                    bm[p % 3], p, cb.bfcnt, flags);

@@ -72,12 +72,21 @@ constexpr int kProbeWant = 100;   // offset in a probe slot of ring[13] when it 
 // dense round: build it once this many rounds have wanted it (a proof usually leaves only a
 // round or two, which do not pay for it).
 constexpr int kSparseWantRounds = 6;
+// A binned dense round costs a third to a half of a sweep: more of them before the transpose.
+constexpr int kSparseWantBinned = 16;
 constexpr int kCertFirstCap = 64;     // longest-path passes per candidate at the first attempt
 constexpr int kCertCandidates = 8;    // gap thresholds tried per attempt (plus the last-round rise set)
 constexpr int kCertEvery = 7;         // default rounds before the first proof attempt
+// ... of a binned game, whose rounds all start from the round before's values and cost less: a
+// first attempt after 7 or 8 rounds more often fails (with 9 the solve of 10^6 vertices of
+// degree 2-12 took 979 us against 1323-1345, that of 1.6 10^6 of degree 3 4.9 ms against 6.4;
+// where 8 is enough, 9 costs 1 to 6%)
+constexpr int kCertEveryBinned = 9;
 constexpr int kGraphSizes = 6;        // captured batches of 1, 2, 4, ..., 32 rounds
 constexpr int kWholeDenseN = 1 << 16; // single launches sweep every round densely; above this size a run of
                                      // sparse rounds goes to the round kernels
+constexpr int64_t kMemorySideCache = 256 << 20;
+constexpr int kBinDensePart = 128;    // a binned round wants the transpose below 1/128 of the vertices
 constexpr int kStopBatch = 4;         // rounds queued ahead of the host when a stop flag is polled
 
 double egs_now_ms() {
@@ -97,10 +106,10 @@ int pow2ceil(int x) {
 struct Layout {
     size_t ptr, edges, cptr, cpred, val, stamp, l0, l1, dbig, dhuge, sbig, shuge, lcnt, mode, ring, rounds, misc,
         tile, fill, stats, statsum, sigma, h, hist, bfcnt, bits, hacc, hcnt, hbest, hflag, tcounts, toffs, tscan,
-        titems, slen, sbase, sedges, bigmask, whole, total;
-    int64_t tcounts_cap;
+        titems, slen, sbase, sedges, bigmask, bedges, bcand, boff, bchunk, bdesc, whole, total;
+    int64_t tcounts_cap, bin_cap, boff_cap;
     int sub_cap;
-    bool phased;
+    bool phased, binned;
 };
 
 constexpr size_t align256c(size_t x) { return (x + 255) & ~(size_t)255; }
@@ -163,6 +172,17 @@ constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
     L.slen = L.phased ? take(ptiles * egs::kMaxPhases * egs::kSliceTile) : 0;
     L.sbase = L.phased ? take(4 * ptiles * egs::kMaxPhases * egs::kSliceWaves) : 0;
     L.sedges = L.phased ? take(8 * m) : 0;
+    // binned dense rounds: words, vertex numbers and candidates of the padded edges
+    L.binned = n_cap >= egs::kBinMinN;
+    L.bin_cap = L.binned ? m_cap + m_cap / 2 + (1 << 20) : 0;
+    if (L.bin_cap > 0x7fffffff) L.bin_cap = 0x7fffffff;
+    L.bedges = L.binned ? take(6 * (size_t)L.bin_cap + 256) : 0;
+    L.bcand = L.binned ? take(8 * (size_t)L.bin_cap) : 0;
+    const size_t chunks = ((size_t)egs::kBinHead * n1 + m) / egs::kBinShareMin + 2;
+    L.boff_cap = L.binned ? (int64_t)((size_t)L.bin_cap / egs::kBinPad + chunks) : 0;
+    L.boff = L.binned ? take(4 * (size_t)L.boff_cap) : 0;
+    L.bchunk = L.binned ? take(8 * (chunks + 1)) : 0;
+    L.bdesc = L.binned ? take(16 * chunks) : 0;
     L.bigmask = L.phased ? take(8 * ((size_t)n_cap / 64 + 2)) : 0;
     L.whole = take(sizeof(egs::WholeCtl));
     L.total = off;
@@ -197,6 +217,11 @@ struct egs_solver {
     int *d_sbase = nullptr;
     int2 *d_sedges = nullptr;
     unsigned long long *d_bigmask = nullptr;
+    uint32_t *d_bedges = nullptr;               // binned dense rounds (large n_cap)
+    int *d_bcand = nullptr, *d_boff = nullptr, *d_bchunk = nullptr;
+    int4 *d_bdesc = nullptr;
+    int64_t bin_cap = 0, boff_cap = 0;          // padded edges and run starts there is room for
+    bool bins_open = false;                     // the binned layout of this prepare is still to be built
     long long *d_h = nullptr;
     egs::WholeCtl *d_whole = nullptr;
     egs::WholePlan whole{};           // nb > 0: iterate() runs the game in single launches (egs_whole.hip)
@@ -281,6 +306,15 @@ static void bind_layout(egs_solver *s, char *b, const Layout &L) {
     s->d_titems = (int2 *)(b + L.titems);
     s->tcounts_cap = L.tcounts_cap;
     s->d_whole = (egs::WholeCtl *)(b + L.whole);
+    if (L.binned) {
+        s->d_bedges = (uint32_t *)(b + L.bedges);
+        s->d_bcand = (int *)(b + L.bcand);
+        s->bin_cap = L.bin_cap;
+        s->boff_cap = L.boff_cap;
+        s->d_boff = (int *)(b + L.boff);
+        s->d_bchunk = (int *)(b + L.bchunk);
+        s->d_bdesc = (int4 *)(b + L.bdesc);
+    }
     if (L.phased) {
         s->d_slen = (uint8_t *)(b + L.slen);
         s->d_sbase = (int *)(b + L.sbase);
@@ -755,6 +789,69 @@ static void bind_game(egs_solver *s, int32_t n, int32_t n0, int64_t m, int32_t m
     s->prepared = false;
     s->whole = egs::WholePlan{};
     s->mirrored = false;
+    s->bins_open = false;
+}
+
+// Binned dense rounds (egs_bins.h) where the packed word holds the weights, the options leave
+// the dense rounds' form open, and they win: a binned round starts from the round before's
+// values only, so it needs a quarter more rounds than sweeps in place, and two launches.  Solves,
+// binned against sweeps (phases above 2^20 vertices): 741 us against 810 at 400,003 vertices of
+// degree 2-16, 1360 against 1677 at 10^6 of degree 3-6, 2.9 ms against 3.7 at 3 10^6 of degree
+// 3-6, 5.5 against 10.8 at 4 10^6 of degree 2-5; skewed degrees 4.8 ms against 5.9 at 450,003
+// and 13.6 against 20.0 at 10^6 of average degree 2.2.  Low even degrees lose (5.2 ms against
+// 4.0 at 2 10^6 of degree 2-5, 6.4 against 4.1 at 1.6 10^6 of degree 3, 9.9 against 8.3 at
+// 4 10^6 of degree 3): their long runs of sparse rounds need the transpose sooner.
+static bool bins_pay(const egs_solver *s) {
+    const egs::DevGame &g = s->g;
+    if (g.n < egs::kBinMinN) return false;
+    if (s->max_outdeg > g.big_deg) return true;
+    return g.n <= egs::kBinHalfN ? g.m >= 4 * (int64_t)g.n : 2 * g.m >= 7 * (int64_t)g.n;
+}
+
+static void pick_bins(egs_solver *s, const egs_options *o) {
+    egs::DevGame &g = s->g;
+    g.bins = 0;
+    g.bin_w = g.bin_parts = g.nchunks = g.bin_share = 0;
+    g.bin_magic = 0;
+    g.bin_once = 0;
+    g.bedges = s->d_bedges;
+    g.bids = (uint16_t *)(s->d_bedges + s->bin_cap);
+    g.cand = s->d_bcand;
+    g.boff = s->d_boff;
+    g.bchunk = s->d_bchunk;
+    g.bdesc = s->d_bdesc;
+    g.hubs = s->max_outdeg > g.huge_deg;
+    if (o->graphs > 0 || o->slices != 0 || !s->d_boff || !bins_pay(s) || g.dense_min > g.n || s->wmax > egs::kBinWmax ||
+        (int64_t)g.mg + 2 * (int64_t)s->wmax >= EGS_TOP || g.n > (int64_t)egs::kBinMax * egs::kBinSlice)
+        return;
+    // slices and parts that fill the device evenly: 512 workgroups with half slices (two to a
+    // compute unit), else 256
+    const bool half = g.n <= egs::kBinHalfN;
+    const int wide = half ? egs::kBinSlice / 2 : egs::kBinSlice, wgs = half ? 512 : 256;
+    const int least = (g.n + wide - 1) / wide;
+    g.bin_parts = std::max(1, wgs / least);
+    const int bins = (std::max(wgs / g.bin_parts, least) + 7) & ~7;
+    g.bin_w = (g.n + bins - 1) / bins;
+    g.bin_magic = (unsigned)((1ull << 32) / (unsigned)g.bin_w + 1);
+    g.bin_share = egs::bin_share(g.n, g.m, bins);
+    const int64_t places = g.m + (int64_t)egs::kBinHead * g.n;
+    g.nchunks = (int)((places + g.bin_share - 1) / g.bin_share);
+    const int64_t padded = g.m + (int64_t)g.nchunks * egs::kBinPad * bins + egs::kBinPad;
+    if (bins > egs::kBinMax || padded > s->bin_cap || (int64_t)(bins + 1) * g.nchunks > s->boff_cap)
+        return;
+    g.bins = bins;
+    g.bin_once = 10 * padded > kMemorySideCache * 3 / 4;
+    // sparse rounds need the transpose, after which the run leaves the bins (build_csc): worth
+    // it only for long tails
+    if (o->dense_pct == 0) g.dense_min = std::max<int64_t>(1, g.n / kBinDensePart);
+}
+
+// Whether one-sweep games lift their static hub lists in the same launch as the sweep.
+static void pick_hub_fused(egs_solver *s) {
+    egs::DevGame &g = s->g;
+    const egs::LaunchShape &sh = s->sh;
+    g.hub_fused = g.phases == 1 && !g.bins && (sh.use_wave || sh.use_block) &&
+                  g.round_grid + g.wave_grid + g.block_grid <= egs::kStatSlots;     // a statistics slot per workgroup
 }
 
 static int pick_shape(egs_solver *s, const egs_options *o) {
@@ -800,7 +897,9 @@ static int pick_shape(egs_solver *s, const egs_options *o) {
         return fail(EGS_E_ARG, "slices must be 0 (auto) or 1..%d (got %d)", egs::kMaxPhases, o->slices);
     g.phases = 1;
     g.slice_shift = 31;
-    if (want > 1 && s->d_slen) {
+    pick_bins(s, o);
+    if (g.bins && o->certify_every == 0) s->cert_every = kCertEveryBinned;
+    if (want > 1 && s->d_slen && !g.bins) {
         int shift = 0;
         while (((int64_t)(want) << shift) < g.n) shift++;          // want slices of 2^shift cover n
         g.slice_shift = shift;
@@ -830,12 +929,10 @@ static int pick_shape(egs_solver *s, const egs_options *o) {
         g.phase_tiles = 96 * 1024 / (egs::kSliceTile * 12);
         g.phase_grid = (int)((tiles + g.phase_tiles - 1) / g.phase_tiles);
     }
-    // one-sweep games lift their static hub lists in the same launch as the low-degree sweep
     g.round_grid = sh.grid;
     g.wave_grid = sh.use_wave ? sh.wave_grid : 0;
     g.block_grid = sh.use_block ? sh.block_grid : 0;
-    g.hub_fused = g.phases == 1 && (sh.use_wave || sh.use_block) &&
-                  g.round_grid + g.wave_grid + g.block_grid <= egs::kStatSlots;     // a statistics slot per workgroup
+    pick_hub_fused(s);
     return EGS_OK;
 }
 
@@ -848,11 +945,17 @@ static hipError_t build_csc(egs_solver *s) {
     if (e == hipSuccess)
         e = hipMemcpyAsync(s->d_ring + 12, s->h_probe + kPinOne, sizeof(int), hipMemcpyHostToDevice, s->stream);
     if (e == hipSuccess) s->csc_built = true;
+    if (s->g.bins) {
+        // sparse rounds from here on, dense ones as sweeps in place
+        s->g.bins = 0;
+        pick_hub_fused(s);
+    }
     return e;
 }
 
 // Set-up of the round kernels: counters, static hub lists, slice layout, initial frontier.
-static int prepare_rounds(egs_solver *s) {
+// A binned game's first round is done with its layout (`first`).
+static int prepare_rounds(egs_solver *s, bool first = false) {
     // graphs hold the launch arguments they were captured with: kept while those stay the same
     if (memcmp(&s->graph_g, &s->g, sizeof(s->g)) != 0 || memcmp(&s->graph_sh, &s->sh, sizeof(s->sh)) != 0) {
         drop_graphs(s);
@@ -875,10 +978,15 @@ static int prepare_rounds(egs_solver *s) {
     if (s->sh.use_block)             // shared lifts of the vertices above huge_deg start empty
         HIP_TRY(egs::launch_hbest_reset(s->g, s->stream));
     HIP_TRY(egs::launch_classify(s->g, s->d_ring + 9, s->stream));
-    // with slices and no transpose the slice set-up also stores the initial state
-    const bool init_in_slices = s->g.phases > 1 && !s->csc_built;
-    HIP_TRY(egs::launch_slices(s->g, s->stream, init_in_slices));
-    HIP_TRY(egs::launch_init(s->g, s->stream, init_in_slices));
+    if (s->g.bins) {
+        s->bins_open = false;
+        HIP_TRY(egs::launch_bin_build(s->g, first, s->stream));
+    } else {
+        // with slices and no transpose the slice set-up also stores the initial state
+        const bool init_in_slices = s->g.phases > 1 && !s->csc_built;
+        HIP_TRY(egs::launch_slices(s->g, s->stream, init_in_slices));
+        HIP_TRY(egs::launch_init(s->g, s->stream, init_in_slices));
+    }
     // the initial frontier's counters ride on the same wait as the timing
     HIP_TRY(hipMemcpyAsync(s->h_probe + kPinInit, s->d_lcnt + 1 * egs::kListCounters,
                            sizeof(int) * egs::kListCounters, hipMemcpyDeviceToHost, s->stream));
@@ -908,6 +1016,7 @@ static bool takes_whole(const egs_options *o) {
 // sweep (none when the run has converged).
 static int leave_whole(egs_solver *s) {
     s->mirrored = false;
+    if (s->bins_open) return prepare_rounds(s);
     if (s->whole.nb == 0) return EGS_OK;
     s->whole.nb = 0;
     if (s->whole_rounds == 0 && !s->st.converged) return prepare_rounds(s);
@@ -1044,10 +1153,16 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     s->whole_rounds = 0;
     s->whole_st = egs_stats{};
     s->mirrored = false;
+    s->bins_open = false;
     s->whole = takes_whole(opt) ? egs::whole_plan(s->g.n, s->g.m, s->g.mg, s->wmax, s->max_outdeg, s->whole_max_nb) : egs::WholePlan{};
     if (s->whole.nb > 0) {
         HIP_TRY(egs::launch_whole_prep(s->whole, s->g, s->d_whole, true, s->stream));
         memset(&s->st, 0, sizeof(s->st));
+    } else if (s->g.bins) {
+        // the values and chunks now; the layout with the first round, in iterate()
+        HIP_TRY(egs::launch_bin_prep(s->g, s->stream));
+        memset(&s->st, 0, sizeof(s->st));
+        s->bins_open = true;
     } else {
         rc = prepare_rounds(s);
         if (rc) return rc;
@@ -1100,9 +1215,18 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
         if (rc) return rc;
         if (status == egs::kWholeSparse) HIP_TRY(build_csc(s));
     }
+    int64_t launched = 0;
+    if (s->bins_open) {
+        const bool first = limit > 0;
+        const int rc = prepare_rounds(s, first);
+        if (rc) return rc;
+        if (first) {
+            s->next_round = 2;
+            launched = 1;
+        }
+    }
     double t0 = 0;
     HIP_TRY(mark_start(s, &t0));
-    int64_t launched = 0;
     int pending = -1;     // probe slot in flight
     bool done = false;
     int batch = 4;        // grow towards batch_rounds so short solves do not overshoot much
@@ -1204,7 +1328,7 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
             HIP_TRY(probe_wait(s, pending));
             if (list_total(s, s->h_probe + kPinProbe + pending * kProbeStride) == 0) done = true;
             // enough rounds wanted to go sparse: build the transpose now
-            if (!done && !s->csc_built && s->h_probe[kPinProbe + pending * kProbeStride + s->probe_want[pending]] >= kSparseWantRounds)
+            if (!done && !s->csc_built && s->h_probe[kPinProbe + pending * kProbeStride + s->probe_want[pending]] >= (s->g.bins ? kSparseWantBinned : kSparseWantRounds))
                 HIP_TRY(build_csc(s));
         }
         pending = slot;

@@ -70,6 +70,19 @@ struct DevGame {
     const void *sedges;   // uint32 (w << sshift) | succ when sshift > 0, else int2 {succ, w}
     int sshift;
     const unsigned long long *bigmask;   // bit v: vertex v is above big_deg (lifted by the wave/block kernels)
+    // Dense rounds over binned edges (egs_bins.h; bins > 0): slices of the successors, successors
+    // per slice with floor(2^32 / bin_w) + 1, parts of the chunks per slice, chunks.
+    int bins, bin_w, bin_parts, nchunks;
+    unsigned bin_magic;
+    uint32_t *bedges;     // (w << 15) | place in slice, per chunk grouped by slice
+    uint16_t *bids;       // the edge's vertex in the chunk
+    int *cand;            // a - w of each edge (8 bytes of room: the proof passes keep w' + h)
+    int *boff;            // [bins + 1][nchunks]: where a chunk's run of a slice starts
+    int *bchunk;          // nchunks + 1 pairs: a chunk's first edge and that edge's vertex
+    int4 *bdesc;          // nchunks: first vertex, vertices and split flags, first and last padded edge
+    int bin_share;        // places of the chunks' line per chunk
+    int bin_once;         // 1: words, vertex numbers and candidates outgrow the memory-side cache
+    int hubs;             // some vertex is above huge_deg
     int round_grid;       // workgroups of k_round's low-degree part
     int hub_fused;        // 1: k_round's grid continues with the hub part in dense rounds
     int wave_grid, block_grid;   // workgroups of the wave and workgroup-per-vertex hub bodies
@@ -89,6 +102,18 @@ constexpr int kPhaseMinN = 1 << 20;        // up to this many vertices the value
 constexpr int kSliceTile = 256;            // vertices per tile of the slice layout
 constexpr int kSliceWaves = kSliceTile / 64;
 constexpr int kMaxSliceDeg = 255;          // a vertex's edges into one slice fit a byte
+
+// Binned games: successors of a slice at most (128 KB of values; half of that up to kBinHalfN
+// vertices), slices at most, the largest |w| of a packed edge.
+constexpr int kBinSlice = 1 << 15;
+constexpr int kBinHalfN = 1 << 21;
+constexpr int kBinMax = 512;
+constexpr int kBinWmax = 65535;
+constexpr int kBinHead = 4;                // places of a vertex on the chunks' line, before its edges
+constexpr int kBinShareMin = 4096, kBinShareMax = 16384;   // places of a chunk
+constexpr int kBinSplitFirst = 1 << 29, kBinSplitLast = 1 << 30, kBinNv = (1 << 29) - 1;   // bdesc's second word
+constexpr int kBinPad = 16;                // runs are padded to this many edges
+constexpr int kBinMinN = 400000;             // the rule on degrees and both sides' times: bins_pay
 
 // Edge k of the slice layout: successor and weight.
 template <bool PACK>
@@ -242,6 +267,12 @@ hipError_t launch_classify(const DevGame &g, int *counts, hipStream_t st);
 // big_deg and counted, without listing, the active ones (no transpose: round 1 sweeps densely)
 hipError_t launch_init(const DevGame &g, hipStream_t st, bool in_slices);
 hipError_t launch_slices(const DevGame &g, hipStream_t st, bool init);
+// Binned games: values to 0 and the chunk bounds; then the layout, with round 1 done on the
+// way (`first`: what follows is round 2) or not.
+int bin_share(int n, int64_t m, int bins);
+inline size_t bin_key_slots(const DevGame &g) { return (size_t)(g.bin_share / (kBinHead + 1) + 4); }   // vertex words of a chunk, with the padding's
+hipError_t launch_bin_prep(const DevGame &g, hipStream_t st);
+hipError_t launch_bin_build(const DevGame &g, bool first, hipStream_t st);
 int pack_shift(int n, int wmax);
 // Round j of a batch (absolute round ring[14] + j); launch_advance ends the batch.
 hipError_t launch_round(const DevGame &g, const LaunchShape &sh, int j, hipStream_t st);

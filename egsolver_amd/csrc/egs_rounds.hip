@@ -21,6 +21,10 @@
 // vertex (k_lift_wave) and, above huge_deg, a workgroup per vertex (k_lift_block), in the
 // same round.  Appends are staged in LDS per workgroup and flushed with one atomic per
 // sub-queue counter.
+#include <algorithm>
+#include <climits>
+
+#include "egs_bins.h"
 #include "egs_device.h"
 #include "egs_internal.h"
 
@@ -159,7 +163,7 @@ struct LiftAcc {
 };
 
 __device__ __forceinline__ void flush_stats(const DevGame &g, LiftAcc &a) {
-    __shared__ unsigned long long red[4][4];
+    __shared__ unsigned long long red[4][16];
     const int wid = threadIdx.x >> 6;
     const int lane = threadIdx.x & 63;
     unsigned long long vals[4] = {a.processed, a.edges, a.lifted, a.preds};
@@ -930,6 +934,282 @@ __global__ __launch_bounds__(256) void k_lift_hubs(DevGame g, int j, int wave_gr
 }
 
 // ---------------------------------------------------------------------------------------
+// binned dense rounds (egs_bins.h)
+// ---------------------------------------------------------------------------------------
+
+// Values to 0, and the chunks: chunk c starts with the first edge at or past c * bin_share on
+// the line where edge k of vertex v lies at k + kBinHead (v + 1).  Vertices cut by a chunk's
+// start get their shared words.
+__global__ __launch_bounds__(256) void k_bin_prep(DevGame g) {
+    const int share = g.bin_share;
+    for (int64_t v = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; v < g.n; v += (int64_t)gridDim.x * blockDim.x) {
+        g.val[v] = 0;
+        const int s = g.ptr[v], e = g.ptr[v + 1];
+        const int64_t head = kBinHead * (v + 1);
+        const int64_t lo = v > 0 ? (head - kBinHead + s - 1) / share + 1 : 0, hi = (head + e - 1) / share;
+        for (int64_t c = lo; c <= hi; c++) {
+            const int first = (int)max((int64_t)s, c * share - head);
+            g.bchunk[2 * c] = first;
+            g.bchunk[2 * c + 1] = (int)v;
+            if (first > s) {
+                g.hacc[v] = INT_MAX;
+                g.hcnt[v] = 0;
+                g.hbest[v] = v >= g.n0 ? LLONG_MAX : LLONG_MIN;
+            }
+        }
+        if (v == g.n - 1)
+            for (int64_t c = hi + 1; c <= g.nchunks; c++) {
+                g.bchunk[2 * c] = (int)g.m;
+                g.bchunk[2 * c + 1] = g.n;
+            }
+    }
+}
+
+// The layout of a chunk, and (FIRST) round 1 on the way: with every value 0 its candidates
+// are the edges' -w, so no gather is needed.  The chunk's edges are read once, consecutive
+// threads on consecutive edges; a mark at each vertex's first edge and a running maximum give
+// every edge its vertex; an LDS counter per slice gives it a place in its run; the words (in
+// two halves), then the vertex numbers, leave through the marks' space in order.  Bound by HBM:
+// 8 bytes an edge in, 6 out; 65 KB of LDS at most let two workgroups share a compute unit
+// (with one, waiting on its own phases, the 2^22-vertex game's layout took 427 us; now 185,
+// round 1 included, and 65 at 10^6 vertices of degree 8).
+template <bool FIRST>
+__global__ __launch_bounds__(1024, 8) void k_bin_build(DevGame g, int nvmax) {
+    constexpr int KE = kBinShareMax / 1024;      // edges a thread
+    extern __shared__ __align__(16) int lds[];
+    int *key = lds;                              // nvmax + 1 vertex words
+    uint16_t *mark = (uint16_t *)(lds + nvmax + 1);
+    __shared__ int cnt[kBinMax], wsum[16];
+    const int t = threadIdx.x, lane = t & 63, wid = t >> 6;
+    const int c = blockIdx.x, nc = g.nchunks;
+    const BinChunk ch = bin_chunk(g, c);
+    const int v0 = ch.v0, nv = ch.nv, e0 = ch.e0, E = ch.e1 - ch.e0, n0l = g.n0 - v0;
+    const int base = (e0 & ~(kBinPad - 1)) + c * kBinPad * g.bins;
+    for (int s = t; s < kBinMax; s += 1024) cnt[s] = 0;
+    for (int p = t; p < E; p += 1024) mark[p] = 0;
+    if (FIRST)
+        for (int i = t; i < nv; i += 1024) key[i] = INT_MAX;
+    __syncthreads();
+    for (int i = t; i < nv; i += 1024) mark[max(g.ptr[v0 + i] - e0, 0)] = (uint16_t)(i + 1);
+    __syncthreads();
+    const int per = (E + 1023) / 1024;
+    {   // marks -> vertex numbers
+        const int p0 = t * per, p1 = min(E, p0 + per);
+        int last = 0;
+        for (int p = p0; p < p1; p++) last = max(last, (int)mark[p]);
+        int inc = last;
+        for (int d = 1; d < 64; d <<= 1) {
+            const int o = __shfl_up(inc, d, 64);
+            if (lane >= d) inc = max(inc, o);
+        }
+        if (lane == 63) wsum[wid] = inc;
+        __syncthreads();
+        int cur = __shfl_up(inc, 1, 64);
+        if (lane == 0) cur = 0;
+        for (int w = 0; w < wid; w++) cur = max(cur, wsum[w]);
+        for (int p = p0; p < p1; p++) {
+            cur = max(cur, (int)mark[p]);
+            mark[p] = (uint16_t)(cur - 1);
+        }
+    }
+    __syncthreads();
+    // slot j of a thread is edge j * 1024 + t of the chunk; `word` its packed edge, `place` its
+    // vertex and, in turn, (slice, place in run) and the place in the chunk
+    int word[KE], place[KE], id[KE];
+#pragma unroll
+    for (int j = 0; j < KE; j++) {
+        word[j] = place[j] = id[j] = 0;
+        const int p = j * 1024 + t;
+        if (p < E) {
+            id[j] = mark[p];
+            const int2 x = edge_nt(g.edges, (int64_t)e0 + p);
+            place[j] = x.x;
+            word[j] = x.y;
+        }
+    }
+#pragma unroll
+    for (int j = 0; j < KE; j++) {
+        const int p = j * 1024 + t;
+        if (p < E) {
+            const int u = place[j], w = word[j];
+            int s = (int)__umulhi((unsigned)u, g.bin_magic), r = u - s * g.bin_w;
+            if (r < 0) {                         // the magic number is rounded up
+                s--;
+                r += g.bin_w;
+            }
+            place[j] = (s << 16) | atomicAdd(&cnt[s], 1);
+            word[j] = (int)(((uint32_t)w << 15) | (uint32_t)r);
+            if (FIRST) atomicMin(&key[id[j]], __builtin_elementwise_sub_sat(0, w) ^ (id[j] >= n0l ? -1 : 0));
+        }
+    }
+    __syncthreads();
+    int padded;                                  // the chunk's edges with their padding
+    {
+        const int mine = t < g.bins ? (cnt[t] + kBinPad - 1) & ~(kBinPad - 1) : 0;
+        const int ex = egs_block_exclusive_scan(mine, wsum, padded);
+        if (t < g.bins) {
+            cnt[t] = ex;
+            g.boff[(size_t)t * nc + c] = base + ex;
+        }
+        if (t == 0) {
+            g.boff[(size_t)g.bins * nc + c] = base + padded;
+            g.bdesc[c] = make_int4(v0, nv | (ch.split_first ? kBinSplitFirst : 0) | (ch.split_last ? kBinSplitLast : 0),
+                                   base, base + padded);
+        }
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < KE; j++) place[j] = j * 1024 + t < E ? cnt[place[j] >> 16] + (place[j] & 0xffff) : INT_MAX;
+    // the marks' space holds bin_share / 2 words, or bin_share vertex numbers
+    uint32_t *stage = (uint32_t *)mark;
+    const int room = g.bin_share / 2;
+    for (int lo = 0; lo < padded; lo += room) {
+        const int len = min(room, padded - lo);
+        for (int p = t; p < len; p += 1024) stage[p] = 0;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KE; j++)
+            if ((unsigned)(place[j] - lo) < (unsigned)len) stage[place[j] - lo] = (uint32_t)word[j];
+        __syncthreads();
+        for (int p = t; p < len; p += 1024) g.bedges[(size_t)base + lo + p] = stage[p];
+        __syncthreads();
+    }
+    for (int lo = 0; lo < padded; lo += 2 * room) {
+        const int len = min(2 * room, padded - lo);
+        for (int p = t; p < len; p += 1024) mark[p] = (uint16_t)nv;
+        __syncthreads();
+#pragma unroll
+        for (int j = 0; j < KE; j++)
+            if ((unsigned)(place[j] - lo) < (unsigned)len) mark[place[j] - lo] = (uint16_t)id[j];
+        __syncthreads();
+        for (int p = t; p < len / 2; p += 1024)
+            ((uint32_t *)g.bids)[((size_t)base + lo) / 2 + p] = ((const uint32_t *)mark)[p];
+        __syncthreads();
+    }
+    if (!FIRST) return;
+    LiftAcc acc;
+    for (int i = t; i < nv; i += 1024) {
+        const int v = v0 + i;
+        int f = key[i];
+        // a vertex of several chunks is finished by the last of them
+        const bool split = (i == 0 && ch.split_first) || (i == nv - 1 && ch.split_last);
+        if (split && !bin_share_fold(g, v, f)) continue;
+        const int d = f ^ (i >= n0l ? -1 : 0);
+        const int up = d > 0;
+        if (up) {
+            g.val[v] = d > g.mg ? EGS_TOP : d;
+            if (d > g.mg) g.ring[15] = 1;
+        }
+        acc.processed++;
+        acc.edges += g.ptr[v + 1] - g.ptr[v];
+        acc.lifted += up;
+        g.stamp[v] = 0;
+        if (g.rise) g.rise[v] = up;              // round 1, or never
+    }
+    if (c == 0 && t == 0) {
+        g.mode[1] = MODE_DENSE;
+        g.mode[3] = 2;                           // round 2's input: the count only
+    }
+    // the risers are the initially active vertices (round 1's input) and round 2's input
+    int total;
+    egs_block_exclusive_scan((int)acc.lifted, wsum, total);
+    if (t == 0 && total > 0) {
+        int bs, ns, bo;
+        reserve_split(g, g.lcnt + 1 * kListCounters, c % kSub, total, bs, ns, bo);
+        reserve_split(g, g.lcnt + 2 * kListCounters, c % kSub, total, bs, ns, bo);
+    }
+    flush_stats(g, acc);
+}
+
+// Round 1 ends: it counts when any vertex was active.
+__global__ __launch_bounds__(64) void k_bin_close(DevGame g) {
+    const int *c = g.lcnt + 1 * kListCounters;
+    const int any = c[threadIdx.x] | (threadIdx.x == 0 ? c[kSub] : 0);
+    if (__ballot(any != 0) != 0 && threadIdx.x == 0) *g.rounds_done = 1;
+    if (threadIdx.x == 0) g.ring[14] = 2;
+}
+
+// Every edge's a - w, from a slice of the values in LDS.  Bound by its streams, 4 bytes an
+// edge in and 4 out, beside bins * parts slices of values.  Binned games have no transpose, so
+// a round is dense or done: every workgroup sees which from the input list's counters, and the
+// first does k_round's bookkeeping, which saves that launch.  73 us on the 2^22-vertex game of
+// degree 8 (268 MB, 3.7 TB/s), 17 on 10^6 vertices of degree 8 and 16 on the skewed 2^20 game,
+// where the slices' load and the runs' latency weigh as much as the streams.
+__global__ __launch_bounds__(1024) void k_bin_gather(DevGame g, int j) {
+    extern __shared__ __align__(16) int vals[];
+    __shared__ int pre[kSub + 2];
+    // the slice and the first edges load beside the counters
+    int slice, part;
+    bin_place(g, blockIdx.x, slice, part);
+    BinWalk walk;
+    walk.start(g, slice, part, g.bin_parts);
+    bin_load(g, slice, (const int *)g.val, vals, [](int x, int) { return x; });
+    const int r = g.ring[14] + j;
+    load_layout(g, r % 3, pre);
+    __syncthreads();
+    const int want = decide_mode(g, r, pre[kSub + 1]);
+    const bool dense = want != MODE_DONE;
+    if (blockIdx.x == 0) {
+        int *z = g.lcnt + ((r + 2) % 3) * kListCounters;
+        for (int i = threadIdx.x; i < kListCounters; i += blockDim.x) z[i] = 0;
+        if (threadIdx.x == 0) {
+            g.mode[r % 3] = dense ? MODE_DENSE : MODE_DONE;
+            if (dense) *g.rounds_done = r;
+            if (dense && want != MODE_DENSE) g.ring[13]++;   // rounds that wanted the transpose
+        }
+    }
+    if (!dense) return;
+    int *cand = g.cand;
+    walk.run([&](int k, uint32_t e0, uint32_t e1) {
+        *(int2 *)(cand + k) = make_int2(__builtin_elementwise_sub_sat(vals[e0 & (kBinSlice - 1)], (int)e0 >> 15),
+                                        __builtin_elementwise_sub_sat(vals[e1 & (kBinSlice - 1)], (int)e1 >> 15));
+    });
+}
+
+// A chunk's lifts from its candidates.  The risers are counted, not listed: the next round is
+// dense whatever they are.  Bound by its streams, 6 bytes an edge in: 49 us on the 2^22-vertex
+// game (201 MB), so a round takes 122 us against 204 for the phased sweep, and 38 against 74
+// for the sweep in place at 10^6 vertices of degree 8, 34 against 109 on the skewed 2^20 game.
+__global__ __launch_bounds__(256) void k_bin_reduce(DevGame g, int j) {
+    extern __shared__ __align__(16) int key[];
+    __shared__ int wsum[4];
+    const int c = blockIdx.x;
+    const int4 desc = g.bdesc[c];
+    const int r = g.ring[14] + j;
+    if (g.mode[r % 3] != MODE_DENSE) return;
+    const int v0 = desc.x, nv = desc.y & kBinNv, n0l = g.n0 - v0;
+    for (int i = threadIdx.x; i <= nv; i += 256) key[i] = INT_MAX;     // one more for the padding
+    __syncthreads();
+    bin_fold<int, int4>(g, g.cand, desc.z, desc.w, n0l, nv, key);
+    __syncthreads();
+    LiftAcc acc;
+    for (int i = threadIdx.x; i < nv; i += 256) {
+        const int v = v0 + i;
+        const int old = g.val[v];
+        int f = key[i];
+        const bool split = (i == 0 && (desc.y & kBinSplitFirst)) || (i == nv - 1 && (desc.y & kBinSplitLast));
+        if ((split && !bin_share_fold(g, v, f)) || old == EGS_TOP) continue;
+        const int d = f ^ (i >= n0l ? -1 : 0);
+        const int t = d > g.mg ? EGS_TOP : max(d, 0);
+        acc.processed++;
+        acc.edges += g.ptr[v + 1] - g.ptr[v];
+        if (old < t) {
+            g.val[v] = t;
+            if (t == EGS_TOP) g.ring[15] = 1;
+            if (g.rise) g.rise[v] = r;
+            acc.lifted++;
+        }
+    }
+    int total;
+    egs_block_exclusive_scan((int)acc.lifted, wsum, total);
+    if (threadIdx.x == 0) {
+        if (total > 0) atomicAdd(&g.lcnt[((r + 1) % 3) * kListCounters + c % kSub], total);
+        if (c == 0) g.mode[3] = r + 1;           // round r+1's input: the count only
+    }
+    flush_stats(g, acc);
+}
+
+// ---------------------------------------------------------------------------------------
 // host side
 // ---------------------------------------------------------------------------------------
 
@@ -976,6 +1256,13 @@ hipError_t launch_resume(const DevGame &g, int next, bool converged, hipStream_t
 }
 
 hipError_t launch_round(const DevGame &g, const LaunchShape &sh, int j, hipStream_t st) {
+    if (g.bins) {
+        hipLaunchKernelGGL(k_bin_gather, dim3(g.bins * g.bin_parts), dim3(1024), (size_t)g.bin_w * sizeof(int), st, g,
+                           j);
+        hipLaunchKernelGGL(k_bin_reduce, dim3(g.nchunks), dim3(256),
+                           bin_key_slots(g) * sizeof(int), st, g, j);
+        return hipGetLastError();
+    }
     const dim3 grid(g.round_grid + (g.hub_fused ? g.wave_grid + g.block_grid : 0));
 #define EGS_ROUND(GG)                                                                            \
     if (g.hub_fused) hipLaunchKernelGGL((k_round<GG, true>), grid, dim3(256), 0, st, g, j);     \
@@ -1004,6 +1291,30 @@ hipError_t launch_round(const DevGame &g, const LaunchShape &sh, int j, hipStrea
         hipLaunchKernelGGL(k_lift_wave, dim3(sh.wave_grid), dim3(256), 0, st, g, j);
     else if (sh.use_block)
         hipLaunchKernelGGL(k_lift_block, dim3(sh.block_grid), dim3(256), 0, st, g, j);
+    return hipGetLastError();
+}
+
+// Places of a chunk: runs of about 104 edges (128 with their padding are one load of a wave).
+int bin_share(int n, int64_t m, int bins) {
+    const int64_t places = m + (int64_t)kBinHead * n;
+    const int64_t s = (int64_t)(104.0 * bins * (double)places / (double)m);
+    return (int)std::max<int64_t>(kBinShareMin, std::min<int64_t>(kBinShareMax, s)) & ~31;
+}
+
+hipError_t launch_bin_prep(const DevGame &g, hipStream_t st) {
+    hipLaunchKernelGGL(k_bin_prep, dim3(grid_for(g.n, 256, 2048)), dim3(256), 0, st, g);
+    return hipGetLastError();
+}
+
+hipError_t launch_bin_build(const DevGame &g, bool first, hipStream_t st) {
+    const int nvmax = g.bin_share / (kBinHead + 1) + 3;
+    const size_t lds = 4 * ((size_t)nvmax + 1) + 2 * (size_t)g.bin_share;
+    if (!first) {
+        hipLaunchKernelGGL(k_bin_build<false>, dim3(g.nchunks), dim3(1024), lds, st, g, nvmax);
+        return launch_init(g, st, false);
+    }
+    hipLaunchKernelGGL(k_bin_build<true>, dim3(g.nchunks), dim3(1024), lds, st, g, nvmax);
+    hipLaunchKernelGGL(k_bin_close, dim3(1), dim3(64), 0, st, g);
     return hipGetLastError();
 }
 
