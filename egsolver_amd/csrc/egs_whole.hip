@@ -40,8 +40,12 @@ constexpr long long kWInf = 1ll << 62;
 __device__ __forceinline__ bool w_member(long long h) { return h >= 0 && h < kWInf / 2; }
 
 // A vote's 64-bit word: sum of per-thread counts, waves that changed something, waves past
-// the divergence bound, arrivals.
-constexpr int kVoteChanged = 24, kVoteOver = 36, kVoteArrive = 48;
+// the divergence bound, arrivals.  A wave field has room for every wave of the largest launch:
+// with one bit less, a pass in which all 4,096 waves changed something read as one past the
+// bound, and a game whose vertices all climb (312,926 of degree 2) was never proved.
+constexpr int kVoteChanged = 22, kVoteOver = 35, kVoteArrive = 48, kVoteWaves = (1 << 13) - 1;
+static_assert(kWholeMaxNb * (int64_t)kWholeShareMax < 1 << kVoteChanged && kWholeMaxNb * 16 <= kVoteWaves &&
+              kVoteChanged + 13 == kVoteOver && kVoteOver + 13 == kVoteArrive, "the fields of a vote hold their sums");
 
 __device__ __forceinline__ unsigned long long ctl_load(const unsigned long long *p) {
     return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
@@ -411,8 +415,8 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
                 }
                 if (!vote(alive, ch, over, tot)) return false;
                 passes++;
-                converged = ((tot >> kVoteChanged) & 0xfff) == 0;
-                diverged = ((tot >> kVoteOver) & 0xfff) != 0;
+                converged = ((tot >> kVoteChanged) & kVoteWaves) == 0;
+                diverged = ((tot >> kVoteOver) & kVoteWaves) != 0;
             }
             const int64_t left = vcount(tot);
             pruned += left < m0;
@@ -695,8 +699,8 @@ __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
                 }
                 tot = sum_vote(alive, ch, over);
                 passes++;
-                converged = ((tot >> kVoteChanged) & 0xfff) == 0;
-                diverged = ((tot >> kVoteOver) & 0xfff) != 0;
+                converged = ((tot >> kVoteChanged) & kVoteWaves) == 0;
+                diverged = ((tot >> kVoteOver) & kVoteWaves) != 0;
             }
             const int64_t left = vcount(tot);
             pruned += left < m0;

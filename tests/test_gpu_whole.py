@@ -201,3 +201,18 @@ def test_several_solvers_at_once():
     for t in ts:
         t.join()
     assert not bad, bad
+
+
+def test_proof_with_every_wave_changing():
+    """256 workgroups whose every wave raises a potential in the same pass: the vote's count of
+    them must not run into its neighbour field, or the proof is refused each time and the run
+    climbs to MG (millions of rounds) by lifting alone."""
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=312926, seed=18, deg_kind=E.games.DEG_FIXED, deg_lo=2, deg_hi=2, alpha=2.1, wmax=54))
+    _say("degree 2, n 312926")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        s.prepare(E.options(max_phases=20000))
+        conv, st = s.iterate()
+        assert conv and st.certificates > 0, st.as_dict()
+        assert s.violations() == 0
