@@ -187,3 +187,46 @@ def test_config4_full_launch(oracle):
         unseeded, seeded = exact_sample(oracle, games, vals, sorted(idx), s)
     _say(f"config 4 sample: {unseeded} games exact against EG0 from 0, {seeded} through the certificate")
     assert unseeded >= 16 and seeded == len(idx)
+
+
+def test_batch_value_layouts(oracle):
+    """The places a workgroup keeps a game's values in: whole with the proofs' own potentials
+    behind them and without, 16 bits each (values past 16 bits are in global memory), and split;
+    rows longer than a group's slots, a single vertex, proofs early, as usual and off."""
+    import egsolver_amd as E
+    K = E.games
+    spec = [(3000, K.DEG_UNIFORM, 2, 16, 1000), (2999, K.DEG_UNIFORM, 1, 9, 300000), (2998, K.DEG_POWERLAW, 1, 900, 60),
+            (2997, K.DEG_FIXED, 2, 2, 50), (200, K.DEG_COMPLETE, 1, 1, 40), (2, K.DEG_FIXED, 1, 1, 7),
+            (2996, K.DEG_UNIFORM, 30, 70, 100)]
+    games = [E.generate(E.GenParams(n=n, seed=50 + i, deg_kind=k, deg_lo=lo, deg_hi=hi, alpha=1.8, wmax=w))
+             for i, (n, k, lo, hi, w) in enumerate(spec)]
+    refs = [lfp(oracle, to_oracle_game(g)) for g in games]
+    assert any(((r > 65535) & (r < 2147483647)).any() for r in refs)
+    with E.Batch() as b:
+        for g in games:
+            b.add(g)
+        b.upload()
+        for lds in (6002, 3000, 1500, 1498, 65):
+            for every in (0, 1, -1):
+                _say(f"layouts, {lds} ints, proofs every {every}")
+                st = b.solve(E.batch_options(lds_ints=lds, certify_every=every))
+                assert st["converged"] == len(games)
+                for i, ref in enumerate(refs):
+                    assert np.array_equal(b.values(i), ref), (lds, every, i)
+
+
+@pytest.mark.parametrize("room", [1, 0])
+def test_batch_thresholds_near_top(oracle, room):
+    """A threshold so high that a TOP value less a weight just stays past every other value, and
+    one higher: the winners and the finite values are those of the game's own threshold."""
+    import dataclasses
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=700, seed=3, deg_kind=E.games.DEG_UNIFORM, deg_lo=2, deg_hi=9, wmax=20))
+    ref = lfp(oracle, to_oracle_game(g))
+    high = dataclasses.replace(g, mg=2147483647 - room - 2 * int(np.abs(g.w).max()))
+    _say(f"threshold {high.mg}")
+    with E.Batch() as b:
+        b.add(high)
+        b.upload()
+        st = b.solve(E.batch_options(max_sweeps=20000))
+        assert st["converged"] == 1 and np.array_equal(b.values(0), ref)

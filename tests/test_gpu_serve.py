@@ -213,3 +213,18 @@ def test_served_read_order_games(oracle):
         bad_ptr[1] = bad_ptr[0]
         with pytest.raises(RuntimeError):
             srv.submit_read_order(owner, bad_ptr, rsucc, rw)
+
+
+def test_served_partial_sweeps_of_short_values(oracle):
+    """Games whose values are 16 bits each in a slice's LDS, or split, stopped part-way and
+    resumed: the values travel through the arena between slices."""
+    import egsolver_amd as E
+    reqs = _requests(11, 10, 1500, 0.0)
+    arena = sum(E.Server.footprint(r.game) for r in reqs) + (1 << 20)
+    for lds in (760, 300):
+        _say(f"serve partial sweeps in {lds} ints, sizes {[r.game.n for r in reqs]}")
+        done, wall, slices = E.run_served(reqs, arena, E.serve_options(slice_kedges=4, lds_ints=lds), max_games=16,
+                                          keep_values=True)
+        assert slices > 10
+        for r in done:
+            assert np.array_equal(r.values, lfp(oracle, to_oracle_game(r.game))), (lds, r.rid, r.game.n)
