@@ -473,13 +473,10 @@ __global__ __launch_bounds__(256) void k_closure_big(DevGame g, int B, int last,
             bool done = true;
             int f = (any ? 1 : 0) | (all ? 0 : 2);
             if (contrib > 1) {
-                if (f) atomicOr(&g.hflag[v], f);
-                if (owner1) atomicMin(&g.hbest[v], best);
-                else atomicMax(&g.hbest[v], best);
-                __threadfence();
+                if (f) egs_complete(atomicOr(&g.hflag[v], f));
+                egs_complete(owner1 ? atomicMin(&g.hbest[v], best) : atomicMax(&g.hbest[v], best));
                 done = atomicAdd(&g.hcnt[v], 1) == contrib - 1;
                 if (done) {
-                    __threadfence();
                     f = atomicExch(&g.hflag[v], 0);
                     best = atomicExch((unsigned long long *)&g.hbest[v],
                                       (unsigned long long)(owner1 ? LLONG_MAX : LLONG_MIN));
@@ -787,13 +784,10 @@ __device__ __forceinline__ void bf_huge_part(const DevGame &g, long long *__rest
             bool last = true;
             int f = (need ? 1 : 0) | (out ? 2 : 0);
             if (contrib > 1) {
-                if (f) atomicOr(&g.hflag[v], f);
-                if (owner1) atomicMin(&g.hbest[v], best);
-                else atomicMax(&g.hbest[v], best);
-                __threadfence();
+                if (f) egs_complete(atomicOr(&g.hflag[v], f));
+                egs_complete(owner1 ? atomicMin(&g.hbest[v], best) : atomicMax(&g.hbest[v], best));
                 last = atomicAdd(&g.hcnt[v], 1) == contrib - 1;
                 if (last) {
-                    __threadfence();
                     f = atomicExch(&g.hflag[v], 0);
                     best = atomicExch((unsigned long long *)&g.hbest[v],
                                       (unsigned long long)(owner1 ? LLONG_MAX : LLONG_MIN));

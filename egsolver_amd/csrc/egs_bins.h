@@ -232,8 +232,7 @@ __device__ __forceinline__ void bin_fold(const DevGame &g, const T *cand, int b,
 // that completes it, which gets the whole fold and leaves the words neutral again.  Only
 // atomics touch the words, and each is complete (its result used) before the next.
 __device__ __forceinline__ bool bin_share_fold(const DevGame &g, int v, int &fold) {
-    const int before = atomicMin(&g.hacc[v], fold);
-    asm volatile("" ::"v"(before) : "memory");
+    egs_complete(atomicMin(&g.hacc[v], fold));
     if (atomicAdd(&g.hcnt[v], 1) != bin_holders(g, v) - 1) return false;
     fold = atomicExch(&g.hacc[v], INT_MAX);
     g.hcnt[v] = 0;
@@ -243,8 +242,7 @@ __device__ __forceinline__ bool bin_share_fold(const DevGame &g, int v, int &fol
 // The same for a longest-path candidate in hbest[v], kept as the workgroup-per-vertex passes
 // keep it (owner 0 a maximum, owner 1 a minimum).
 __device__ __forceinline__ bool bin_share_best(const DevGame &g, int v, bool owner1, long long &best) {
-    const long long before = owner1 ? atomicMin(&g.hbest[v], best) : atomicMax(&g.hbest[v], best);
-    asm volatile("" ::"v"(before) : "memory");
+    egs_complete(owner1 ? atomicMin(&g.hbest[v], best) : atomicMax(&g.hbest[v], best));
     if (atomicAdd(&g.hcnt[v], 1) != bin_holders(g, v) - 1) return false;
     best = (long long)atomicExch((unsigned long long *)&g.hbest[v],
                                  (unsigned long long)(owner1 ? LLONG_MAX : LLONG_MIN));

@@ -858,7 +858,8 @@ __device__ __forceinline__ void hub_block(const DevGame &g, int r, int mode, int
         if (part >= contrib) continue;                   // the whole workgroup: u is shared
         // a TOP value is final; every contributor sees it (only v's own last contributor
         // changes v's value in a round, after all others have counted in)
-        if (g.val[v] == EGS_TOP) continue;
+        const int old = g.val[v];
+        if (old == EGS_TOP) continue;
         const bool owner1 = v >= g.n0;
         int key = EGS_TOP;
         for (int c = part; c < chunks; c += contrib) {
@@ -873,11 +874,9 @@ __device__ __forceinline__ void hub_block(const DevGame &g, int r, int mode, int
             for (int c = part; c < chunks; c += contrib) acc.edges += (uint32_t)(min(e, s + (c + 1) * kHugeChunk) - (s + c * kHugeChunk));
             bool last = true;
             if (contrib > 1) {
-                atomicMin(&g.hacc[v], key);
-                __threadfence();
+                egs_complete(atomicMin(&g.hacc[v], key));
                 last = atomicAdd(&g.hcnt[v], 1) == contrib - 1;
                 if (last) {
-                    __threadfence();
                     key = atomicExch(&g.hacc[v], EGS_TOP);   // every contribution, and the reset
                     g.hcnt[v] = 0;
                 }
@@ -888,8 +887,7 @@ __device__ __forceinline__ void hub_block(const DevGame &g, int r, int mode, int
         __syncthreads();
         if (*s_last) {
             const int t = egs_unkey(*s_key, owner1);
-            const int old = g.val[v];
-            const bool lifted = old < t;
+            const bool lifted = old < t;         // old was read before the barriers: thread 0 stores t
             if (threadIdx.x == 0) {
                 acc.processed++;
                 if (lifted) { g.val[v] = t; acc.lifted++; if (g.rise) g.rise[v] = r; if (t == EGS_TOP) g.ring[15] = 1; }
