@@ -104,7 +104,7 @@ int pow2ceil(int x) {
 // n_cap vertices and m_cap edges.  constexpr so that the size of the no-allocation
 // workspace below is known at compile time.
 struct Layout {
-    size_t ptr, edges, cptr, cpred, val, stamp, l0, l1, dbig, dhuge, sbig, shuge, lcnt, mode, ring, rounds, misc,
+    size_t ptr, edges, cptr, cpred, cweight, val, stamp, l0, l1, dbig, dhuge, sbig, shuge, lcnt, mode, ring, rounds, misc,
         tile, fill, stats, statsum, sigma, h, hist, bfcnt, bits, hacc, hcnt, hbest, hflag, tcounts, toffs, tscan,
         titems, slen, sbase, sedges, bigmask, bedges, bcand, boff, bchunk, bdesc, whole, total;
     int64_t tcounts_cap, bin_cap, boff_cap;
@@ -178,6 +178,7 @@ constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
     if (L.bin_cap > 0x7fffffff) L.bin_cap = 0x7fffffff;
     L.bedges = L.binned ? take(6 * (size_t)L.bin_cap + 256) : 0;
     L.bcand = L.binned ? take(8 * (size_t)L.bin_cap) : 0;
+    L.cweight = L.binned ? L.bcand : take(4 * m);      // a game leaves the bins with its transpose
     const size_t chunks = ((size_t)egs::kBinHead * n1 + m) / egs::kBinShareMin + 2;
     L.boff_cap = L.binned ? (int64_t)((size_t)L.bin_cap / egs::kBinPad + chunks) : 0;
     L.boff = L.binned ? take(4 * (size_t)L.boff_cap) : 0;
@@ -200,7 +201,7 @@ struct egs_solver {
     int64_t m_cap = 0;
     void *block = nullptr;
     size_t block_bytes = 0;
-    int *d_ptr = nullptr, *d_cptr = nullptr, *d_cpred = nullptr, *d_val = nullptr;
+    int *d_ptr = nullptr, *d_cptr = nullptr, *d_cpred = nullptr, *d_cweight = nullptr, *d_val = nullptr;
     int *d_stamp = nullptr, *d_list[2] = {nullptr, nullptr}, *d_dbig = nullptr, *d_dhuge = nullptr;
     int *d_sbig = nullptr, *d_shuge = nullptr, *d_lcnt = nullptr, *d_mode = nullptr;
     int *d_ring = nullptr, *d_rounds = nullptr, *d_misc = nullptr, *d_tile = nullptr, *d_fill = nullptr;
@@ -274,6 +275,7 @@ static void bind_layout(egs_solver *s, char *b, const Layout &L) {
     s->d_edges = (int2 *)(b + L.edges);
     s->d_cptr = (int *)(b + L.cptr);
     s->d_cpred = (int *)(b + L.cpred);
+    s->d_cweight = (int *)(b + L.cweight);
     s->d_val = (int *)(b + L.val);
     s->d_stamp = (int *)(b + L.stamp);
     s->d_list[0] = (int *)(b + L.l0);
@@ -810,6 +812,7 @@ static bool bins_pay(const egs_solver *s) {
 
 static void pick_bins(egs_solver *s, const egs_options *o) {
     egs::DevGame &g = s->g;
+    g.cweight = nullptr;
     g.bins = 0;
     g.bin_w = g.bin_parts = g.nchunks = g.bin_share = 0;
     g.bin_magic = 0;
@@ -938,8 +941,15 @@ static int pick_shape(egs_solver *s, const egs_options *o) {
 
 // Transpose on the solver stream, then open the sparse round modes (ring[12] = 1).
 static hipError_t build_csc(egs_solver *s) {
-    hipError_t e = egs::transpose_sorted_fits(s->g.n, s->g.m, s->tcounts_cap, s->m_cap)
-                       ? egs::launch_transpose_sorted(s->g, s->d_tcounts, s->d_toffs, s->d_tscan, s->d_titems,
+    const bool sorted = egs::transpose_sorted_fits(s->g.n, s->g.m, s->tcounts_cap, s->m_cap);
+    // with the weights where there are hubs to keep out of the rounds (pred_can_rise; without,
+    // the look at them costs a round 1.5 us of 13 and saves nothing: 2-regular games took 13%
+    // longer); in the place of a binned game's candidates.  Graphs keep the arguments they were
+    // captured with, so not there.
+    int *cweight = sorted && s->sh.use_wave && !s->use_graphs && egs::transpose_weights_fit(s->g.n, s->wmax) ? s->d_cweight : nullptr;
+    s->g.cweight = cweight;
+    hipError_t e = sorted
+                       ? egs::launch_transpose_sorted(s->g, s->d_tcounts, s->d_toffs, s->d_tscan, s->d_titems, cweight,
                                                       s->stream)
                        : egs::launch_transpose(s->g, s->d_tile, s->d_fill, s->stream);
     if (e == hipSuccess)

@@ -32,6 +32,7 @@ struct DevGame {
     const int2 *edges;    // m packed {successor, weight}
     const int *cptr;      // n+1 CSC offsets
     const int *cpred;     // m predecessors
+    const int *cweight;   // the weights of their edges (null: the transpose does not hold them)
     int *val;             // n values
     int *stamp;           // n: last round a vertex was claimed for / queued for
     int *list[2];         // output lists, ping-pong: kSub*sub_cap + n slots each
@@ -244,7 +245,9 @@ hipError_t launch_transpose(const DevGame &g, int *tile_sum, int *fill, hipStrea
 int transpose_bshift(int n);
 int64_t transpose_counts_len(int n, int64_t m);
 bool transpose_sorted_fits(int n, int64_t m, int64_t counts_cap, int64_t items_cap);
-hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int *scan_tiles, int2 *items,
+// cweight (may be null, for games that transpose_weights_fit): the weights of cpred's edges.
+bool transpose_weights_fit(int n, int wmax);
+hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int *scan_tiles, int2 *items, int *cweight,
                                    hipStream_t st);
 // bad (may be null): a non-zero word makes the kernels return at once.
 hipError_t launch_exclusive_scan(const int *in, int n, int *tile_sum, int *out, hipStream_t st,

@@ -173,12 +173,18 @@ __global__ __launch_bounds__(256) void k_tr_matrix(const int *__restrict__ in, i
 
 constexpr int kTrU = 8;   // chunks of 64 whose loads are in flight together
 
+// An item's second word: the destination within the bucket, under the weight when the
+// predecessor lists carry weights (they fit: transpose_weights_fit).
+__device__ __forceinline__ int tr_item(int2 edge, int dmask, int bshift, int weights) {
+    return (edge.x & dmask) | (weights ? (int)((unsigned)edge.y << bshift) : 0);
+}
+
 // One wave per tile: the tile's run of each bucket is this wave's alone, so it is written
 // contiguously and in edge order (a lane's rank among the lanes of the same bucket comes
 // from ballots over the bucket bits).  pos[] starts at the run starts the scan gave.
 __global__ __launch_bounds__(64) void k_tr_scatter(const int *__restrict__ src, const int2 *__restrict__ edges,
                                                    int64_t m, int bshift, int nb, const int *__restrict__ offs,
-                                                   int2 *__restrict__ items) {
+                                                   int weights, int2 *__restrict__ items) {
     extern __shared__ int pos[];                   // [nb]
     const int lane = threadIdx.x;
     const int bits = 32 - __clz(nb - 1 > 0 ? nb - 1 : 1);
@@ -201,7 +207,7 @@ __global__ __launch_bounds__(64) void k_tr_scatter(const int *__restrict__ src, 
             const int bk = ew[q].x >> bshift;
             const unsigned long long eq = match_lanes(valid ? bk : -1, bits + 1);
             const int base = valid ? pos[bk] : 0;
-            if (valid) items[base + __popcll(eq & lanes_below())] = make_int2(sv[q], ew[q].x & dmask);
+            if (valid) items[base + __popcll(eq & lanes_below())] = make_int2(sv[q], tr_item(ew[q], dmask, bshift, weights));
             if (valid && (eq & lanes_below()) == 0) pos[bk] = base + __popcll(eq);
         }
     }
@@ -214,10 +220,11 @@ __global__ __launch_bounds__(64) void k_tr_scatter(const int *__restrict__ src, 
 // waves in order), and each wave places its run in order.
 __global__ __launch_bounds__(256) void k_tr_bucket(const int2 *__restrict__ items, int n, int64_t m, int bshift,
                                                    int tiles, const int *__restrict__ offs, int skip_below,
-                                                   int *__restrict__ cptr, int *__restrict__ cpred) {
+                                                   int *__restrict__ cptr, int *__restrict__ cpred,
+                                                   int *__restrict__ cweight) {
     extern __shared__ int cd[];                   // [kTrWaves][width]
     __shared__ int lds[4];
-    const int width = 1 << bshift;
+    const int width = 1 << bshift, dmask = width - 1;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int b = blockIdx.x;
     const int64_t i0 = offs[(size_t)b * tiles];
@@ -230,7 +237,7 @@ __global__ __launch_bounds__(256) void k_tr_bucket(const int2 *__restrict__ item
     for (int64_t c0 = w0; c0 < w1; c0 += 64 * kTrU) {
         int d[kTrU];
 #pragma unroll
-        for (int q = 0; q < kTrU; q++) d[q] = c0 + q * 64 + lane < w1 ? items[c0 + q * 64 + lane].y : -1;
+        for (int q = 0; q < kTrU; q++) d[q] = c0 + q * 64 + lane < w1 ? items[c0 + q * 64 + lane].y & dmask : -1;
 #pragma unroll
         for (int q = 0; q < kTrU; q++)
             if (d[q] >= 0) atomicAdd(&cd[wave * width + d[q]], 1);
@@ -269,10 +276,14 @@ __global__ __launch_bounds__(256) void k_tr_bucket(const int2 *__restrict__ item
 #pragma unroll
         for (int q = 0; q < kTrU; q++) {
             const bool valid = c0 + q * 64 + lane < w1;
-            const unsigned long long eq = match_lanes(valid ? it[q].y : -1, bshift + 1);
-            const int base = valid ? cd[wave * width + it[q].y] : 0;
-            if (valid) cpred[base + __popcll(eq & lanes_below())] = it[q].x;
-            if (valid && (eq & lanes_below()) == 0) cd[wave * width + it[q].y] = base + __popcll(eq);
+            const int d = it[q].y & dmask;
+            const unsigned long long eq = match_lanes(valid ? d : -1, bshift + 1);
+            const int base = valid ? cd[wave * width + d] : 0;
+            if (valid) {
+                cpred[base + __popcll(eq & lanes_below())] = it[q].x;
+                if (cweight) cweight[base + __popcll(eq & lanes_below())] = it[q].y >> bshift;
+            }
+            if (valid && (eq & lanes_below()) == 0) cd[wave * width + d] = base + __popcll(eq);
         }
     }
 }
@@ -308,10 +319,11 @@ __device__ __forceinline__ int bucket_of_slot(const int *start, int nb, int i) {
 // bucket leaves as whole lines instead of one partial line per item.  An item waits in LDS
 // as 32 bits: (source - the tile's first source) << bshift | destination within the bucket,
 // or the edge's offset in the tile in place of the source difference when the tile's
-// sources span 2^(32 - bshift) or more (only possible with vertices that have no edges).
+// sources span 2^(32 - bshift) or more (only possible with vertices that have no edges) and
+// with weights, which are read again from the tile.
 __global__ __launch_bounds__(1024) void k_tr_scatter_lds(const int *__restrict__ src, const int2 *__restrict__ edges,
                                                          int64_t m, int bshift, int nb, const int *__restrict__ offs,
-                                                         int2 *__restrict__ items) {
+                                                         int weights, int2 *__restrict__ items) {
     extern __shared__ int ldyn[];
     unsigned *cw = (unsigned *)ldyn;                                    // [16][nb] halves
     unsigned short *c16 = (unsigned short *)ldyn;
@@ -325,7 +337,7 @@ __global__ __launch_bounds__(1024) void k_tr_scatter_lds(const int *__restrict__
     const int64_t e0 = (int64_t)blockIdx.x * kTrTile, e1 = min(m, e0 + kTrTile);
     const int cnt = (int)(e1 - e0);
     const int src0 = src[e0];
-    const bool by_source = (int64_t)src[e1 - 1] - src0 < (1ll << (32 - bshift));
+    const bool by_source = !weights && (int64_t)src[e1 - 1] - src0 < (1ll << (32 - bshift));
     const int wbase = wave * kTrLChunks * 64;
     int d[kTrLChunks], sv[kTrLChunks];
 #pragma unroll
@@ -380,7 +392,8 @@ __global__ __launch_bounds__(1024) void k_tr_scatter_lds(const int *__restrict__
         const unsigned x = slot[i];
         const int key = (int)(x >> bshift);
         const int b = bucket_of_slot(lstart, nb, i);
-        items[delta[b] + i] = make_int2(by_source ? src0 + key : src[e0 + key], (int)(x & (unsigned)dmask));
+        items[delta[b] + i] = make_int2(by_source ? src0 + key : src[e0 + key],
+                                        weights ? tr_item(edges[e0 + key], dmask, bshift, 1) : (int)(x & (unsigned)dmask));
     }
 }
 
@@ -389,9 +402,10 @@ __global__ __launch_bounds__(1024) void k_tr_scatter_lds(const int *__restrict__
 // (a random 4-byte store per item reached HBM as a partial line, about 8x the bytes).
 __global__ __launch_bounds__(1024) void k_tr_bucket_lds(const int2 *__restrict__ items, int n, int64_t m, int bshift,
                                                         int tiles, const int *__restrict__ offs, int cap,
-                                                        int *__restrict__ cptr, int *__restrict__ cpred) {
+                                                        int *__restrict__ cptr, int *__restrict__ cpred,
+                                                        int *__restrict__ cweight) {
     extern __shared__ int ldyn[];
-    const int width = 1 << bshift;
+    const int width = 1 << bshift, dmask = width - 1;
     unsigned *cw = (unsigned *)ldyn;                                    // [16][width] halves
     unsigned short *c16 = (unsigned short *)ldyn;
     int *out = ldyn + kTrLWaves * width / 2;                            // [cap]
@@ -408,13 +422,13 @@ __global__ __launch_bounds__(1024) void k_tr_bucket_lds(const int2 *__restrict__
 #pragma unroll
     for (int q = 0; q < kTrLBucketChunks; q++) {
         const int i = w0 + q * 64 + lane;
-        it[q] = i < w1 ? items[i0 + i] : make_int2(0, -1);
+        it[q] = i < w1 ? items[i0 + i] : make_int2(0, 0);
     }
     for (int i = threadIdx.x; i < kTrLWaves * width / 2; i += blockDim.x) cw[i] = 0;
     __syncthreads();
 #pragma unroll
     for (int q = 0; q < kTrLBucketChunks; q++)
-        if (it[q].y >= 0) lds_count16(cw, wave * width + it[q].y);
+        if (w0 + q * 64 + lane < w1) lds_count16(cw, wave * width + (it[q].y & dmask));
     __syncthreads();
     int carry = 0;
     for (int d0 = 0; d0 < width; d0 += blockDim.x) {
@@ -441,15 +455,23 @@ __global__ __launch_bounds__(1024) void k_tr_bucket_lds(const int2 *__restrict__
     if (b == gridDim.x - 1 && threadIdx.x == 0) cptr[n] = (int)m;
 #pragma unroll
     for (int q = 0; q < kTrLBucketChunks; q++) {
-        const bool valid = it[q].y >= 0;
-        const int d = it[q].y;
-        const unsigned long long eq = match_lanes(d, bshift + 1);
-        const int base = valid ? c16[wave * width + d] : 0;
-        if (valid) out[base + __popcll(eq & lanes_below())] = it[q].x;
+        const bool valid = w0 + q * 64 + lane < w1;
+        const int d = it[q].y & dmask;
+        const unsigned long long eq = match_lanes(valid ? d : -1, bshift + 1);
+        const int base = valid ? c16[wave * width + d] : 0, at = base + __popcll(eq & lanes_below());
+        if (valid) out[at] = it[q].x;
+        it[q].x = at;
         if (valid && (eq & lanes_below()) == 0) c16[wave * width + d] = (unsigned short)(base + __popcll(eq));
     }
     __syncthreads();
     for (int i = threadIdx.x; i < cnt; i += blockDim.x) cpred[i0 + i] = out[i];
+    if (!cweight) return;
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < kTrLBucketChunks; q++)
+        if (w0 + q * 64 + lane < w1) out[it[q].x] = it[q].y >> bshift;
+    __syncthreads();
+    for (int i = threadIdx.x; i < cnt; i += blockDim.x) cweight[i0 + i] = out[i];
 }
 
 // Bucket width 2^bshift: at least 2048 destinations and at most kTrMaxBuckets buckets.
@@ -469,9 +491,11 @@ bool transpose_sorted_fits(int n, int64_t m, int64_t counts_cap, int64_t items_c
            m <= items_cap && n > 0 && m > 0 && m < 0x7fffffff;
 }
 
-hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int *scan_tiles, int2 *items,
+bool transpose_weights_fit(int n, int wmax) { return wmax < 1 << (31 - transpose_bshift(n)); }
+
+hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int *scan_tiles, int2 *items, int *cweight,
                                    hipStream_t st) {
-    const int n = g.n;
+    const int n = g.n, weights = cweight != nullptr;
     const int64_t m = g.m;
     const int bshift = transpose_bshift(n);
     const int nb = (int)(((int64_t)n + (1LL << bshift) - 1) >> bshift);
@@ -494,10 +518,10 @@ hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int
     if (nb <= kTrLMaxBuckets) {
         const size_t lds = sizeof(int) * ((size_t)kTrLWaves * nb / 2 + 2 * (size_t)nb + kTrTile);
         hipLaunchKernelGGL(k_tr_scatter_lds, dim3(tiles), dim3(1024), lds, st, (const int *)src, g.edges, m, bshift, nb,
-                           (const int *)offs, items);
+                           (const int *)offs, weights, items);
     } else {
         hipLaunchKernelGGL(k_tr_scatter, dim3(tiles), dim3(64), sizeof(int) * (size_t)nb, st, (const int *)src, g.edges,
-                           m, bshift, nb, (const int *)offs, items);
+                           m, bshift, nb, (const int *)offs, weights, items);
     }
     // buckets of at most `cap` items are placed in LDS (16 x width 16-bit counters and
     // out[cap]); the rest, or every bucket when the counters do not fit, in HBM
@@ -506,11 +530,11 @@ hipError_t launch_transpose_sorted(const DevGame &g, int *counts, int *offs, int
     if (cap > 0) {
         const size_t lds = (size_t)counters + sizeof(int) * (size_t)cap;
         hipLaunchKernelGGL(k_tr_bucket_lds, dim3(nb), dim3(1024), lds, st, (const int2 *)items, n, m, bshift, tiles,
-                           (const int *)counts, cap, const_cast<int *>(g.cptr), const_cast<int *>(g.cpred));
+                           (const int *)counts, cap, const_cast<int *>(g.cptr), const_cast<int *>(g.cpred), cweight);
     }
     hipLaunchKernelGGL(k_tr_bucket, dim3(nb), dim3(256), sizeof(int) * (size_t)kTrWaves << bshift, st,
                        (const int2 *)items, n, m, bshift, tiles, (const int *)counts, cap > 0 ? cap : -1,
-                       const_cast<int *>(g.cptr), const_cast<int *>(g.cpred));
+                       const_cast<int *>(g.cptr), const_cast<int *>(g.cpred), cweight);
     return hipGetLastError();
 }
 
