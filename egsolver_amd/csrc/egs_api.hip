@@ -87,6 +87,7 @@ constexpr int kWholeDenseN = 1 << 16; // single launches sweep every round dense
                                      // sparse rounds goes to the round kernels
 constexpr int64_t kMemorySideCache = 256 << 20;
 constexpr int kBinDensePart = 128;    // a binned round wants the transpose below 1/128 of the vertices
+constexpr int kTailRounds = 4096;     // rounds of a one-workgroup launch at most (tens of milliseconds)
 constexpr int kStopBatch = 4;         // rounds queued ahead of the host when a stop flag is polled
 
 double egs_now_ms() {
@@ -1240,6 +1241,7 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
     int pending = -1;     // probe slot in flight
     bool done = false;
     int batch = 4;        // grow towards batch_rounds so short solves do not overshoot much
+    int64_t listed = -1;  // items of the latest list read back (-1: not known)
     while (!done && launched < limit) {
         int nb = (int)std::min<int64_t>(batch, limit - launched);
         const bool accel = s->cert_every > 0;
@@ -1289,6 +1291,7 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
                 // proving small sets does not pay an attempt every few rounds
                 batch = 1;        // the fixpoint often follows at once: probe again early
                 nb = 1;
+                listed = -1;
             } else {
                 s->cert_gap = std::min(s->cert_gap * 2, 1 << 16);
                 if (cr.cap_hit) s->cert_cap = std::min(s->cert_cap * 2, s->cert_max_passes);
@@ -1297,6 +1300,30 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
             pending = -1;
         }
         if (accel) nb = (int)std::max<int64_t>(1, std::min<int64_t>(nb, s->next_cert - (s->next_round - 1)));
+        // a short list after the transpose: the sparse tail, in launches of as many rounds as are
+        // left before the next proof attempt (not with a stop flag, which is polled every round)
+        if (listed > 0 && listed <= egs::tail_items(s->sh) && s->csc_built && !s->use_graphs && !s->stop_flag) {
+            int64_t most = std::min<int64_t>(limit - launched, kTailRounds);
+            if (accel) most = std::max<int64_t>(1, std::min(most, s->next_cert - (s->next_round - 1)));
+            HIP_TRY(egs::launch_tail(s->g, s->sh, (int)most, s->stream));
+            // the counters of all three lists, the modes and the ring lie in this order
+            int *hp = s->h_probe + kPinProbe;
+            HIP_TRY(hipMemcpyAsync(hp, s->d_lcnt, sizeof(int) * (size_t)(s->d_ring + 16 - s->d_lcnt), hipMemcpyDeviceToHost,
+                                   s->stream));
+            HIP_TRY(probe_mark(s, 0));
+            HIP_TRY(probe_wait(s, 0));
+            pending = -1;
+            const int reached = hp[s->d_ring + 14 - s->d_lcnt];
+            const int ran = reached - (int)s->next_round;
+            listed = -1;
+            if (ran > 0) {
+                s->next_round = reached;
+                launched += ran;
+                listed = list_total(s, hp + (reached % 3) * egs::kListCounters);
+                if (listed == 0) done = true;
+                continue;
+            }
+        }
         int k = 0;
         if (s->use_graphs) {
             for (int b = kGraphSizes - 1; b >= 0; b--)
@@ -1336,7 +1363,8 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
         HIP_TRY(probe_mark(s, slot));
         if (pending >= 0) {
             HIP_TRY(probe_wait(s, pending));
-            if (list_total(s, s->h_probe + kPinProbe + pending * kProbeStride) == 0) done = true;
+            listed = list_total(s, s->h_probe + kPinProbe + pending * kProbeStride);
+            if (listed == 0) done = true;
             // enough rounds wanted to go sparse: build the transpose now
             if (!done && !s->csc_built && s->h_probe[kPinProbe + pending * kProbeStride + s->probe_want[pending]] >= (s->g.bins ? kSparseWantBinned : kSparseWantRounds))
                 HIP_TRY(build_csc(s));

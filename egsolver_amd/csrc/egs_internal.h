@@ -280,6 +280,11 @@ int pack_shift(int n, int wmax);
 // Round j of a batch (absolute round ring[14] + j); launch_advance ends the batch.
 hipError_t launch_round(const DevGame &g, const LaunchShape &sh, int j, hipStream_t st);
 hipError_t launch_advance(const DevGame &g, int rounds, hipStream_t st);
+// Rounds in one workgroup from the next one on, `limit` at most, while each is sparse and its
+// list short; ring[14] tells the round reached.  For lists of up to tail_items(sh).
+constexpr int kTailLanes = 2048;           // items times lanes a vertex: two turns of the workgroup
+int tail_items(const LaunchShape &sh);
+hipError_t launch_tail(const DevGame &g, const LaunchShape &sh, int limit, hipStream_t st);
 // Round `next` is the first of the round kernels on values reached otherwise (after
 // launch_prepare_reset): a full sweep, or none when they have converged.
 hipError_t launch_resume(const DevGame &g, int next, bool converged, hipStream_t st);

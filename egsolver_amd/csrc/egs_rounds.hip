@@ -545,6 +545,147 @@ __global__ __launch_bounds__(256) void k_round(DevGame g, int j) {
     flush_stats(g, acc);
 }
 
+// ---------------------------------------------------------------------------------------
+// the sparse tail in one workgroup
+// ---------------------------------------------------------------------------------------
+
+// Rounds of QUEUE mode while their lists are short, `limit` of them at most: one workgroup, the
+// lists in LDS, a barrier where the round kernels have a launch.  A round of a few hundred
+// vertices is a chain of dependent loads: ten of them and two launches take the round kernels
+// 16 to 20 us, mostly misses past an L2 that each launch starts cold; here the chain is six,
+// through one compute unit's L1 and a warm L2 (3.3 us a round on the skewed 2^20 game).
+// A list past `most` items ends the run after its round, as an empty one does, and the state
+// left is the round kernels' own: the next round's list (in the overflow region) and counters,
+// the last mode, ring[14].  It returns at once where the next round is not of QUEUE mode.
+constexpr int kTailCap = 8192;             // items of a list kept in LDS
+constexpr int kTailHubs = 2048;            // most items of a round (launch_tail)
+
+template <int G>
+__global__ __launch_bounds__(1024) void k_tail(DevGame g, int limit, int most) {
+    __shared__ int lists[2][kTailCap], hub[kTailHubs];
+    __shared__ int pre[kSub + 2], wmin[16];
+    __shared__ int s_go, s_out, s_hubs;
+    const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6, gl = tid % G;
+    int r = g.ring[14];
+    load_layout(g, r % 3, pre);
+    __syncthreads();
+    int c = pre[kSub + 1];
+    if (tid == 0) {
+        const int want = decide_mode(g, r, c);
+        s_go = want == MODE_QUEUE && gate_mode(g, want, r) == MODE_QUEUE && c <= most;
+    }
+    __syncthreads();
+    if (!s_go) return;
+    for (int i = tid; i < c; i += 1024) lists[0][i] = g.list[r & 1][layout_slot(g, pre, i)];
+    LiftAcc acc;
+    int at = 0, rounds = 0;
+    while (true) {
+        const int *in = lists[at];
+        int *out = lists[at ^ 1], *far = g.list[(r + 1) & 1] + kSub * g.sub_cap;   // items past kTailCap, by place
+        if (tid == 0) { s_out = 0; s_hubs = 0; }
+        __syncthreads();
+        // the predecessors of u, which rose, by lanes l of n (stamps are set by atomics past
+        // the L1, so they are read past it)
+        auto push = [&](int u, int old, int now, bool hubs_run, int l, int n) {
+            const int ce = g.cptr[u + 1];
+            for (int k = g.cptr[u] + l; k < ce; k += n) {
+                const int p = g.cpred[k];
+                const int stamp = __hip_atomic_load(&g.stamp[p], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                if (stamp > r) continue;
+                if (g.cweight && !pred_can_rise(g, p, stamp, g.cweight[k], old, now, r, hubs_run)) continue;
+                if (atomicMax(&g.stamp[p], r + 1) > r) continue;
+                const int pos = atomicAdd(&s_out, 1);
+                if (pos < kTailCap) out[pos] = p;
+                else far[pos] = p;
+            }
+        };
+        auto rise = [&](int v, int t) {
+            g.val[v] = t;
+            if (g.rise) g.rise[v] = r;
+            if (t == EGS_TOP) g.ring[15] = 1;
+            acc.lifted++;
+            acc.preds += (uint32_t)(g.cptr[v + 1] - g.cptr[v]);
+        };
+        for (int i0 = 0; i0 < c; i0 += 1024 / G) {
+            const int i = i0 + tid / G;
+            int v = 0, s = 0, e = 0, old = EGS_TOP;
+            if (i < c) {
+                v = in[i];
+                s = g.ptr[v];
+                e = g.ptr[v + 1];
+                if (e - s > g.big_deg) {
+                    if (gl == 0) hub[atomicAdd(&s_hubs, 1)] = v;
+                    e = s;
+                } else {
+                    old = g.val[v];
+                    if (gl == 0) {
+                        acc.processed++;
+                        acc.edges += (uint32_t)(e - s);
+                    }
+                }
+            }
+            const int t = lift_value<G>(g, s, e, gl, v >= g.n0);
+            if (old < t && e > s) {
+                if (gl == 0) rise(v, t);
+                push(v, old, t, false, gl, G);
+            }
+        }
+        __syncthreads();
+        const int hubs = s_hubs;
+        for (int h = 0; h < hubs; h++) {
+            const int v = hub[h], s = g.ptr[v], e = g.ptr[v + 1], old = g.val[v];
+            if (old == EGS_TOP) continue;
+            int key = egs_group_min<64>(key_over_edges<8>(g, s, e, tid, 1024, v >= g.n0));
+            if (lane == 0) wmin[wid] = key;
+            __syncthreads();                     // `old` has been read by everyone, too
+            key = wmin[0];
+            for (int w = 1; w < 16; w++) key = min(key, wmin[w]);
+            const int t = egs_unkey(key, v >= g.n0);
+            if (tid == 0) {
+                acc.processed++;
+                acc.edges += (uint32_t)(e - s);
+                if (old < t) rise(v, t);
+            }
+            if (old < t) push(v, old, t, true, tid, 1024);
+            __syncthreads();
+        }
+        __syncthreads();
+        c = s_out;
+        r++;
+        rounds++;
+        at ^= 1;
+        if (c == 0 || c > most || rounds >= limit) break;
+        __syncthreads();                         // s_out is read by everyone before it is cleared
+    }
+    for (int i = tid; i < min(c, kTailCap); i += 1024) g.list[r & 1][kSub * g.sub_cap + i] = lists[at][i];
+    for (int i = tid; i < kListCounters; i += 1024) {
+        g.lcnt[(r % 3) * kListCounters + i] = i == kSub ? c : 0;
+        g.lcnt[((r + 1) % 3) * kListCounters + i] = 0;
+    }
+    if (tid == 0) {
+        g.mode[(r + 2) % 3] = MODE_QUEUE;
+        g.ring[3 + r % 3] = 0;
+        g.ring[6 + r % 3] = 0;
+        g.ring[14] = r;
+        *g.rounds_done = r - 1;
+    }
+    flush_stats(g, acc);
+}
+
+int tail_items(const LaunchShape &sh) { return std::min(kTailHubs, kTailLanes / sh.group); }
+
+hipError_t launch_tail(const DevGame &g, const LaunchShape &sh, int limit, hipStream_t st) {
+    const int most = 2 * tail_items(sh) < kTailHubs ? 2 * tail_items(sh) : kTailHubs;
+    switch (sh.group) {
+    case 1: hipLaunchKernelGGL(k_tail<1>, dim3(1), dim3(1024), 0, st, g, limit, most); break;
+    case 2: hipLaunchKernelGGL(k_tail<2>, dim3(1), dim3(1024), 0, st, g, limit, most); break;
+    case 4: hipLaunchKernelGGL(k_tail<4>, dim3(1), dim3(1024), 0, st, g, limit, most); break;
+    case 8: hipLaunchKernelGGL(k_tail<8>, dim3(1), dim3(1024), 0, st, g, limit, most); break;
+    default: hipLaunchKernelGGL(k_tail<16>, dim3(1), dim3(1024), 0, st, g, limit, most); break;
+    }
+    return hipGetLastError();
+}
+
 // Exclusive prefix sum over the 64 lanes of a wave (every lane active).
 __device__ __forceinline__ int wave_excl_scan(int x) { return egs_wave_incl_scan(x) - x; }
 

@@ -31,3 +31,32 @@ def test_hub_queues_exact(oracle, i, certify_every):
             assert conv
             vals = s.values()
             assert np.array_equal(vals, ref), (opt, np.count_nonzero(vals != ref))
+
+
+@pytest.mark.parametrize("leaves", [500, 8192, 8193, 30000])
+def test_one_workgroup_rounds_hand_over(leaves):
+    """A value that travels up a chain, one vertex a round, then to `leaves` vertices at once
+    (past the lists a workgroup keeps, they go to the round kernels), then up a second chain."""
+    import egsolver_amd as E
+    from egsolver_amd.games import Game
+    chain = 4200                                  # past one launch's rounds
+    # owner 1 everywhere: 0 a sink, 1..chain the first chain, then the leaves, then the second
+    leaf0, second = 1 + chain, 1 + chain + leaves
+    n = second + chain
+    succ = np.zeros(n, np.int32)
+    succ[1:leaf0] = np.arange(chain)
+    succ[leaf0:second] = chain
+    succ[second] = leaf0 + leaves // 2
+    succ[second + 1:] = np.arange(second, n - 1)
+    w = np.zeros(n, np.int32)
+    w[1] = -5
+    g = Game(n=n, n0=0, ptr=np.arange(n + 1, dtype=np.int32), succ=succ, w=w, mg=5, ext_of_int=np.arange(n, dtype=np.int32))
+    ref = np.full(n, 5, np.int32)
+    ref[0] = 0
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        print(f"[gpu-case] chain of {chain}, {leaves} leaves", flush=True)
+        s.prepare(E.options(certify_every=-1, dense_pct=101))
+        conv, st = s.iterate()
+        assert conv and st.phases == 2 * chain + 1
+        assert np.array_equal(s.values(), ref)
