@@ -1387,6 +1387,13 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
 
 int egs_solver_stats(egs_solver *s, egs_stats *st) {
     if (!s || !st) return fail(EGS_E_ARG, "null argument");
+    // asked between prepare and the first round: the initial frontier has not been made where
+    // the first launch of the run would make it
+    const bool unborn = s->prepared && (s->bins_open || (s->whole.nb > 0 && s->whole_rounds == 0 && !s->st.converged));
+    if (unborn) {
+        HIP_TRY(hipSetDevice(s->device));
+        if (int rc = leave_whole(s)) return rc;
+    }
     HIP_TRY(close_prepare(s));
     *st = s->st;
     return EGS_OK;

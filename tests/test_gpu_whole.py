@@ -216,3 +216,22 @@ def test_proof_with_every_wave_changing():
         conv, st = s.iterate()
         assert conv and st.certificates > 0, st.as_dict()
         assert s.violations() == 0
+
+
+@pytest.mark.parametrize("n", [61, 20011, 420001])
+def test_initial_frontier_before_the_first_round(oracle, n):
+    """The statistics between prepare and the first round hold the initial frontier's size,
+    whatever runs the rounds, and the solve after them is the usual one."""
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=n, seed=4, deg_kind=E.games.DEG_UNIFORM, deg_lo=3, deg_hi=9, wmax=50))
+    _say(f"initial frontier of {n}")
+    neg = (g.w < 0).astype(np.int64)
+    cnt, deg = np.add.reduceat(neg, g.ptr[:-1]), np.diff(g.ptr)
+    act = np.where(np.arange(n) < g.n0, cnt == deg, cnt > 0)
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        s.prepare()
+        st = s.stats()
+        assert st.initial_active == act.sum() and st.ms_prepare > 0
+        conv, st = s.iterate()
+        assert conv and st.initial_active == act.sum() and s.violations() == 0
