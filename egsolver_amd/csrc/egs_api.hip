@@ -76,6 +76,7 @@ constexpr int kSparseWantRounds = 6;
 constexpr int kSparseWantBinned = 16;
 constexpr int kCertFirstCap = 64;     // longest-path passes per candidate at the first attempt
 constexpr int kCertCandidates = 8;    // gap thresholds tried per attempt (plus the last-round rise set)
+constexpr int kCertTryRounds = 12;    // a candidate's launches and read-back, in rounds
 constexpr int kCertEvery = 7;         // default rounds before the first proof attempt
 // ... of a binned game, whose rounds all start from the round before's values and cost less: a
 // first attempt after 7 or 8 rounds more often fails (with 9 the solve of 10^6 vertices of
@@ -1293,7 +1294,7 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
                 nb = 1;
                 listed = -1;
             } else {
-                s->cert_gap = std::min(s->cert_gap * 2, 1 << 16);
+                s->cert_gap = egs::cert_next_gap(s->cert_gap, s->cert_every, cr.passes + kCertTryRounds * cr.tried);
                 if (cr.cap_hit) s->cert_cap = std::min(s->cert_cap * 2, s->cert_max_passes);
             }
             s->next_cert = s->next_round - 1 + s->cert_gap;

@@ -138,6 +138,17 @@ struct LaunchShape {
     int wave_grid, block_grid;
 };
 
+// Rounds to the next proof attempt after one that proved nothing and cost as much as `cost`
+// rounds: twice as many as to this one, while attempts would take less than a sixteenth of the
+// rounds.  Doubled without end, a long run whose vertices could be proved at round r went on to
+// the next power of two: games of degree 2 with 485,000 vertices took 61, 135 and 368 ms, with
+// at most eight times the cost between attempts 34, 91 and 256; runs that no proof helps took
+// 2 to 8% longer then, which sixteen halves.
+__host__ __device__ inline int cert_next_gap(int gap, int every, int cost) {
+    const int64_t twice = 2 * (int64_t)gap, most = 16 * (int64_t)cost, g = twice < most ? twice : most;
+    return (int)(g > every ? g : every);
+}
+
 // A whole solve in one launch (egs_whole.hip).
 constexpr int kWholeMaxNb = 256;           // workgroups at most
 constexpr int kWholeGroups = 8;            // groups of workgroups in a vote

@@ -119,7 +119,7 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
         key[i] = INT_MAX;
         if (fresh && a.rise) a.rise[v0 + i] = 0;
     }
-    if (tid == 0) { s_acc[0] = 0; s_acc[1] = 0; s_sum[0] = 0; s_sum[1] = 0; }
+    if (tid == 0) { s_acc[0] = 0; s_acc[1] = 0; s_sum[0] = 0; s_sum[1] = 0; s_ncand = 0; }
     __syncthreads();
     // this thread's edges [elo, elo + cnt), the local vertex of the first one, and the slots
     // after which its fold goes to the vertex's key (a row's last edge, the thread's last)
@@ -451,12 +451,13 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
         if (known && vcount(tot) == 0) { status = kWholeDone; break; }
         if (r - a.round0 >= a.limit) break;
         if (a.every > 0 && known && r >= next_cert) {
+            const int before = passes;
             if (!prove((int)r, cap)) return;
             attempts++;
             if (marked > 0) {
                 certs++;
             } else {
-                gap = min(gap * 2, 1 << 16);
+                gap = cert_next_gap(gap, a.every, passes - before + 2 * s_ncand);
                 if (cap_hit) cap = min(cap * 2, a.max_passes);
             }
             next_cert = r + gap;
@@ -529,7 +530,7 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
 // values, rise stamps and potentials in registers and LDS holds what others gather.  A round
 // is D V gathers, three VALU operations each, and one workgroup barrier, in place; the form
 // above spends its time on the folds' LDS atomics and its second phase (1.8 us a round at
-// n = 1,499, degree 4, against EGS_SMALL_US here).
+// n = 1,499, degree 4, against 0.5 here).
 template <int D, int V>
 __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
     extern __shared__ __align__(16) long long dyn[];
@@ -570,6 +571,7 @@ __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
         }
     }
     if (tid < 3) s_flag[tid] = 0;
+    if (tid == 0) s_ncand = 0;
     if (tid < 2) { s_acc[tid] = 0; s_sum[tid] = 0; }
     __syncthreads();
     int slot = 0, par = 0;
@@ -730,12 +732,13 @@ __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
         if (known && !up) { status = kWholeDone; break; }
         if (r - a.round0 >= a.limit) break;
         if (a.every > 0 && known && r >= next_cert) {
+            const int before = passes;
             prove((int)r, cap);
             attempts++;
             if (marked > 0) {
                 certs++;
             } else {
-                gap = min(gap * 2, 1 << 16);
+                gap = cert_next_gap(gap, a.every, passes - before + 2 * s_ncand);
                 if (cap_hit) cap = min(cap * 2, a.max_passes);
             }
             next_cert = r + gap;
