@@ -571,7 +571,6 @@ __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
         }
     }
     if (tid < 3) s_flag[tid] = 0;
-    if (tid == 0) s_ncand = 0;
     if (tid < 2) { s_acc[tid] = 0; s_sum[tid] = 0; }
     __syncthreads();
     int slot = 0, par = 0;
@@ -732,13 +731,14 @@ __global__ __launch_bounds__(1024) void k_whole_small(WholeArgs a) {
         if (known && !up) { status = kWholeDone; break; }
         if (r - a.round0 >= a.limit) break;
         if (a.every > 0 && known && r >= next_cert) {
-            const int before = passes;
             prove((int)r, cap);
             attempts++;
             if (marked > 0) {
                 certs++;
             } else {
-                gap = cert_next_gap(gap, a.every, passes - before + 2 * s_ncand);
+                // without cert_next_gap's bound: its registers cost every round 4% (plain value
+                // iteration at n = 1,499: 690 us against 660)
+                gap = min(gap * 2, 1 << 16);
                 if (cap_hit) cap = min(cap * 2, a.max_passes);
             }
             next_cert = r + gap;
