@@ -543,7 +543,7 @@ def main():
         "roofline": {
             "bound": "hbm", "achieved": plain["achieved_gbps"], "peak": HBM_PEAK_GBPS, "unit": "GB/s",
             "frac": plain["achieved_gbps"] / HBM_PEAK_GBPS, "traffic": traffic,
-            "kernel": "dense round: k_round (mode decision) + k_dense_fused (8 successor-range phases in one launch)",
+            "kernel": "dense round: k_bin_gather (candidates from LDS-resident slices of the values) + k_bin_reduce",
             "algorithmic_bytes_per_launch": plain["algorithmic_bytes_per_round"],
             "avg_launch_ms": plain["device_ms_per_round"],
             "copy_kernel_gbps": copy_gbps,
