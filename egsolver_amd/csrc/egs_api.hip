@@ -812,7 +812,9 @@ static bool bins_pay(const egs_solver *s) {
     return g.n <= egs::kBinHalfN ? g.m >= 4 * (int64_t)g.n : 2 * g.m >= 7 * (int64_t)g.n;
 }
 
-static void pick_bins(egs_solver *s, const egs_options *o) {
+// whole: the game runs in single launches, which need none of this; what takes such a run over
+// (leave_whole) finds no layout built for it, so it gets sweeps.
+static void pick_bins(egs_solver *s, const egs_options *o, bool whole) {
     egs::DevGame &g = s->g;
     g.cweight = nullptr;
     g.bins = 0;
@@ -826,7 +828,7 @@ static void pick_bins(egs_solver *s, const egs_options *o) {
     g.bchunk = s->d_bchunk;
     g.bdesc = s->d_bdesc;
     g.hubs = s->max_outdeg > g.huge_deg;
-    if (o->graphs > 0 || o->slices != 0 || !s->d_boff || !bins_pay(s) || g.dense_min > g.n || s->wmax > egs::kBinWmax ||
+    if (whole || o->graphs > 0 || o->slices != 0 || !s->d_boff || !bins_pay(s) || g.dense_min > g.n || s->wmax > egs::kBinWmax ||
         (int64_t)g.mg + 2 * (int64_t)s->wmax >= EGS_TOP || g.n > (int64_t)egs::kBinMax * egs::kBinSlice)
         return;
     // slices and parts that fill the device evenly: 512 workgroups with half slices (two to a
@@ -859,7 +861,7 @@ static void pick_hub_fused(egs_solver *s) {
                   g.round_grid + g.wave_grid + g.block_grid <= egs::kStatSlots;     // a statistics slot per workgroup
 }
 
-static int pick_shape(egs_solver *s, const egs_options *o) {
+static int pick_shape(egs_solver *s, const egs_options *o, bool whole) {
     egs::DevGame &g = s->g;
     egs::LaunchShape &sh = s->sh;
     egs_options def{};
@@ -902,7 +904,7 @@ static int pick_shape(egs_solver *s, const egs_options *o) {
         return fail(EGS_E_ARG, "slices must be 0 (auto) or 1..%d (got %d)", egs::kMaxPhases, o->slices);
     g.phases = 1;
     g.slice_shift = 31;
-    pick_bins(s, o);
+    pick_bins(s, o, whole);
     if (g.bins && o->certify_every == 0) s->cert_every = kCertEveryBinned;
     if (want > 1 && s->d_slen && !g.bins) {
         int shift = 0;
@@ -1153,7 +1155,8 @@ static int run_whole(egs_solver *s, int64_t limit, int *status) {
 int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     if (!s || !s->loaded) return fail(EGS_E_STATE, "egs_solver_prepare: no game loaded");
     HIP_TRY(hipSetDevice(s->device));
-    int rc = pick_shape(s, opt);
+    const egs::WholePlan plan = takes_whole(opt) ? egs::whole_plan(s->g.n, s->g.m, s->g.mg, s->wmax, s->max_outdeg, s->whole_max_nb) : egs::WholePlan{};
+    int rc = pick_shape(s, opt, plan.nb > 0);
     if (rc) return rc;
     HIP_TRY(close_prepare(s));
     s->csc_built = false;
@@ -1166,7 +1169,7 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     s->whole_st = egs_stats{};
     s->mirrored = false;
     s->bins_open = false;
-    s->whole = takes_whole(opt) ? egs::whole_plan(s->g.n, s->g.m, s->g.mg, s->wmax, s->max_outdeg, s->whole_max_nb) : egs::WholePlan{};
+    s->whole = plan;
     if (s->whole.nb > 0) {
         HIP_TRY(egs::launch_whole_prep(s->whole, s->g, s->d_whole, true, s->stream));
         memset(&s->st, 0, sizeof(s->st));

@@ -235,3 +235,128 @@ def test_initial_frontier_before_the_first_round(oracle, n):
         assert st.initial_active == act.sum() and st.ms_prepare > 0
         conv, st = s.iterate()
         assert conv and st.initial_active == act.sum() and s.violations() == 0
+
+
+def _zero_wait(s, us):
+    from egsolver_amd import _native as N
+    fn = N.egs().egs_solver_whole_wait
+    fn.argtypes = [ctypes.c_void_p, ctypes.c_int64]
+    fn.restype = None
+    fn(s.h, us)
+
+
+# hubs from 400,000 vertices on, where every game with one takes binned rounds unless a single
+# launch takes it: at the least size, thinner with larger hubs, and one hub among low degrees
+HUB_GAMES = [(400000, 1, 500, 2.1), (420001, 1, 300, 2.1), (500009, 1, 9000, 2.6), (400003, 2, 3, 0)]
+
+
+def _hub_game(i):
+    import egsolver_amd as E
+    n, lo, hi, alpha = HUB_GAMES[i]
+    if alpha:
+        return E.generate(E.GenParams(n=n, seed=70 + i, deg_kind=E.games.DEG_POWERLAW, deg_lo=lo, deg_hi=hi, alpha=alpha, wmax=60))
+    rng = np.random.default_rng(70 + i)
+    deg = rng.integers(lo, hi + 1, n)
+    deg[n // 3] = 5000
+    ptr = np.zeros(n + 1, np.int32)
+    ptr[1:] = np.cumsum(deg)
+    succ = rng.integers(0, n, ptr[-1]).astype(np.int32)
+    w = rng.integers(-60, 61, ptr[-1]).astype(np.int32)
+    return E.Game(n=n, n0=n // 2, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(n, ptr, w), ext_of_int=np.arange(n, dtype=np.int32))
+
+
+@pytest.mark.parametrize("i", range(len(HUB_GAMES)))
+def test_hub_games_leave_the_single_launch(i):
+    """Every way out of a single launch for the games that binned rounds would take too, on a
+    solver whose work space still holds a binned game's layout: the round kernels go on without
+    one, before the first round and after it."""
+    import egsolver_amd as E
+    from egsolver_amd import verify
+    g = _hub_game(i)
+    assert g.n + g.m <= 256 * 7168 and 64 < g.max_outdeg
+    other = E.generate(E.GenParams(n=450007, seed=9, deg_kind=E.games.DEG_UNIFORM, deg_lo=2, deg_hi=9, wmax=100))
+    _say(f"hub game n {g.n} m {g.m} maxdeg {g.max_outdeg}")
+    with E.Solver(max(g.n, other.n), max(g.m, other.m)) as s:
+        s.load(g)
+        s.prepare(E.options(slices=1))                       # sweeps in place
+        conv, st0 = s.iterate()
+        assert conv and s.violations() == 0
+        want = s.values()
+        assert want.any()
+        s.load(other)
+        s.prepare()
+        conv, _ = s.iterate()
+        assert conv and s.violations() == 0
+        s.load(g)
+
+        def finish(what):
+            conv, st = s.iterate()
+            vals = s.values()
+            assert conv and np.array_equal(vals, want), (what, np.count_nonzero(vals != want))
+            assert st.initial_active == st0.initial_active, what
+
+        def out_by(what):
+            if what == "stats":
+                s.stats()
+            elif what == "steps":
+                for k in (0, 3, 1):
+                    s.iterate(max_phases=k)
+            elif what == "values":
+                s.set_values(np.zeros(g.n, np.int32))
+            elif what == "transpose":
+                s.csc()
+            elif what == "certificate":
+                s.top_certificate()
+            elif what == "no patience":
+                _zero_wait(s, 0)
+        for what in ("nothing", "stats", "steps", "values", "transpose", "certificate", "no patience"):
+            _say(what)
+            s.prepare()
+            out_by(what)
+            finish(what)
+            _zero_wait(s, 4000)
+        # after the run, and after a capped one
+        s.prepare()
+        finish("run")
+        rep = verify.certify(s, g, want)
+        assert rep["ok"], rep
+        conv, _ = s.iterate()
+        assert conv and np.array_equal(s.values(), want)
+        s.prepare(E.options(max_phases=2))
+        conv, st = s.iterate()
+        assert not conv and st.phases == 2
+        s.csc()
+        conv, _ = s.iterate(max_phases=0)
+        assert not conv and np.all(s.values() <= want)
+
+
+def test_hub_games_on_two_threads():
+    """Two solvers that both ask for the whole device: what the single launches cannot take goes
+    to the round kernels."""
+    import threading
+    import egsolver_amd as E
+    games = [_hub_game(0), _hub_game(1)]
+    want, bad = [], []
+    for g in games:
+        with E.Solver(g.n, g.m) as s:
+            s.load(g)
+            s.prepare(E.options(slices=1))
+            conv, _ = s.iterate()
+            assert conv and s.violations() == 0
+            want.append(s.values())
+    _say("two hub games at once")
+
+    def work(i):
+        with E.Solver(games[i].n, games[i].m) as s:
+            s.load(games[i])
+            for _ in range(6):
+                s.prepare()
+                conv, _ = s.iterate()
+                if not conv or not np.array_equal(s.values(), want[i]):
+                    bad.append(i)
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    assert not bad, bad
