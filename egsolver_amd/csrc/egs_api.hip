@@ -1043,16 +1043,16 @@ static int leave_whole(egs_solver *s) {
 
 // Workgroups of the single launches under way per device.  A launch whose workgroups would not
 // all fit beside those of other solvers is not made (they would wait for each other until
-// their limit); the round kernels take the game.
+// their limit); the round kernels take the game.  A workgroup takes a compute unit: 1,024
+// threads of 87 to 128 registers (egs_whole.hip) leave no room for a second, whatever its LDS.
 struct WholeRoom {
     std::atomic<int> &used;
     int want;
     bool ok;
     WholeRoom(const egs_solver *s) : used(slots()[(unsigned)s->device % 64]), want(0), ok(true) {
         if (s->whole.nb == 1) return;                          // waits for nobody
-        // two workgroups of 1,024 threads share a compute unit when their LDS allows
-        want = s->whole.nb * (egs::whole_lds(s->whole) > 79 * 1024 ? 2 : 1);
-        ok = used.fetch_add(want) + want <= 2 * s->cus;
+        want = s->whole.nb;
+        ok = used.fetch_add(want) + want <= s->cus;
     }
     ~WholeRoom() { used.fetch_sub(want); }
     static std::atomic<int> *slots() {

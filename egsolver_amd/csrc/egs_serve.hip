@@ -268,9 +268,9 @@ int grow_solver(egs_server *s, LargeWorker &wk, int n, int64_t m) {
     while (mc < m) mc *= 2;
     int rc = egs_solver_create(s->device, nc, mc, &wk.solver);
     if (rc) return sfail(rc, "large-route solver: %s", egs_last_error());
-    // two workgroups of a worker's single launches fit a compute unit: the default workers'
-    // launches fit the units a slice leaves to the large route (kLargeCus) together
-    egs::solver_limit_whole(wk.solver, kLargeCus * 2 / std::max(kLargeWorkers, s->large_workers));
+    // a workgroup of a single launch takes a compute unit: the workers' launches fit the units
+    // a slice leaves to the large route (kLargeCus) together
+    egs::solver_limit_whole(wk.solver, kLargeCus / std::max(kLargeWorkers, s->large_workers));
     wk.n = nc;
     wk.m = mc;
     return EGS_OK;

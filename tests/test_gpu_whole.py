@@ -237,7 +237,7 @@ def test_initial_frontier_before_the_first_round(oracle, n):
         assert conv and st.initial_active == act.sum() and s.violations() == 0
 
 
-def _zero_wait(s, us):
+def _patience(s, us):
     from egsolver_amd import _native as N
     fn = N.egs().egs_solver_whole_wait
     fn.argtypes = [ctypes.c_void_p, ctypes.c_int64]
@@ -308,13 +308,13 @@ def test_hub_games_leave_the_single_launch(i):
             elif what == "certificate":
                 s.top_certificate()
             elif what == "no patience":
-                _zero_wait(s, 0)
+                _patience(s, 0)
         for what in ("nothing", "stats", "steps", "values", "transpose", "certificate", "no patience"):
             _say(what)
             s.prepare()
             out_by(what)
             finish(what)
-            _zero_wait(s, 4000)
+            _patience(s, 4000)
         # after the run, and after a capped one
         s.prepare()
         finish("run")
@@ -360,3 +360,40 @@ def test_hub_games_on_two_threads():
     for t in ts:
         t.join()
     assert not bad, bad
+
+
+def test_launches_at_once_are_resident():
+    """Two solvers whose launches together have more workgroups than the device holds, one to a
+    compute unit: the second is not made.  With a second's patience at the barrier, launches
+    that wait for each other would show as a solve of more than a second."""
+    import threading
+    import time
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=200003, seed=31, deg_kind=E.games.DEG_FIXED, deg_lo=8, deg_hi=8, wmax=100))
+    _say("two launches of 256 workgroups")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        want = _rounds(s)
+    bad, longest = [], [0.0, 0.0]
+    start = threading.Barrier(2)
+
+    def work(i):
+        with E.Solver(g.n, g.m) as s:
+            s.load(g)
+            _patience(s, 1000000)
+            start.wait()
+            for _ in range(60):
+                t0 = time.perf_counter()
+                s.prepare()
+                conv, _ = s.iterate()
+                longest[i] = max(longest[i], time.perf_counter() - t0)
+                if not conv or not np.array_equal(s.values(), want):
+                    bad.append(i)
+    ts = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in ts:
+        t.start()
+    for t in ts:
+        t.join()
+    _say(f"longest solves {longest}")
+    assert not bad, bad
+    assert max(longest) < 0.9, longest
