@@ -10,7 +10,6 @@
 #include <string.h>
 
 #include <algorithm>
-#include <atomic>
 #include <chrono>
 
 #include "../../include/egs.h"
@@ -484,6 +483,11 @@ static hipError_t replay_batch(egs_solver *s, int k) {
         }
     }
     return hipGraphLaunch(s->graph[k], s->stream);
+}
+
+egs::DeviceUnits &egs::device_units(int device) {
+    static DeviceUnits units[64];
+    return units[(unsigned)device % 64];
 }
 
 // The large-route workers of a server share the compute units a slice leaves free.
@@ -1041,24 +1045,17 @@ static int leave_whole(egs_solver *s) {
     return EGS_OK;
 }
 
-// Workgroups of the single launches under way per device.  A launch whose workgroups would not
-// all fit beside those of other solvers is not made (they would wait for each other until
-// their limit); the round kernels take the game.  A workgroup takes a compute unit: 1,024
-// threads of 87 to 128 registers (egs_whole.hip) leave no room for a second, whatever its LDS.
+// A single launch whose workgroups would not all fit beside other launches is not made (they
+// would wait for each other until their limit); the round kernels take the game.
 struct WholeRoom {
-    std::atomic<int> &used;
+    egs::DeviceUnits &u;
     int want;
     bool ok;
-    WholeRoom(const egs_solver *s) : used(slots()[(unsigned)s->device % 64]), want(0), ok(true) {
-        if (s->whole.nb == 1) return;                          // waits for nobody
-        want = s->whole.nb;
-        ok = used.fetch_add(want) + want <= s->cus;
+    WholeRoom(const egs_solver *s) : u(egs::device_units(s->device)), want(s->whole.nb > 1 ? egs::units_of(s->whole.nb, s->cus) : 0) {
+        ok = want == 0 ||                                      // one workgroup waits for nobody
+             u.single.fetch_add(want) + want + u.games.load() <= s->cus;
     }
-    ~WholeRoom() { used.fetch_sub(want); }
-    static std::atomic<int> *slots() {
-        static std::atomic<int> u[64];
-        return u;
-    }
+    ~WholeRoom() { u.single.fetch_sub(want); }
 };
 
 // Rounds in single launches until the fixpoint, `limit` more rounds, or a state that the

@@ -264,8 +264,8 @@ int egs_batch_solve(egs_batch *b, const egs_batch_options *o, egs_batch_stats *o
     int lds_ints = o->lds_ints > 0 ? o->lds_ints : 1 << 30;   // default: all the LDS a workgroup may hold
     lds_ints = std::min(lds_ints, (b->lds_limit - 2048) / 4);
     const int per_cu = o->blocks_per_cu > 0 ? o->blocks_per_cu : 1;
-    const int grid = std::max(1, b->cus * per_cu);
     const int ng = (int)b->games.size();
+    const int grid = std::min(std::max(1, b->cus * per_cu), ng);
     std::vector<int> order(ng);
     std::vector<double> cost(ng);
     for (int i = 0; i < ng; i++) {
@@ -283,6 +283,7 @@ int egs_batch_solve(egs_batch *b, const egs_batch_options *o, egs_batch_stats *o
     egs::CertArgs ca{o->certify_every == 0 ? egs::kGameCertifyEvery : (o->certify_every < 0 ? 0 : o->certify_every),
                      o->cert_max_passes > 0 ? o->cert_max_passes : 1024, egs::kGameFirstCap,
                      egs::kGameCandidates};
+    const egs::UnitsHeld held(egs::device_units(b->device).games, egs::units_of(grid, b->cus));
     BHIP(hipEventRecord(b->ev_a, b->stream));
     hipLaunchKernelGGL(egs::k_games, dim3(grid), dim3(threads), sizeof(int) * (size_t)lds_ints, b->stream,
                        (const egs::GameDesc *)b->d_descs, (const int *)b->d_order, ng, b->d_counter, lds_ints,

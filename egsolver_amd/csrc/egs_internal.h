@@ -5,12 +5,34 @@
 #include <limits.h>
 #include <stdint.h>
 
+#include <atomic>
+
 struct egs_solver;
 
 namespace egs {
 
 // Workgroups of a solver's single launches (egs_whole.hip) at most.
 void solver_limit_whole(egs_solver *s, int max_nb);
+
+// Compute units of a device held by this process's launches under way: single launches, whose
+// workgroups wait for one another, and the many-games kernel, whose workgroups stay for long.
+// A workgroup of either takes a unit (1,024 threads of 87 to 128 registers; all of its LDS).
+// A launch's workgroups go to the eight XCDs in turn and stay with their XCD, full or not:
+// every launch holds as many units of each, and the many-games kernel has a workgroup per game
+// at most (with 256 for 100 games the first to come took them, whole XCDs at a time, and a solve
+// beside them waited for their end; 200 games with a workgroup each leave it its 0.6 ms).
+inline int units_of(int workgroups, int cus) { return workgroups > cus ? cus : (workgroups + 7) / 8 * 8; }
+struct DeviceUnits {
+    std::atomic<int> single{0}, games{0};
+};
+DeviceUnits &device_units(int device);
+struct UnitsHeld {
+    std::atomic<int> &held;
+    int n;
+    UnitsHeld(std::atomic<int> &h, int units) : held(h), n(units) { held.fetch_add(n); }
+    ~UnitsHeld() { held.fetch_sub(n); }
+    UnitsHeld(const UnitsHeld &) = delete;
+};
 
 // Frontier lists are split into kSub sub-queues of sub_cap slots plus one overflow region
 // of n slots; a workgroup appends to sub-queue (blockIdx.x % kSub), so no counter sees

@@ -216,6 +216,7 @@ struct egs_server {
     int64_t admitted = 0;     // admissions so far (slot sequence numbers)
     int hi_slot = -1;         // highest slot index ever used (descriptor/state copies cover 0..hi_slot)
     bool slice_kernel = false;  // the running slice launched the many-games kernel
+    int units = 0;              // compute units counted as held by it
     int large_n = 0;          // games with n >= large_n take the device-wide route
     // Large route: persistent worker threads take games from large_queue, solve them on
     // their own solver and stream, and hand them back through large_done.  mu guards
@@ -268,9 +269,9 @@ int grow_solver(egs_server *s, LargeWorker &wk, int n, int64_t m) {
     while (mc < m) mc *= 2;
     int rc = egs_solver_create(s->device, nc, mc, &wk.solver);
     if (rc) return sfail(rc, "large-route solver: %s", egs_last_error());
-    // a workgroup of a single launch takes a compute unit: the workers' launches fit the units
-    // a slice leaves to the large route (kLargeCus) together
-    egs::solver_limit_whole(wk.solver, kLargeCus / std::max(kLargeWorkers, s->large_workers));
+    // a single launch fits the units a slice leaves to the large route; beside another worker's
+    // it is made where both fit (WholeRoom)
+    egs::solver_limit_whole(wk.solver, 2 * kLargeCus / std::max(kLargeWorkers, s->large_workers));
     wk.n = nc;
     wk.m = mc;
     return EGS_OK;
@@ -402,6 +403,11 @@ int submit_large(egs_server *s, int ticket, int32_t n, int32_t n0, int64_t m, in
     return ticket;
 }
 
+void release_units(egs_server *s) {
+    egs::device_units(s->device).games.fetch_sub(s->units);
+    s->units = 0;
+}
+
 // Free the internalisation work space whose kernels have finished.
 void reclaim_transients(egs_server *s) {
     for (size_t i = 0; i < s->transients.size();) {
@@ -524,6 +530,7 @@ int egs_server_destroy(egs_server *s) {
     (void)hipSetDevice(s->device);
     if (s->compute) (void)hipStreamSynchronize(s->compute);
     if (s->copy) (void)hipStreamSynchronize(s->copy);
+    release_units(s);
     stop_workers(s);
     if (s->arena) (void)hipFree(s->arena);
     if (s->d_small) (void)hipFree(s->d_small);
@@ -834,9 +841,15 @@ int egs_server_launch(egs_server *s, const egs_serve_options *o) {
     if (threads != 256 && threads != 512 && threads != 1024) return sfail(EGS_E_ARG, "threads must be 256, 512 or 1024");
     int lds_ints = o->lds_ints > 0 ? o->lds_ints : 1 << 30;   // default: all the LDS a workgroup may hold
     lds_ints = std::min(lds_ints, (s->lds_limit - 2048) / 4);
-    // while large-route games are in flight the slice leaves compute units to their kernels
-    const int free_cus = large_in_flight == 0 ? 0 : o->large_cus < 0 ? 0 : o->large_cus > 0 ? o->large_cus : kLargeCus;
-    const int grid = std::max(1, std::max(1, s->cus - free_cus) * (o->blocks_per_cu > 0 ? o->blocks_per_cu : 1));
+    // while large-route games are in flight the slice leaves compute units to their kernels: as
+    // many as asked for, or as two workers' single launches hold just now
+    egs::DeviceUnits &du = egs::device_units(s->device);
+    int free_cus = 0;
+    if (large_in_flight > 0) {
+        free_cus = o->large_cus < 0 ? 0 : o->large_cus > 0 ? o->large_cus : kLargeCus;
+        free_cus = std::max(free_cus, std::min(du.single.load(), 2 * kLargeCus));
+    }
+    const int grid = std::min((int)s->active.size(), std::max(1, s->cus - free_cus) * (o->blocks_per_cu > 0 ? o->blocks_per_cu : 1));
     const int64_t max_sweeps = o->slice_sweeps > 0 ? o->slice_sweeps : INT64_MAX;
     const int64_t wg_budget = 1000 * (int64_t)(o->slice_kedges > 0 ? o->slice_kedges : kSliceKedges);
     egs::CertArgs ca{o->certify_every == 0 ? egs::kGameCertifyEvery : (o->certify_every < 0 ? 0 : o->certify_every),
@@ -855,6 +868,9 @@ int egs_server_launch(egs_server *s, const egs_serve_options *o) {
     if (any_ro)   // owner counts and MGs of games internalised on the device
         hipLaunchKernelGGL(egs::k_ro_patch_descs, dim3(std::max(1, (s->hi_slot + 256) / 256)), dim3(256), 0,
                            s->compute, s->d_descs, (const egs::ReadOrderMeta *)s->d_meta, s->hi_slot + 1);
+    release_units(s);
+    s->units = egs::units_of(grid, s->cus);
+    du.games.fetch_add(s->units);
     SHIP(hipEventRecord(s->ev_a, s->compute));
     hipLaunchKernelGGL(egs::k_games, dim3(grid), dim3(threads), sizeof(int) * (size_t)lds_ints, s->compute,
                        (const egs::GameDesc *)s->d_descs, (const int *)s->d_order, (int)s->active.size(),
@@ -876,6 +892,7 @@ int egs_server_wait(egs_server *s, int32_t *done, int32_t cap) {
     s->last_slice_ms = 0;
     if (s->slice_kernel) {
         SHIP(hipEventSynchronize(s->ev_slice));
+        release_units(s);
         float ms = 0.f;
         SHIP(hipEventElapsedTime(&ms, s->ev_a, s->ev_slice));
         s->last_slice_ms = ms;

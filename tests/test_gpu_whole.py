@@ -397,3 +397,64 @@ def test_launches_at_once_are_resident():
     _say(f"longest solves {longest}")
     assert not bad, bad
     assert max(longest) < 0.9, longest
+
+
+def _long_batch(count, sweeps):
+    """Games of two vertices, one of which climbs a unit a sweep until it passes MG."""
+    import egsolver_amd as E
+    ptr = np.array([0, 1, 2], np.int32)
+    succ = np.array([0, 0], np.int32)
+    w = np.array([-1, 1 - sweeps], np.int32)
+    g = E.Game(n=2, n0=0, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(2, ptr, w), ext_of_int=np.arange(2, dtype=np.int32))
+    return [g] * count
+
+
+@pytest.mark.parametrize("beside", ["batch", "server"])
+def test_single_launch_beside_many_games(beside):
+    """A launch whose workgroups cannot all run while the many-games kernel holds most compute
+    units is not made: the round kernels solve the game on the units that are left, long before
+    the others are done."""
+    import threading
+    import time
+    import egsolver_amd as E
+    from egsolver_amd.batch import batch_options
+    from egsolver_amd.serve import serve_options
+    g = E.generate(E.GenParams(n=200003, seed=32, deg_kind=E.games.DEG_FIXED, deg_lo=8, deg_hi=8, wmax=100))
+    many = _long_batch(200, 150000)
+    _say(f"a solve beside a {beside} on 200 compute units")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        want = _rounds(s)
+        s.prepare()
+        s.iterate()
+        _patience(s, 1000000)
+        if beside == "batch":
+            b = E.Batch()
+            for x in many:
+                b.add(x)
+            b.upload()
+            t = threading.Thread(target=lambda: b.solve(batch_options(certify_every=-1)))
+            t.start()
+            time.sleep(0.02)
+            running = t.is_alive
+        else:
+            srv = E.Server(64 << 20, max_games=256)
+            for x in many:
+                assert srv.submit(x) is not None
+            srv.launch(serve_options(certify_every=-1))
+            running = lambda: not srv.ready()
+        assert running()
+        t0 = time.perf_counter()
+        s.prepare()
+        conv, _ = s.iterate()
+        took = time.perf_counter() - t0
+        assert running() and took < 0.1, f"the solve waited for the games beside it: {took} s"
+        assert conv and np.array_equal(s.values(), want)
+        if beside == "batch":
+            t.join()
+        else:
+            srv.wait()
+            srv.close()
+        s.prepare()
+        conv, _ = s.iterate()
+        assert conv and np.array_equal(s.values(), want)
