@@ -517,6 +517,12 @@ __global__ __launch_bounds__(256) void k_closure_big(DevGame g, int B, int last,
 // nothing leaves a closed D and a fixpoint on it.  Changed vertices set their bit in `cur`;
 // `clear` (the bitmap of pass p+1, last read in pass p-1) is zeroed.  The pass returns at
 // once when pass p-1 changed nothing or the potentials have passed the divergence bound.
+// flags[1] holds the number of the pass that passed the bound, plus one, and stops the passes
+// after it, not that one: workgroups of the same launch share vertices and must all count in.
+__device__ __forceinline__ bool bf_over(const int *flags, int p) {
+    const int f = flags[1];
+    return f != 0 && f <= p;
+}
 // A pass does nothing when the one before changed nothing, or when it changed so many vertices
 // (at least bin_min, if that is not 0) that the binned kernels take it.
 __device__ __forceinline__ bool bf_idle(int changed, int bin_min) {
@@ -528,7 +534,7 @@ __device__ __forceinline__ void bf_pass_part(const DevGame &g, long long *__rest
                                              const unsigned *__restrict__ prev, unsigned *__restrict__ cur,
                                              unsigned *__restrict__ clear, int p, int *__restrict__ cnt,
                                              int *__restrict__ flags, int bin_min, int bid, int nblk) {
-    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || flags[1]) return;
+    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || bf_over(flags, p)) return;
     const int64_t words = bm_total(g.n);
     for (int64_t i = (int64_t)bid * blockDim.x + threadIdx.x; i < words; i += (int64_t)nblk * blockDim.x)
         clear[i] = 0u;
@@ -636,7 +642,7 @@ __device__ __forceinline__ void bf_pass_part(const DevGame &g, long long *__rest
                 h[v] = best;
                 bm_set(cur, g.n, v);
                 local++;
-                if (best > bound) atomicOr(&flags[1], 1);
+                if (best > bound) atomicMax(&flags[1], p + 1);
             }
         }
     }
@@ -659,7 +665,7 @@ __device__ __forceinline__ void bf_big_part(const DevGame &g, long long *__restr
                                             int *__restrict__ cnt, int *__restrict__ flags, int bin_min, int bid,
                                             int nblk) {
     __shared__ long long sm[4];
-    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || flags[1]) return;
+    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || bf_over(flags, p)) return;
     const long long scale = (long long)g.n + 1;
     const int nb = g.ring[9], items = nb;               // the huge list: k_bf_huge
     int local = 0;
@@ -711,7 +717,7 @@ __device__ __forceinline__ void bf_big_part(const DevGame &g, long long *__restr
                 h[v] = best;
                 bm_set(cur, g.n, v);
                 local++;
-                if (best > bound) atomicOr(&flags[1], 1);
+                if (best > bound) atomicMax(&flags[1], p + 1);
             }
         }
     }
@@ -739,7 +745,7 @@ __device__ __forceinline__ void bf_huge_part(const DevGame &g, long long *__rest
     __shared__ long long sm[4];
     __shared__ long long s_best;
     __shared__ int s_last, s_flag;
-    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || flags[1]) return;
+    if (bf_idle(cnt[(p - 1) % kCntSlots], bin_min) || bf_over(flags, p)) return;
     const int nh = g.ring[10];
     if (nh == 0) return;
     const long long scale = (long long)g.n + 1;
@@ -810,7 +816,7 @@ __device__ __forceinline__ void bf_huge_part(const DevGame &g, long long *__rest
                 h[v] = b;
                 bm_set(cur, g.n, v);
                 local++;
-                if (b > bound) atomicOr(&flags[1], 1);
+                if (b > bound) atomicMax(&flags[1], p + 1);
             }
         }
         __syncthreads();
@@ -930,7 +936,7 @@ __global__ __launch_bounds__(1024) void k_bin_gather_h(DevGame g, const long lon
                                                        const int *__restrict__ cnt, const int *__restrict__ flags,
                                                        int bin_min) {
     extern __shared__ __align__(16) long long hs[];
-    if (cnt[(p - 1) % kCntSlots] < bin_min || flags[1]) return;
+    if (cnt[(p - 1) % kCntSlots] < bin_min || bf_over(flags, p)) return;
     int slice, part;
     bin_place(g, blockIdx.x, slice, part);
     BinWalk walk;
@@ -952,7 +958,7 @@ __global__ __launch_bounds__(256) void k_bin_pass(DevGame g, long long bound, lo
                                                   int *__restrict__ cnt, int *__restrict__ flags, int bin_min) {
     extern __shared__ __align__(16) long long hkey[];
     const int4 desc = g.bdesc[blockIdx.x];
-    if (cnt[(p - 1) % kCntSlots] < bin_min || flags[1]) return;
+    if (cnt[(p - 1) % kCntSlots] < bin_min || bf_over(flags, p)) return;
     const int64_t words = bm_total(g.n);
     for (int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; i < words; i += (int64_t)gridDim.x * blockDim.x)
         clear[i] = 0u;
@@ -977,7 +983,7 @@ __global__ __launch_bounds__(256) void k_bin_pass(DevGame g, long long bound, lo
             removed++;
         } else if (best > hv) {
             h[v] = best;
-            if (best > bound) atomicOr(&flags[1], 1);
+            if (best > bound) atomicMax(&flags[1], p + 1);
         } else {
             continue;
         }
@@ -1124,7 +1130,7 @@ int certify_top(const DevGame &g, const CertBuffers &cb, int wmax, int last, int
     int64_t cands[41];
     int ncand = gap_candidates(cb.pinned, cb.pinned + kBins, wmax, g.mg, cands, std::min(max_cands, 40));
     cands[ncand++] = -1;                    // the vertices that rose in round `last`
-    int *flags = cb.hist + 2 * kBins;       // [0] removed, [1] bound exceeded, [2] unused, [3] members
+    int *flags = cb.hist + 2 * kBins;       // [0] removed, [1] bound exceeded (bf_over), [2] unused, [3] members
     int *fl = cb.pinned + 2 * kBins;        // flags readback (4 ints), then the counter ring
     int *cnt = fl + 4;
     const int64_t words = ((int64_t)g.n + 31) >> 5, bm_len = words + (words + 31) / 32;

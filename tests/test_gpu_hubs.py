@@ -1,5 +1,7 @@
 """Sparse rounds of games with hubs, whose predecessor lists carry the edges' weights: only
 vertices that can rise are queued, and the fixpoint is the oracle's."""
+import ctypes
+
 import numpy as np
 import pytest
 
@@ -60,3 +62,38 @@ def test_one_workgroup_rounds_hand_over(leaves):
         conv, st = s.iterate()
         assert conv and st.phases == 2 * chain + 1
         assert np.array_equal(s.values(), ref)
+
+
+@pytest.mark.parametrize("steps", [600, 1200])
+def test_hub_in_a_candidate_that_diverges(oracle, steps):
+    """Proof passes that pass the divergence bound while several workgroups share a hub: each of
+    them has to finish its part of the pass, or the hub's next lifts fold a part of its edges only.
+
+    A staircase s_t (value t, reached in round t) makes g rise every round; in the proofs g keeps
+    only its positive self-loop and diverges.  The hub follows g, three below it by its last edges."""
+    import egsolver_amd as E
+    from egsolver_amd.games import Game
+    edges = 6000
+    n = steps + 3                                 # hub, g, s_0 .. s_steps
+    hub = np.full(edges, 1, np.int32)
+    hub_w = np.zeros(edges, np.int32)
+    hub_w[-100:] = 3
+    stairs = np.arange(steps + 1, dtype=np.int32) + 2
+    succ = np.concatenate([hub, [1], stairs, [2], stairs[:-1]]).astype(np.int32)
+    w = np.concatenate([hub_w, [3], np.zeros(steps + 1), [0], np.full(steps, -1)]).astype(np.int32)
+    deg = np.concatenate([[edges, steps + 2], np.ones(steps + 1)]).astype(np.int64)
+    ptr = np.concatenate([[0], np.cumsum(deg)]).astype(np.int32)
+    g = Game(n=n, n0=1, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(n, ptr, w), ext_of_int=np.arange(n, dtype=np.int32))
+    ref = np.concatenate([[steps - 3, steps], np.arange(steps + 1)]).astype(np.int32)
+    assert np.array_equal(lfp(oracle, to_oracle_game(g)), ref)
+    stop = ctypes.c_uint32(0)
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        for k in range(6):
+            print(f"[gpu-case] diverging hub, {steps} steps, run {k}", flush=True)
+            # a stop flag keeps the sparse rounds out of one workgroup, where nothing is shared
+            s.prepare(E.options(dense_pct=101, certify_every=2 + k, cert_max_passes=8192, stop_flag=stop))
+            conv, st = s.iterate()
+            assert conv and st.cert_attempts > 5
+            vals = s.values()
+            assert np.array_equal(vals, ref), (k, vals[:2], ref[:2])
