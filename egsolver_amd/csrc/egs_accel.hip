@@ -157,10 +157,11 @@ constexpr int kCntSlots = 64;
 
 constexpr int kBigU = 4;   // edges in flight per lane in the workgroup-per-vertex kernels
 constexpr int kClosureU = 4;   // edges in flight per thread in k_closure (one thread per vertex)
-// A pass is binned after one that changed this part of the vertices.  With hubs, which nearly
-// every change makes k_bf_all read whole, much sooner: on the skewed 2^20 game its passes
-// over the first candidate took 186 us and more at 1/64 changed, 60 us at a few hundred, a
-// binned pass 50 us.
+// The first passes of a candidate are binned while each changes this part of the vertices; the
+// first that does not is followed by sweeping passes to the end, whose counters hold only a
+// flag.  With hubs, which nearly every change makes k_bf_all read whole, the part is much
+// smaller: on the skewed 2^20 game its passes over the first candidate took 186 us and more at
+// 1/64 changed, 60 us at a few hundred, a binned pass 50 us.
 constexpr int kBinPassPart = 64, kBinPassPartHubs = 2048;
 constexpr int kBfU = 2;        // edges in flight per lane in k_bf_pass
 
@@ -523,8 +524,9 @@ __device__ __forceinline__ bool bf_over(const int *flags, int p) {
     const int f = flags[1];
     return f != 0 && f <= p;
 }
-// A pass does nothing when the one before changed nothing, or when it changed so many vertices
-// (at least bin_min, if that is not 0) that the binned kernels take it.
+// A pass does nothing when the one before changed nothing, or when that was a binned pass (or
+// the closure check) that changed at least bin_min vertices, if bin_min is not 0: the binned
+// kernels go on.
 __device__ __forceinline__ bool bf_idle(int changed, int bin_min) {
     return changed == 0 || (bin_min && changed >= bin_min);
 }
@@ -1185,25 +1187,26 @@ int certify_top(const DevGame &g, const CertBuffers &cb, int wmax, int last, int
                                cb.bfcnt, flags, kBigGrid, 2 * kBigGrid);
         int queued = 1;                     // passes queued so far: pass 0 is the closure's
         int passes = 0;
+        int from = bin_min;                 // 0 once the binned passes are over
         bool converged = false, diverged = false, rejected = false;
         while (!converged && !diverged && !rejected && passes < cap) {
             if (stop && *stop) return 0;    // abandon the candidate: nothing was marked
             const int upto = std::min(cap, queued == 1 ? first_chunk : queued + chunk);
             for (int p = queued; p < upto; p++) {
-                if (bin_min) {
+                if (from) {
                     hipLaunchKernelGGL(k_bin_gather_h, dim3(g.bins * h_parts), dim3(1024),
                                        (size_t)g.bin_w * sizeof(long long), st, g, (const long long *)cb.h, h_parts, p,
-                                       (const int *)cb.bfcnt, (const int *)flags, bin_min);
+                                       (const int *)cb.bfcnt, (const int *)flags, from);
                     hipLaunchKernelGGL(k_bin_pass, dim3(g.nchunks), dim3(256), bin_key_slots(g) * sizeof(long long), st,
-                                       g, bound, cb.h, bm[p % 3], bm[(p + 1) % 3], p, cb.bfcnt, flags, bin_min);
+                                       g, bound, cb.h, bm[p % 3], bm[(p + 1) % 3], p, cb.bfcnt, flags, from);
                 }
                 // with vertices above big_deg, their parts of the pass run in the same launch
                 if (has_big)
                     launch_bf_all(G, bf_grid, kBigGrid, 2 * kBigGrid, st, g, cb.h, bound, bm[(p - 1) % 3], bm[p % 3],
-                                  bm[(p + 1) % 3], p, cb.bfcnt, flags, bin_min);
+                                  bm[(p + 1) % 3], p, cb.bfcnt, flags, from);
                 else
                     launch_bf_pass(G, bf_grid, st, g, cb.h, bound, bm[(p - 1) % 3], bm[p % 3], bm[(p + 1) % 3], p,
-                                   cb.bfcnt, flags, bin_min);
+                                   cb.bfcnt, flags, from);
             }
             if (hipMemcpyAsync(fl, flags, sizeof(int) * 4, hipMemcpyDeviceToHost, st) != hipSuccess) return -1;
             if (hipMemcpyAsync(cnt, cb.bfcnt, sizeof(int) * kCntSlots, hipMemcpyDeviceToHost, st) != hipSuccess)
@@ -1215,6 +1218,7 @@ int certify_top(const DevGame &g, const CertBuffers &cb, int wmax, int last, int
                 passes = p + 1;
                 if (cnt[p % kCntSlots] == 0) { converged = true; res.last_passes = passes; break; }
             }
+            if (cnt[(upto - 1) % kCntSlots] < from) from = 0;
             queued = upto;
         }
         if (rejected) continue;
