@@ -230,3 +230,33 @@ def test_batch_thresholds_near_top(oracle, room):
         b.upload()
         st = b.solve(E.batch_options(max_sweeps=20000))
         assert st["converged"] == 1 and np.array_equal(b.values(0), ref)
+
+
+@pytest.mark.parametrize("n,X", [(400, 1000000), (45000, 1000)])
+def test_proof_that_only_the_full_scale_finds(n, X):
+    """A ring of 300 vertices that player 1 wins by one unit a turn, fed from high values: a proof
+    at a scale below 300 raises its potentials for ever, one at n + 1 ends.  Potentials of 32 and
+    16 bits in the values' place; the sweeps are capped, since lifting alone climbs for hours."""
+    import egsolver_amd as E
+    from egsolver_amd.batch import batch_options
+    k, L, extra = 5, 300, 10
+    ring = 1 + k
+    lists = [[(0, 0)]] + [[(i - 1, -X)] for i in range(1, ring)]
+    lists += [[(ring + L - 1, -1), (k, 0)]] + [[(ring + j - 1, 0)] for j in range(1, L)]
+    lists += [[(0, -X)]] * extra
+    lists += [[(v, 0)] for v in range(len(lists), n)]
+    ptr = np.concatenate([[0], np.cumsum([len(x) for x in lists])]).astype(np.int32)
+    succ = np.array([e[0] for x in lists for e in x], np.int32)
+    w = np.array([e[1] for x in lists for e in x], np.int32)
+    g = E.Game(n=n, n0=0, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(n, ptr, w), ext_of_int=np.arange(n, dtype=np.int32))
+    want = np.zeros(n, np.int32)
+    want[:ring] = X * np.arange(ring)
+    want[ring:ring + L] = 2147483647
+    want[ring + L:ring + L + extra] = X
+    with E.Batch() as b:
+        b.add(g)
+        b.upload()
+        print(f"[gpu-case] ring of {L} in {n}", flush=True)
+        st = b.solve(batch_options(max_sweeps=5000))
+        assert st["converged"] == 1 and st["certificates"] == 1, st
+        assert np.array_equal(b.values(0), want)
