@@ -1388,12 +1388,20 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
 
 int egs_solver_stats(egs_solver *s, egs_stats *st) {
     if (!s || !st) return fail(EGS_E_ARG, "null argument");
-    // asked between prepare and the first round: the initial frontier has not been made where
-    // the first launch of the run would make it
+    // asked between prepare and the first round, where the first launch of the run would make the
+    // initial frontier: it is counted here (with every value 0 the vertices that a lift changes)
+    // and the run left as it is
     const bool unborn = s->prepared && (s->bins_open || (s->whole.nb > 0 && s->whole_rounds == 0 && !s->st.converged));
     if (unborn) {
         HIP_TRY(hipSetDevice(s->device));
-        if (int rc = leave_whole(s)) return rc;
+        double t0 = 0;
+        float ms = 0.f;
+        int64_t active = 0;
+        HIP_TRY(mark_start(s, &t0));
+        if (int rc = egs_solver_count_violations(s, &active)) return rc;
+        HIP_TRY(mark_stop(s, t0, &ms));
+        s->st.initial_active = (int32_t)active;
+        s->st.ms_prepare = ms;
     }
     HIP_TRY(close_prepare(s));
     *st = s->st;

@@ -1,6 +1,7 @@
 """Whole solves in one launch (egs_whole.hip): exact against the oracle or the round kernels
 at the sizes where its forms begin and end, and the hand-over to the round kernels."""
 import ctypes
+import zlib
 
 import numpy as np
 import pytest
@@ -458,3 +459,23 @@ def test_single_launch_beside_many_games(beside):
         s.prepare()
         conv, _ = s.iterate()
         assert conv and np.array_equal(s.values(), want)
+
+
+@pytest.mark.parametrize("n,hi", [(20011, 16), (87148, 16), (450011, 9)])
+def test_statistics_leave_the_run_alone(n, hi):
+    """Statistics asked for before the first round do not change what runs it: the synchronous
+    rounds of a single launch, or of a binned game, count the same lifts as without the question."""
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=n, seed=14, deg_kind=E.games.DEG_UNIFORM, deg_lo=2, deg_hi=hi, wmax=100))
+    _say(f"statistics of {n}")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        seen = []
+        for ask in (False, True, True):
+            s.prepare(E.options(certify_every=-1, max_phases=30))
+            if ask:
+                st = s.stats()
+                assert st.phases == 0 and st.initial_active == seen[0][0] and not s.values().any()
+            _, st = s.iterate()
+            seen.append((st.initial_active, st.phases, st.edges_relaxed, st.lifted, zlib.crc32(s.values())))
+        assert seen[0] == seen[1] == seen[2]
