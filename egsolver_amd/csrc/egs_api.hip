@@ -1229,7 +1229,7 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
     }
     int64_t launched = 0;
     if (s->bins_open) {
-        const bool first = limit > 0;
+        const bool first = limit > 0 && !(s->stop_flag && *s->stop_flag);
         const int rc = prepare_rounds(s, first);
         if (rc) return rc;
         if (first) {

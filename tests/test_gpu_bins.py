@@ -178,3 +178,22 @@ def test_no_initial_lift():
         conv, st = s.iterate()
         assert conv and st.phases == 0 and st.initial_active == 0
         assert not s.values().any() and s.violations() == 0
+
+
+def test_stop_flag_before_the_first_round():
+    """A run stopped before it begins does no round, the one done with the layout included; with
+    the flag cleared it goes on to the fixpoint."""
+    import egsolver_amd as E
+    g = _generate(410009, 1, 2, 8, 0, 100, 9)
+    _say("stopped before the first round")
+    stop = ctypes.c_uint32(1)
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        want = _sweeps(s)
+        s.prepare(E.options(stop_flag=stop))
+        conv, st = s.iterate()
+        assert not conv and st.phases == 0 and st.lifted == 0 and st.initial_active > 0
+        assert not s.values().any()
+        stop.value = 0
+        conv, st = s.iterate()
+        assert conv and np.array_equal(s.values(), want)
