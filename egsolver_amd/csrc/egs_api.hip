@@ -1213,7 +1213,8 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
     if (s->next_round + limit > 0x7ffffff0LL) limit = 0x7ffffff0LL - s->next_round;
     if (s->whole.nb > 0) {
         int status = egs::kWholeNone, rc = EGS_OK;
-        if (max_phases < 0 && !s->st.converged) {
+        // (no launch where no round is allowed: the round kernels' set-up tells the frontier's size)
+        if (max_phases < 0 && !s->st.converged && (limit > 0 || s->whole_rounds > 0)) {
             const int64_t before = s->whole_rounds;
             rc = run_whole(s, limit, &status);
             if (rc) return rc;

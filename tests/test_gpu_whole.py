@@ -479,3 +479,26 @@ def test_statistics_leave_the_run_alone(n, hi):
             _, st = s.iterate()
             seen.append((st.initial_active, st.phases, st.edges_relaxed, st.lifted, zlib.crc32(s.values())))
         assert seen[0] == seen[1] == seen[2]
+
+
+@pytest.mark.parametrize("n", [61, 5000, 20011])
+@pytest.mark.parametrize("negative", [True, False])
+def test_no_round_allowed(n, negative):
+    """A round cap of 0: the statistics still hold the initial frontier, and a game in which
+    nothing is active has converged."""
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=n, seed=4, deg_kind=E.games.DEG_UNIFORM, deg_lo=2, deg_hi=3, wmax=50))
+    w = g.w if negative else np.abs(g.w)
+    g = E.Game(n=n, n0=g.n0, ptr=g.ptr, succ=g.succ, w=w, mg=E.games.compute_mg(n, g.ptr, w), ext_of_int=g.ext_of_int)
+    neg = (w < 0).astype(np.int64)
+    cnt, deg = np.add.reduceat(neg, g.ptr[:-1]), np.diff(g.ptr)
+    act = np.where(np.arange(n) < g.n0, cnt == deg, cnt > 0)
+    _say(f"no round, n {n}")
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        s.prepare(E.options(max_phases=0))
+        for _ in range(2):
+            conv, st = s.iterate()
+            assert conv == (not negative) == bool(st.converged)
+            assert st.phases == 0 and st.initial_active == act.sum()
+            assert not s.values().any()
