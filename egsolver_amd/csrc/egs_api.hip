@@ -173,10 +173,13 @@ constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
     L.slen = L.phased ? take(ptiles * egs::kMaxPhases * egs::kSliceTile) : 0;
     L.sbase = L.phased ? take(4 * ptiles * egs::kMaxPhases * egs::kSliceWaves) : 0;
     L.sedges = L.phased ? take(8 * m) : 0;
-    // binned dense rounds: words, vertex numbers and candidates of the padded edges
+    // binned dense rounds: words, vertex numbers and candidates of the padded edges, in whole
+    // cache lines (the vertex numbers follow the words and are read four at a time) and with
+    // room for a step past the last index in 31 bits
     L.binned = n_cap >= egs::kBinMinN;
     L.bin_cap = L.binned ? m_cap + m_cap / 2 + (1 << 20) : 0;
-    if (L.bin_cap > 0x7fffffff) L.bin_cap = 0x7fffffff;
+    if (L.bin_cap > 0x7fff0000) L.bin_cap = 0x7fff0000;
+    L.bin_cap &= ~(int64_t)63;
     L.bedges = L.binned ? take(6 * (size_t)L.bin_cap + 256) : 0;
     L.bcand = L.binned ? take(8 * (size_t)L.bin_cap) : 0;
     L.cweight = L.binned ? L.bcand : take(4 * m);      // a game leaves the bins with its transpose
@@ -190,6 +193,8 @@ constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
     L.total = off;
     return L;
 }
+static_assert(make_layout(egs::kBinMinN, 2000001).bin_cap % 64 == 0 && make_layout(1 << 23, 0x7fffffff).bin_cap % 64 == 0,
+              "vertex numbers behind the words are aligned at every capacity");
 
 }  // namespace
 

@@ -197,3 +197,17 @@ def test_stop_flag_before_the_first_round():
         stop.value = 0
         conv, st = s.iterate()
         assert conv and np.array_equal(s.values(), want)
+
+
+@pytest.mark.parametrize("extra", [0, 1, 2, 3])
+def test_any_edge_capacity(extra):
+    """The vertex numbers lie behind the packed words, whose room follows from the capacity."""
+    import egsolver_amd as E
+    g = _generate(400013, 1, 2, 8, 0, 100, 12)
+    _say(f"capacity m + {extra}")
+    with E.Solver(g.n, g.m + extra) as s:
+        s.load(g)
+        want = _sweeps(s)
+        s.prepare()
+        conv, _ = s.iterate()
+        assert conv and np.array_equal(s.values(), want)
