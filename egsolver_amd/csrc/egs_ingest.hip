@@ -80,8 +80,9 @@ __global__ __launch_bounds__(256) void k_rd_rows(const int *__restrict__ rptr, c
         if (t == 0) s_row[rows] = rptr[r0 + rows];
         s_worst[t] = 0;
         __syncthreads();
-        const int e1 = s_row[rows];
-        for (int e = s_row[0] + t; e < e1; e += 256) {
+        const unsigned e1 = (unsigned)s_row[rows];
+        for (unsigned at = (unsigned)s_row[0] + t; at < e1; at += 256) {   // past 2^31 in the last step
+            const int e = (int)at;
             int lo = 0, hi = rows;                   // largest row starting at or before e
             while (hi - lo > 1) {
                 const int mid = (lo + hi) >> 1;
