@@ -650,8 +650,10 @@ int egs_solver_load(egs_solver *s, int mem, int32_t n, int32_t n0, int64_t m, in
         }
         s->max_outdeg = mx;
         s->wmax = wm;
-        hipError_t e1 = hipMemcpy(s->d_ptr, ptr, sizeof(int) * ((size_t)n + 1), hipMemcpyHostToDevice);
-        hipError_t e2 = hipMemcpy(s->d_edges, packed, sizeof(int2) * (size_t)m, hipMemcpyHostToDevice);
+        // what a prepare of the game before has queued still reads the arrays
+        const hipError_t e0 = hipStreamSynchronize(s->stream);
+        hipError_t e1 = e0 != hipSuccess ? e0 : hipMemcpy(s->d_ptr, ptr, sizeof(int) * ((size_t)n + 1), hipMemcpyHostToDevice);
+        hipError_t e2 = e1 != hipSuccess ? e1 : hipMemcpy(s->d_edges, packed, sizeof(int2) * (size_t)m, hipMemcpyHostToDevice);
         free(packed);
         HIP_TRY(e1);
         HIP_TRY(e2);

@@ -90,3 +90,24 @@ def test_device_load_equals_host_load(n, hi):
             conv, _ = x.iterate()
             assert conv
         assert np.array_equal(s.values(), ref.values())
+
+
+def test_load_behind_a_queued_prepare():
+    """A game loaded from the host while the prepare of the one before is still queued."""
+    import egsolver_amd as E
+    big = E.generate(E.GenParams(n=1300000, seed=5, deg_kind=E.games.DEG_UNIFORM, deg_lo=2, deg_hi=4, wmax=50))
+    games = [E.generate(E.GenParams(n=n, seed=6, deg_kind=E.games.DEG_UNIFORM, deg_lo=2, deg_hi=9, wmax=50)) for n in (900, 450019)]
+    print("[gpu-case] load behind a queued prepare", flush=True)
+    with E.Solver(big.n, max(big.m, games[1].m)) as s:
+        for g in games:
+            s.load(big)
+            s.prepare(E.options(slices=4))
+            s.prepare()
+            s.load(g)
+            s.prepare()
+            conv, _ = s.iterate()
+            assert conv and s.violations() == 0
+            vals = s.values()
+            s.prepare(E.options(slices=1, group=2))
+            conv, _ = s.iterate()
+            assert conv and np.array_equal(s.values(), vals)
