@@ -110,12 +110,13 @@ struct Layout {
         titems, slen, sbase, sedges, bigmask, bedges, bcand, boff, bchunk, bdesc, whole, total;
     int64_t tcounts_cap, bin_cap, boff_cap;
     int sub_cap;
-    bool phased, binned;
+    bool phased, binned, weights;
 };
 
 constexpr size_t align256c(size_t x) { return (x + 255) & ~(size_t)255; }
 
-constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
+// lean: without the arrays that only make rounds faster (the binned layout, the transpose's weights).
+constexpr Layout make_layout(int32_t n_cap, int64_t m_cap, bool lean = false) {
     Layout L{};
     const size_t n1 = (size_t)n_cap + 1, m = (size_t)m_cap;
     const size_t tiles = (size_t)(n_cap + 4095) / 4096 + 1;
@@ -176,13 +177,14 @@ constexpr Layout make_layout(int32_t n_cap, int64_t m_cap) {
     // binned dense rounds: words, vertex numbers and candidates of the padded edges, in whole
     // cache lines (the vertex numbers follow the words and are read four at a time) and with
     // room for a step past the last index in 31 bits
-    L.binned = n_cap >= egs::kBinMinN;
+    L.binned = n_cap >= egs::kBinMinN && !lean;
     L.bin_cap = L.binned ? m_cap + m_cap / 2 + (1 << 20) : 0;
     if (L.bin_cap > 0x7fff0000) L.bin_cap = 0x7fff0000;
     L.bin_cap &= ~(int64_t)63;
     L.bedges = L.binned ? take(6 * (size_t)L.bin_cap + 256) : 0;
     L.bcand = L.binned ? take(8 * (size_t)L.bin_cap) : 0;
-    L.cweight = L.binned ? L.bcand : take(4 * m);      // a game leaves the bins with its transpose
+    L.weights = !lean;
+    L.cweight = L.binned ? L.bcand : L.weights ? take(4 * m) : 0;   // a game leaves the bins with its transpose
     const size_t chunks = ((size_t)egs::kBinHead * n1 + m) / egs::kBinShareMin + 2;
     L.boff_cap = L.binned ? (int64_t)((size_t)L.bin_cap / egs::kBinPad + chunks) : 0;
     L.boff = L.binned ? take(4 * (size_t)L.boff_cap) : 0;
@@ -281,7 +283,7 @@ static void bind_layout(egs_solver *s, char *b, const Layout &L) {
     s->d_edges = (int2 *)(b + L.edges);
     s->d_cptr = (int *)(b + L.cptr);
     s->d_cpred = (int *)(b + L.cpred);
-    s->d_cweight = (int *)(b + L.cweight);
+    s->d_cweight = L.weights ? (int *)(b + L.cweight) : nullptr;
     s->d_val = (int *)(b + L.val);
     s->d_stamp = (int *)(b + L.stamp);
     s->d_list[0] = (int *)(b + L.l0);
@@ -593,9 +595,15 @@ int egs_solver_create(int device, int32_t n_cap, int64_t m_cap, egs_solver **out
     s->whole_max_nb = s->cus;
     s->n_cap = n_cap;
     s->m_cap = m_cap;
-    const Layout L = make_layout(n_cap, m_cap);
-    s->block_bytes = L.total;
+    Layout L = make_layout(n_cap, m_cap);
     if (hipMalloc(&s->block, L.total) != hipSuccess) {
+        // 28 bytes an edge where there is no room for 49 (32 below kBinMinN vertices)
+        (void)hipGetLastError();
+        L = make_layout(n_cap, m_cap, true);
+        s->block = nullptr;
+    }
+    s->block_bytes = L.total;
+    if (!s->block && hipMalloc(&s->block, L.total) != hipSuccess) {
         egs_solver_destroy(s);
         return fail(EGS_E_NOMEM, "hipMalloc of %zu bytes failed", L.total);
     }

@@ -211,3 +211,38 @@ def test_any_edge_capacity(extra):
         s.prepare()
         conv, _ = s.iterate()
         assert conv and np.array_equal(s.values(), want)
+
+
+def test_solver_where_memory_is_short():
+    """A solver whose full work space does not fit the free memory goes without the binned layout
+    and the transpose's weights, and solves large uniform and skewed games all the same."""
+    import torch
+    import egsolver_amd as E
+    games = [_generate(430007, 1, 2, 8, 0, 100, 9), _generate(450007, 2, 1, 50000, 2.1, 100, 63)]
+    n_cap, m_cap = 1 << 20, 1 << 29
+    want = []
+    for g in games:
+        with E.Solver(g.n, g.m) as s:
+            s.load(g)
+            want.append(_sweeps(s))
+    torch.cuda.empty_cache()
+    free0 = torch.cuda.mem_get_info()[0]
+    with E.Solver(n_cap, m_cap):
+        full = free0 - torch.cuda.mem_get_info()[0]
+    assert full > 40 * m_cap
+    left = int(0.75 * full)
+    _say(f"full {full >> 20} MiB, left {left >> 20} MiB")
+    held, step = [], 32 << 30
+    try:
+        while (over := torch.cuda.mem_get_info()[0] - left) > 1 << 20:
+            held.append(torch.empty(min(step, over), dtype=torch.uint8, device="cuda"))
+        with E.Solver(n_cap, m_cap) as s:
+            for g, w in zip(games, want):
+                s.load(g)
+                for opt in ({}, {"dense_pct": 60}):
+                    s.prepare(E.options(**opt))
+                    conv, _ = s.iterate()
+                    assert conv and np.array_equal(s.values(), w)
+    finally:
+        held.clear()
+        torch.cuda.empty_cache()
