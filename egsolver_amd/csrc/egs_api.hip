@@ -239,6 +239,7 @@ struct egs_solver {
     int whole_max_nb = 0;             // workgroups of such a launch at most
     int64_t whole_wait = egs::kWholeWait;
     int64_t whole_rounds = 0;         // rounds of the run they have done
+    bool whole_gave_up = false;       // the last of them gave up: the values are past those rounds
     egs_stats whole_st{};             // what those rounds counted
     int wmax = 0;
     int cert_every = 32, cert_gap = 32, cert_max_passes = 1024;
@@ -271,6 +272,7 @@ struct egs_solver {
     int max_outdeg = 0;
     int64_t next_round = 1;
     int64_t phase_cap = 0;
+    bool capped = false;              // by the options, not by the reference's bound
     int batch_rounds = 32;
     const volatile uint32_t *stop_flag = nullptr;
     egs_stats st{};
@@ -909,6 +911,7 @@ static int pick_shape(egs_solver *s, const egs_options *o, bool whole) {
     if (o->graphs < -1 || o->graphs > 1) return fail(EGS_E_ARG, "graphs must be -1, 0 or 1 (got %d)", o->graphs);
     s->use_graphs = o->graphs > 0 && !o->stop_flag && !s->no_alloc;
     s->phase_cap = egs_max_loop_c(g.m, g.n, g.mg, o->max_phases);
+    s->capped = o->max_phases >= 0;
     s->stop_flag = o->stop_flag;
     s->cert_every = o->certify_every == 0 ? kCertEvery : (o->certify_every < 0 ? 0 : o->certify_every);
     s->cert_max_passes = o->cert_max_passes > 0 ? o->cert_max_passes : 1024;
@@ -1044,6 +1047,16 @@ static bool takes_whole(const egs_options *o) {
                   o->dense_pct == 0 && o->slices == 0 && o->phase_wgs_per_cu == 0 && o->graphs == 0 && !o->stop_flag);
 }
 
+// Vertices of g with lift(val)(v) != val(v).
+static int count_violations(egs_solver *s, const egs::DevGame &g, int64_t *violations) {
+    HIP_TRY(egs::launch_violations(g, (unsigned long long *)s->d_misc, s->stream));
+    unsigned long long *h = (unsigned long long *)(s->h_probe + kPinViol);
+    HIP_TRY(hipMemcpyAsync(h, s->d_misc, sizeof(unsigned long long), hipMemcpyDeviceToHost, s->stream));
+    HIP_TRY(hipStreamSynchronize(s->stream));
+    *violations = (int64_t)*h;
+    return EGS_OK;
+}
+
 // Hand a run over from single launches to the round kernels: their whole set-up when it has
 // not begun, else the counters and lists, with the values reached and the next round a full
 // sweep (none when the run has converged).
@@ -1052,11 +1065,20 @@ static int leave_whole(egs_solver *s) {
     if (s->bins_open) return prepare_rounds(s);
     if (s->whole.nb == 0) return EGS_OK;
     s->whole.nb = 0;
-    if (s->whole_rounds == 0 && !s->st.converged) return prepare_rounds(s);
+    const bool reached = s->whole_gave_up && !s->capped;
+    if (s->whole_rounds == 0 && !s->st.converged && !reached) return prepare_rounds(s);
     HIP_TRY(egs::launch_prepare_reset(s->g, s->stream));
     if (s->sh.use_block) HIP_TRY(egs::launch_hbest_reset(s->g, s->stream));
     HIP_TRY(egs::launch_classify(s->g, s->d_ring + 9, s->stream));
     HIP_TRY(egs::launch_resume(s->g, (int)s->next_round, s->st.converged != 0, s->stream));
+    if (s->whole_rounds == 0 && !s->st.converged) {
+        // the initial frontier: the vertices that a lift of zeros changes (the stamps are zeros now)
+        egs::DevGame zero = s->g;
+        zero.val = s->d_stamp;
+        int64_t active = 0;
+        if (int rc = count_violations(s, zero, &active)) return rc;
+        s->st.initial_active = (int32_t)active;
+    }
     return EGS_OK;
 }
 
@@ -1129,6 +1151,7 @@ static int run_whole(egs_solver *s, int64_t limit, int *status) {
         }
         if (!got) {
             *status = egs::kWholeNone;
+            s->whole_gave_up = true;
             break;
         }
         const int64_t ran = res->rounds - s->whole_rounds;
@@ -1178,6 +1201,7 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     s->cert_cap = std::min(kCertFirstCap, s->cert_max_passes);
     s->cert_pass_hint = 0;
     s->whole_rounds = 0;
+    s->whole_gave_up = false;
     s->whole_st = egs_stats{};
     s->mirrored = false;
     s->bins_open = false;
@@ -1464,12 +1488,7 @@ int egs_solver_read_csc(egs_solver *s, int32_t *cptr, int32_t *cpred) {
 int egs_solver_count_violations(egs_solver *s, int64_t *violations) {
     if (!s || !s->loaded || !violations) return fail(EGS_E_STATE, "egs_solver_count_violations: nothing loaded");
     HIP_TRY(hipSetDevice(s->device));
-    HIP_TRY(egs::launch_violations(s->g, (unsigned long long *)s->d_misc, s->stream));
-    unsigned long long *h = (unsigned long long *)(s->h_probe + kPinViol);
-    HIP_TRY(hipMemcpyAsync(h, s->d_misc, sizeof(unsigned long long), hipMemcpyDeviceToHost, s->stream));
-    HIP_TRY(hipStreamSynchronize(s->stream));
-    *violations = (int64_t)*h;
-    return EGS_OK;
+    return count_violations(s, s->g, violations);
 }
 
 int egs_solver_set_values(egs_solver *s, const int32_t *host_values) {

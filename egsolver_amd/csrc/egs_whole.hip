@@ -25,7 +25,8 @@
 // The barrier needs every workgroup resident.  A workgroup that waits past its limit raises
 // the abort flag and leaves; the others see the flag in their own waits and leave too, and
 // the host goes on with the round kernels from the values reached (any prefix of the rounds
-// is a valid start of theirs, and so is a partly marked proven set).
+// is a valid start of theirs, and so is a partly marked proven set; only a run with a round cap
+// begins again, since the rounds of a launch that gave up are not counted).
 #include <climits>
 
 #include "egs_device.h"
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
             for (int spin = 1; x == 0; spin++) {
                 __builtin_amdgcn_s_sleep(1);
                 x = ctl_load(p);
-                if ((spin & 63) == 0 && x == 0) {
+                if (((spin & 63) == 0 || a.wait == 0) && x == 0) {
                     const bool late = wall_clock64() - t0 > a.wait;
                     if (late) ctl_store(&a.ctl->abort_flag, 1);
                     if (late || ctl_load(&a.ctl->abort_flag)) {

@@ -502,3 +502,26 @@ def test_no_round_allowed(n, negative):
             assert conv == (not negative) == bool(st.converged)
             assert st.phases == 0 and st.initial_active == act.sum()
             assert not s.values().any()
+
+
+@pytest.mark.parametrize("n", [20000, 150000])
+def test_values_reached_by_a_launch_that_gives_up(n):
+    """Every vertex but the sink rises once, in the first round: a launch that gives up after it
+    leaves nothing to lift.  A run with a round cap begins again: its rounds are counted."""
+    import egsolver_amd as E
+    succ = np.zeros(n, np.int32)
+    w = np.full(n, -5, np.int32)
+    w[0] = 0
+    ptr = np.arange(n + 1, dtype=np.int32)
+    g = E.Game(n=n, n0=0, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(n, ptr, w), ext_of_int=np.arange(n, dtype=np.int32))
+    want = np.full(n, 5, np.int32)
+    want[0] = 0
+    _say(f"values reached, n {n}")
+    with E.Solver(n, n) as s:
+        s.load(g)
+        for patience, cap, lifted in ((4000, -1, n - 1), (0, -1, 0), (0, 50, n - 1)):
+            _patience(s, patience)
+            s.prepare(E.options(max_phases=cap))
+            conv, st = s.iterate()
+            assert conv and np.array_equal(s.values(), want)
+            assert st.lifted == lifted and st.initial_active == n - 1, st.as_dict()
