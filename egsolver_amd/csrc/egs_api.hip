@@ -254,6 +254,7 @@ struct egs_solver {
     char *h_out = nullptr;    // pinned, 2 x out_half bytes, made at the first larger read-back
     size_t out_half = 0;
     bool mirrored = false;    // h_small holds the values of the run that has just converged
+    bool values_out = false;  // their device address was handed out: read-backs go to the device
     int probe_want[2] = {kProbeWant, kProbeWant};   // where each probe slot holds ring[13]
     hipEvent_t ev_probe[2] = {nullptr, nullptr};
     hipEvent_t ev_a = nullptr, ev_b = nullptr;
@@ -1125,7 +1126,7 @@ static int run_whole(egs_solver *s, int64_t limit, int *status) {
     // no-allocation solver has none and copies it from device memory
     egs::WholeResult *res = (egs::WholeResult *)(s->h_probe + kPinWhole);
     // one workgroup stores its values into the small read-back area on its way out
-    a.mirror = s->whole.nb == 1 && 4 * (size_t)g.n <= s->out_small ? (int *)s->h_small : nullptr;
+    a.mirror = s->whole.nb == 1 && !s->values_out && 4 * (size_t)g.n <= s->out_small ? (int *)s->h_small : nullptr;
     a.out = s->no_alloc ? (egs::WholeResult *)s->d_misc : res;
     *status = egs::kWholeNone;
     WholeRoom room(s);
@@ -1470,7 +1471,12 @@ int egs_solver_read_winning(egs_solver *s, uint32_t *host_bits) {
     return EGS_OK;
 }
 
-const int32_t *egs_solver_device_values(egs_solver *s) { return s ? s->d_val : nullptr; }
+const int32_t *egs_solver_device_values(egs_solver *s) {
+    if (!s) return nullptr;
+    s->values_out = true;
+    s->mirrored = false;
+    return s->d_val;
+}
 
 void *egs_solver_stream(egs_solver *s) { return s ? (void *)s->stream : nullptr; }
 

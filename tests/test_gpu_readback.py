@@ -37,3 +37,31 @@ def test_values_equal_device_values(n):
         assert np.array_equal(s.values(), pattern)
         s.prepare(E.options(max_phases=6))
         assert not s.values().any()
+
+
+@pytest.mark.parametrize("n", [5, 2000, 5999])
+@pytest.mark.parametrize("ask", ["before", "after"])
+def test_values_written_by_address(n, ask):
+    """Values changed through the device address are what a read-back returns."""
+    import torch
+    import egsolver_amd as E
+    from egsolver_amd import _native as N
+
+    class View:
+        def __init__(self, address):
+            self.__cuda_array_interface__ = {"shape": (n,), "typestr": "<i4", "strides": None, "data": (int(address), False),
+                                             "version": 2}
+    g = _ring(n)
+    print(f"[gpu-case] values by address, n {n}", flush=True)
+    with E.Solver(n, g.m) as s:
+        s.load(g)
+        if ask == "before":
+            t = torch.as_tensor(View(N.egs().egs_solver_device_values(s.h)), device="cuda")
+        s.prepare()
+        s.iterate()
+        if ask == "after":
+            t = torch.as_tensor(View(N.egs().egs_solver_device_values(s.h)), device="cuda")
+        pattern = torch.arange(n, dtype=torch.int32, device="cuda") * 3 + 1
+        t.copy_(pattern)
+        torch.cuda.synchronize()
+        assert np.array_equal(s.values(), pattern.cpu().numpy())
