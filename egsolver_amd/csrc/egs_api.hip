@@ -254,6 +254,7 @@ struct egs_solver {
     char *h_out = nullptr;    // pinned, 2 x out_half bytes, made at the first larger read-back
     size_t out_half = 0;
     bool mirrored = false;    // h_small holds the values of the run that has just converged
+    bool values_set = false;  // the run's values were replaced (egs_solver_set_values)
     bool values_out = false;  // their device address was handed out: read-backs go to the device
     int probe_want[2] = {kProbeWant, kProbeWant};   // where each probe slot holds ring[13]
     hipEvent_t ev_probe[2] = {nullptr, nullptr};
@@ -973,7 +974,9 @@ static hipError_t build_csc(egs_solver *s) {
     // the look at them costs a round 1.5 us of 13 and saves nothing: 2-regular games took 13%
     // longer); in the place of a binned game's candidates.  Graphs keep the arguments they were
     // captured with, so not there.
-    int *cweight = sorted && s->sh.use_wave && !s->use_graphs && egs::transpose_weights_fit(s->g.n, s->wmax) ? s->d_cweight : nullptr;
+    // A vertex that replaced values leave below its lift is in no round's work, which the look at
+    // the weights (pred_can_rise) rests on: not there either.
+    int *cweight = sorted && !s->values_set && s->sh.use_wave && !s->use_graphs && egs::transpose_weights_fit(s->g.n, s->wmax) ? s->d_cweight : nullptr;
     s->g.cweight = cweight;
     hipError_t e = sorted
                        ? egs::launch_transpose_sorted(s->g, s->d_tcounts, s->d_toffs, s->d_tscan, s->d_titems, cweight,
@@ -1205,6 +1208,7 @@ int egs_solver_prepare(egs_solver *s, const egs_options *opt) {
     s->whole_gave_up = false;
     s->whole_st = egs_stats{};
     s->mirrored = false;
+    s->values_set = false;
     s->bins_open = false;
     s->whole = plan;
     if (s->whole.nb > 0) {
@@ -1501,6 +1505,8 @@ int egs_solver_set_values(egs_solver *s, const int32_t *host_values) {
     if (!s || !s->prepared || !host_values) return fail(EGS_E_STATE, "egs_solver_set_values: call egs_solver_prepare first");
     HIP_TRY(hipSetDevice(s->device));
     if (int rc = leave_whole(s)) return rc;
+    s->values_set = true;
+    s->g.cweight = nullptr;
     HIP_TRY(hipMemcpyAsync(s->d_val, host_values, sizeof(int) * (size_t)s->g.n, hipMemcpyHostToDevice, s->stream));
     // the values may hold TOP: the phased rounds then read their TOP masks (ring[15])
     HIP_TRY(hipMemcpyAsync(s->d_ring + 15, s->h_probe + kPinOne, sizeof(int), hipMemcpyHostToDevice, s->stream));

@@ -97,3 +97,29 @@ def test_hub_in_a_candidate_that_diverges(oracle, steps):
             assert conv and st.cert_attempts > 5
             vals = s.values()
             assert np.array_equal(vals, ref), (k, vals[:2], ref[:2])
+
+
+@pytest.mark.parametrize("built", ["before", "after"])
+def test_replaced_values_below_their_lift(built):
+    """Sparse rounds from replaced values: a vertex far below its lift rises when a successor
+    does, whatever that successor's value was, in a game with hubs."""
+    import egsolver_amd as E
+    from egsolver_amd.games import Game
+    # owner 0: p takes the smaller of a and b; owner 1: hub (100 edges to the sink), a, b, sink
+    succ = np.array([2, 3] + [4] * 100 + [4, 4, 4], np.int32)
+    w = np.array([0, 0] + [0] * 100 + [-5, -4, 0], np.int32)
+    ptr = np.array([0, 2, 102, 103, 104, 105], np.int32)
+    g = Game(n=5, n0=1, ptr=ptr, succ=succ, w=w, mg=E.games.compute_mg(5, ptr, w), ext_of_int=np.arange(5, dtype=np.int32))
+    stop = ctypes.c_uint32(0)
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        print(f"[gpu-case] replaced values, transpose {built}", flush=True)
+        # sparse rounds from the first on, or with the transpose asked for after the replacement
+        s.prepare(E.options(certify_every=-1, big_deg=8, stop_flag=stop,
+                            dense_pct=101 if built == "before" else 100))
+        s.set_values(np.array([0, 0, 5, 3, 0], np.int32))
+        if built == "after":
+            s.csc()
+        conv, _ = s.iterate()
+        assert conv and s.values().tolist() == [4, 0, 5, 4, 0]
+        assert s.violations() == 0
