@@ -508,8 +508,6 @@ extern "C" {
 
 const char *egs_last_error(void) { return g_err; }
 
-// Wait limit of the single launches' barriers in microseconds (tests force it to 0: a launch
-// then gives up as soon as a workgroup has to wait, and the round kernels take over).
 void egs_solver_whole_wait(egs_solver *s, int64_t us) { s->whole_wait = us * 100; }
 
 int egs_device_query(int device, egs_device_info *out) {
@@ -1333,8 +1331,8 @@ int egs_solver_iterate(egs_solver *s, int64_t max_phases, egs_stats *st) {
                 s->st.certificates++;
                 s->st.top_marked += cr.marked;
                 // the marking kernel has named the next round (ring[11]) a full sweep
-                // the spacing only grows (doubled by failures): a long run that keeps
-                // proving small sets does not pay an attempt every few rounds
+                // the spacing stays as the failures before left it (cert_next_gap): a long run
+                // that keeps proving small sets does not pay an attempt every few rounds
                 batch = 1;        // the fixpoint often follows at once: probe again early
                 nb = 1;
                 listed = -1;

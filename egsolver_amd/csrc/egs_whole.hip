@@ -8,8 +8,9 @@
 // their share of the game on chip for the whole solve and meet at a barrier in memory:
 //   * workgroup b owns consecutive vertices, cut so that vertices plus edges are even
 //     (k_whole_prep); their values, partial keys and proof potentials live in LDS;
-//   * a thread owns up to R consecutive edges, in registers, whatever the degrees: it folds
-//     them into its vertices' LDS keys with one LDS atomic per vertex it touches;
+//   * a thread owns up to R consecutive edges, in registers (with R = 16, 70 to 111 of them
+//     spill to scratch), whatever the degrees: it folds them into its vertices' LDS keys with
+//     one LDS atomic per vertex it touches;
 //   * a round gathers the successors' values (LDS in the one-workgroup form, else global
 //     memory), folds, applies the lifts of its own vertices and votes on the risers.
 // Rounds are synchronous; values only rise and never pass the least fixpoint, and a round in
@@ -807,7 +808,7 @@ WholePlan whole_plan(int n, int64_t m, int mg, int wmax, int max_outdeg, int max
     // a TOP value less a weight stays past MG; potentials stay far below kWInf
     if ((int64_t)mg + wmax >= EGS_TOP) return p;
     if (((double)n + 1) * mg + (double)n * (((double)n + 1) * wmax + 1) > 0.5e18) return p;
-    // a thread's slots stay in registers up to 16 (of 128 a thread has): past that they spill
+    // at most 16 slots a thread, of which 8 to 16 registers (of 128 a thread has) spill already
     const int D = max_outdeg <= 4 ? 4 : max_outdeg <= 8 ? 8 : 16;
     const int V = n <= 1024 ? 1 : 2;
     if (max_outdeg <= 16 && n <= 2048 && D * V <= 16) {

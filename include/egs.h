@@ -48,12 +48,15 @@ typedef struct egs_options {
                                0 = auto (12), > 100 = never sweep */
     int32_t certify_every;  /* rounds between attempts to prove climbing vertices TOP
                                (exact; attempts back off while they fail);
-                               0 = auto (7), < 0 = never */
+                               0 = auto (7; 9 in binned rounds), < 0 = never */
     int32_t cert_max_passes;/* ceiling of the longest-path passes per proof candidate
                                (the cap starts at 64 and doubles while candidates run
                                out of passes); 0 = auto (1024) */
     int64_t max_phases;     /* phase cap; < 0 = the reference bound n*m*MG+1
-                               (src/egsolver.c:64-90) */
+                               (src/egsolver.c:64-90).  What a phase covers depends on the
+                               form of the rounds (sweeps in place see values of the same
+                               round, single launches and binned rounds do not), so the
+                               number a game needs differs between forms and options */
     const volatile uint32_t *stop_flag;  /* polled before every round and before each step
                                of a proof attempt; non-zero stops the run early with
                                partial values (the reference's timeout_expired,
@@ -61,8 +64,10 @@ typedef struct egs_options {
                                src/dev_EG_alg.cu:376).  With a stop flag at most 4 rounds
                                are queued ahead of the host. */
     int32_t slices;         /* dense rounds in successor-range phases (their value gathers
-                               stay in L2): 0 = auto (8 phases when n > 2^20 and the solver
-                               was created with n_cap >= 2^20), 1 = one sweep, 2..16 = at most
+                               stay in L2): 0 = auto (binned rounds from 400,000 vertices on
+                               where degree or hubs make them pay, else 8 phases when
+                               n > 2^20 and the solver was created with n_cap >= 2^20),
+                               1 = one sweep, 2..16 = at most
                                that many phases over slices of a power-of-two size.  Phased
                                games lift vertices above 255 edges with the wavefront kernels
                                (big_deg is capped at 255). */
@@ -83,8 +88,12 @@ typedef struct egs_stats {
     int64_t pred_visits;    /* sum of in-degree over lifted vertices */
     int32_t converged;      /* 1 when the frontier emptied (values are the fixpoint) */
     int32_t initial_active; /* size of the initial frontier */
-    double ms_prepare;      /* pack + transpose + initial frontier (device time) */
-    double ms_iterate;      /* fixpoint rounds and proofs (device time) */
+    double ms_prepare;      /* set-up of the rounds and initial frontier (device time).  Where
+                               the first iterate does it (single launches, binned games) it
+                               is known after that: of a single launch the time its kernel
+                               spends on it, of a binned game the layout and first round */
+    double ms_iterate;      /* fixpoint rounds and proofs (device time; of single launches the
+                               time inside the kernel, without the launch and its wait) */
     int64_t cert_attempts;  /* TOP proofs attempted */
     int64_t certificates;   /* TOP proofs that succeeded */
     int64_t cert_passes;    /* longest-path passes spent on proofs */
@@ -184,6 +193,10 @@ const int32_t *egs_solver_device_values(egs_solver *s);
 int egs_solver_read_csc(egs_solver *s, int32_t *cptr, int32_t *cpred);
 /* Stream the solver enqueues on (hipStream_t). */
 void *egs_solver_stream(egs_solver *s);
+/* No reference counterpart.  How long a workgroup of a single launch (a small or mid-size game
+ * solved in one kernel) waits for the others, in microseconds (default 4,000), before the
+ * launch gives up and the round kernels go on from the values reached; 0 = at its first wait. */
+void egs_solver_whole_wait(egs_solver *s, int64_t us);
 
 /* One-shot: create, load from host, prepare, iterate to the cap, read values back. */
 int egs_solve(int device, int32_t n, int32_t n0, int64_t m, int32_t mg, const int32_t *ptr,
@@ -214,7 +227,7 @@ int egs_solver_top_certificate(egs_solver *s, int32_t max_passes, int64_t *host_
 /* No reference counterpart.  For callers that cannot allocate device memory (code under
  * HIP graph capture, tight serving loops, harnesses that forbid hipMalloc): egs_solve for a
  * game already on the device, with no allocation of any kind.  The solver's workspace is
- * a fixed array in the library's device memory (26 MiB per device that runs it,
+ * a fixed array in the library's device memory (30 MiB per device that runs it,
  * held until the process ends), so games are limited to 65,536 vertices and 1,048,576
  * edges (EGS_E_CAPACITY beyond).  d_ptr[n+1], d_succ[m], d_w[m] and d_values[n] are device
  * arrays of the current device; work runs on `stream` (a hipStream_t; NULL = the null
