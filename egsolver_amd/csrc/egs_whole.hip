@@ -13,9 +13,10 @@
 //     one LDS atomic per vertex it touches;
 //   * a round gathers the successors' values (LDS in the one-workgroup form, else global
 //     memory), folds, applies the lifts of its own vertices and votes on the risers.
-// Rounds are synchronous; values only rise and never pass the least fixpoint, and a round in
-// which nothing rose ends the run at lift(val) == val.  The TOP proofs are those of
-// egs_accel.hip (same candidates, same passes, evaluated on every member).
+// Rounds are synchronous; values only rise and never pass the least fixpoint, and a round that
+// began with every value visible and in which nothing rose ends the run at lift(val) == val.
+// The TOP proofs are those of egs_accel.hip (same candidates, same passes, evaluated on every
+// member).
 //
 // Bound: the barrier (1.9 us for the arrivals and their answer, and an agent release and
 // acquire per workgroup, 0.7 us in all with 64 workgroups and 3.4 us with 256) and one
@@ -449,15 +450,20 @@ __global__ __launch_bounds__(1024) void k_whole(WholeArgs a) {
     const long long tick1 = wall_clock64();
     // a launch that goes on has rounds behind it whose risers are not known: it sweeps first
     bool known = false;
+    // The round after a proof may read values from before it: the vertices marked TOP are stored
+    // with no barrier behind them.  A quiet one says nothing.
+    bool marks = false;
     for (;;) {
-        if (known && vcount(tot) == 0) { status = kWholeDone; break; }
+        if (known && !marks && vcount(tot) == 0) { status = kWholeDone; break; }
         if (r - a.round0 >= a.limit) break;
+        marks = false;
         if (a.every > 0 && known && r >= next_cert) {
             const int before = passes;
             if (!prove((int)r, cap)) return;
             attempts++;
             if (marked > 0) {
                 certs++;
+                marks = !ONE;
             } else {
                 gap = cert_next_gap(gap, a.every, passes - before + 2 * s_ncand);
                 if (cap_hit) cap = min(cap * 2, a.max_passes);

@@ -525,3 +525,23 @@ def test_values_reached_by_a_launch_that_gives_up(n):
             conv, st = s.iterate()
             assert conv and np.array_equal(s.values(), want)
             assert st.lifted == lifted and st.initial_active == n - 1, st.as_dict()
+
+
+# the last proof leaves a few vertices that rise only through what it marked (the first of these
+# games ended nine vertices too low, 162 rounds in)
+@pytest.mark.parametrize("n,hi,alpha,seed", [(21810, 9384, 2.3859819550988592, 183094), (21810, 9384, 2.4, 5),
+                                             (40013, 60, 2.5, 6), (90007, 3000, 2.6, 7), (12011, 40, 2.6, 8)])
+def test_vertices_that_rise_through_a_proof_alone(oracle, n, hi, alpha, seed):
+    import egsolver_amd as E
+    g = E.generate(E.GenParams(n=n, seed=seed, deg_kind=E.games.DEG_POWERLAW, deg_lo=1, deg_hi=hi, alpha=alpha, wmax=1))
+    _say(f"through a proof n {g.n} m {g.m}")
+    ref = None
+    with E.Solver(g.n, g.m) as s:
+        s.load(g)
+        for every in (0, 2, 3, 5, 11):
+            s.prepare(E.options(certify_every=every))
+            conv, st = s.iterate()
+            assert conv and s.violations() == 0, (every, st.as_dict())
+            if ref is None:
+                ref = oracle.eg0(to_oracle_game(g), threads=8)[0]
+            assert np.array_equal(s.values(), ref), every
