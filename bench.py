@@ -263,14 +263,16 @@ def skewed_game(E, args):
 
 def transpose_ms(E, s, reps=3):
     """Device time of the transpose alone: prepares that build it up front (every round
-    sparse-capable, dense_pct > 100) less prepares that do not, medians of `reps`."""
+    sparse-capable, dense_pct > 100) less prepares of the same rounds that do not (sweeps in as
+    many slices, not binned), medians of `reps`."""
     def prep(opt):
         ts = []
         for _ in range(reps):
             s.prepare(opt)
             ts.append(s.stats().ms_prepare)
         return float(np.median(ts))
-    return prep(E.options(dense_pct=101)) - prep(E.options())
+    slices = 8 if s.n > 1 << 20 else 1
+    return prep(E.options(dense_pct=101, slices=slices)) - prep(E.options(slices=slices))
 
 
 def gen_many(E, family, seed, count, scale_n=1.0, workers=16):

@@ -91,7 +91,8 @@ typedef struct egs_stats {
     double ms_prepare;      /* set-up of the rounds and initial frontier (device time).  Where
                                the first iterate does it (single launches, binned games) it
                                is known after that: of a single launch the time its kernel
-                               spends on it, of a binned game the layout and first round */
+                               spends on it, of a binned game the layout and first round
+                               (asked for before: the time to count the frontier) */
     double ms_iterate;      /* fixpoint rounds and proofs (device time; of single launches the
                                time inside the kernel, without the launch and its wait) */
     int64_t cert_attempts;  /* TOP proofs attempted */
